@@ -76,7 +76,7 @@ def variant_key(plan, kind, ncoils):
 # kernels of each timed stage (short names as fold_counters derives them)
 STAGE_KERNELS = {
     "grid": ("samp_transpose_kernel", "grid_matrix_t_kernel", "grid_matrix_kernel", "matrix_fold_kernel",
-             "grid_tiles_kernel", "grid_runs_kernel", "grid_kernel", "fold_kernel"),
+             "tiles_copy_kernel", "grid_tiles_kernel", "grid_runs_kernel", "grid_kernel", "fold_kernel"),
     "interp": ("interp_staged_kernel", "interp_kernel"),
     "fft_fwd": ("fft_cols_fwd_kernel", "fft_rows_kernel|false"),
     "fft_adj": ("fft_rows_kernel|true", "fft_cols_inv_kernel"),
@@ -359,11 +359,11 @@ def kooshball_bench(dev, osfs=(2.0, 1.5), compare_runs=False, compare_tiles=True
                     tune=False):
     """3D kooshball kernels: 128^3 image, 8 coils, 20000 golden-means spokes x
     256 samples, KB width 4, osf 2.0 (256^3 grid) and 1.5 (192^3): the
-    automatic plan's gridding (the gridding matrix) and staged interpolation,
+    automatic plan's gridding (tiles on the matrix cores) and staged interpolation,
     the whole forward and adjoint transforms, with
-    ``compare_tiles`` the register-tile gridding and with ``compare_runs`` the
+    ``compare_tiles`` the tile gridding asked for and with ``compare_runs`` the
     register-run gridding too; with ``tune`` the autotuner's choice among the
-    matrix and register-tile griddings (with their split thresholds) and the
+    matrix and tile griddings (with their split thresholds) and the
     staged interpolation's 3D tiles, timed the same way. Durations from HIP
     events on the launch stream; algorithmic bytes as for the 2D workload.
     Returns a dict."""
@@ -399,7 +399,7 @@ def kooshball_bench(dev, osfs=(2.0, 1.5), compare_runs=False, compare_tiles=True
         case["nufft_adj_ms"] = time_kernel(lambda: b.adjoint(), reps, dev)
         b = None
         if compare_tiles:
-            retune(plan, grid_mode=4)  # register tiles
+            retune(plan, grid_mode=4)  # tiles
             torch.cuda.synchronize(dev)
             case["tiles_plan_bytes"] = plan.interpolator.device_bytes()
             b = BatchedNUFFT([plan], 8)
@@ -518,7 +518,7 @@ def main():
     ap.add_argument("--serve-rate", type=float, default=400.0)
     ap.add_argument("--tune-cache", default=None, help="directory of the autotuner's cache file")
     ap.add_argument("--grid-mode", type=int, default=0,
-                    help="with --kooshball: gridding variant of the timed plan (0 automatic, 4 register tiles)")
+                    help="with --kooshball: gridding variant of the timed plan (0 automatic, 4 tiles)")
     ap.add_argument("--grid-split", type=int, default=None,
                     help="after tuning, force this gridding split (for the matrix: the long-row threshold), "
                          "to profile each variant the tuner may pick")

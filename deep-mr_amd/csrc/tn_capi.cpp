@@ -60,7 +60,8 @@ void make_jobs(const tn_plan *plan, int64_t nbatch, int64_t grid_off, int64_t sa
         j.pbin_off = plan->d_pbin_off + (int64_t)f * plan->nitiles_total;
         j.mrow = plan->d_mrow ? plan->d_mrow + (int64_t)f * gvol : nullptr;
         j.mnz = plan->d_mnz;
-        j.taps = plan->d_taps ? plan->d_taps + (int64_t)f * p.npts * 4 : nullptr;
+        j.tent = plan->d_tent;
+        j.taps = plan->d_taps ? plan->d_taps + (int64_t)f * p.npts * tiles_tap_stride(p.ndim, plan->wpad) : nullptr;
         j.mlong = p.grid_split == 0  ? (p.ndim == 3 ? kMatrixLongRow3d : kMatrixLongRow)
                   : p.grid_split < 0 ? matrix_stage(p.ndim)
                                      : std::min(p.grid_split, matrix_stage(p.ndim));
@@ -161,11 +162,53 @@ static const std::vector<MatrixRun> &matrix_runs(const tn_plan *pl, int64_t f, i
     return out;
 }
 
+// Coils per tile-gridding item: every coil up to kTilesBlocks blocks of 8 (the
+// blocks of an item share its weights), more coils in equal chunks.
+static int tiles_chunk(int64_t nbatch) {
+    const int64_t blocks = (nbatch + 7) / 8, chunks = (blocks + kTilesBlocks - 1) / kTilesBlocks;
+    return (int)(8 * ((blocks + std::max<int64_t>(chunks, 1) - 1) / std::max<int64_t>(chunks, 1)));
+}
+
+// Entries per workgroup of a split tile, for plans without a split of their
+// own: four waves' worth, doubled until the table's partial tiles fit the
+// fixed gridding workspace, so that allocation-free launches take every table.
+static int tiles_doubling(const std::vector<Job> &jobs, const std::vector<const tn_plan *> &plan_of) {
+    for (int times = 1;; times *= 2) {
+        int64_t floats = 0;
+        for (size_t ji = 0; ji < jobs.size(); ++ji) {
+            const Job &j = jobs[ji];
+            const tn_plan *pl = plan_of[ji];
+            if (pl->p.grid_split != 0) continue;
+            const int64_t part = (int64_t)kTilesWave * (kBlock / kWave) * times;
+            const int32_t *off = pl->h_bin_off.data() + (j.bin_off - pl->d_bin_off);
+            int64_t parts = 0;
+            for (int64_t tl = 0; tl < pl->ntiles_total; ++tl) {
+                const int64_t n = off[tl + 1] - off[tl];
+                if (n > part) parts += (n + part - 1) / part;
+            }
+            floats += parts * 2 * j.nbatch * j.T[0] * j.T[1] * j.T[2];
+        }
+        if (floats <= kStaticScratchFloats || times >= 1 << 20) return times;
+    }
+}
+
+// Whether a table's tile gridding reads its samples from a coil-minor copy:
+// from kTilesCopyBytes of them on, or where a job's offsets pass 32 bits.
+static bool tiles_copy(const std::vector<Job> &jobs) {
+    int64_t bytes = 0;
+    bool wide = false;
+    for (const Job &j : jobs) {
+        bytes += (int64_t)sizeof(float2) * j.npts * j.nbatch;
+        wide |= (j.nbatch - 1) * j.samp_bstride + j.npts >= (1ll << 29);
+    }
+    return wide || bytes >= kTilesCopyBytes;
+}
+
 // Work lists. Interpolation items are (job, sample block, coil range);
 // gridding items are (job, tile, coil range). `plan_of[j]` is the plan job j
 // came from (for its chunk preferences).
 static int build_tables_for(const std::vector<Job> &jobs, const std::vector<const tn_plan *> &plan_of,
-                            LaunchTables &t, bool force_gather = false, bool no_copy = false) {
+                            LaunchTables &t, bool force_gather = false, int lr_coeffs = 0) {
     t.kind_interp = interp_kind(jobs);
     t.kind_grid = t.kind_interp;
     int64_t max_plane = 1, max_region = 1, max_rows = 1, max_cells = 1;
@@ -182,15 +225,13 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
         if (pl->grid_mode != gmode) return fail(TN_E_ARG, "batched plans must share the gridding variant");
     t.grid_mode = gmode;
     const int gndim = kind_ndim(t.kind_grid);
-    // LDS sizing of the LDS gridding kernels (register tiles: of the LDS-atomic
-    // kernel that serves their low-rank launches)
-    const int lmode = gmode == kGridTiles ? kGridSpread : gmode;
-    if (gmode != kGridMatrix && grid_lds_bytes(1, max_plane, wc, lmode, gndim) > kGridLdsBudget)
+    const bool lds_grid = gmode != kGridMatrix && gmode != kGridTiles;
+    if (lds_grid && grid_lds_bytes(1, max_plane, wc, gmode, gndim) > kGridLdsBudget)
         return fail(TN_E_ARG, "gridding tile too large for LDS (%zu bytes for one coil)",
-                    grid_lds_bytes(1, max_plane, wc, lmode, gndim));
+                    grid_lds_bytes(1, max_plane, wc, gmode, gndim));
     int lds_coils = 1;
     while (lds_coils < (gmode == kGridRuns ? kRunsMaxCoils : 64) &&
-           grid_lds_bytes(lds_coils + 1, max_plane, wc, lmode, gndim) <= kGridLdsBudget)
+           grid_lds_bytes(lds_coils + 1, max_plane, wc, gmode, gndim) <= kGridLdsBudget)
         ++lds_coils;
     const size_t region_coil = (size_t)max_region * 2 * sizeof(float);
     // the staged interpolation's row table (one int per (z, y) row of a
@@ -227,9 +268,11 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
         mat_cpl = (cwmax == 16 || (cwmax >= 4 && kind_ndim(t.kind_grid) == 2)) ? 2 : 1;
         if (!inplace && cwmax > 0) mat_cpi = std::min(kBlock, kBlock / (cwmax / mat_cpl) * kMatrixPasses);
     }
-    std::vector<Item> interp, grid, fold, tr;
+    std::vector<Item> interp, grid, fold, tr, joined;
     std::vector<int64_t> slot_base;
     int64_t scratch = 0;
+    const int tiles_times = gmode == kGridTiles ? tiles_doubling(jobs, plan_of) : 0;
+    const bool tcopy = gmode == kGridTiles && lr_coeffs == 0 && !force_gather && tiles_copy(jobs);
     for (size_t ji = 0; ji < jobs.size(); ++ji) {
         const Job &j = jobs[ji];
         const tn_plan *pl = plan_of[ji];
@@ -237,10 +280,10 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
         // one coil per wave (more coils per item cost occupancy, which hides
         // the latency of its LDS read-add-write chains)
         const int gc_auto = gmode == kGridRuns    ? std::min(lds_coils, kBlock / kWave)
-                            : gmode == kGridTiles ? std::min(lds_coils, kTilesCoils)
+                            : gmode == kGridTiles ? tiles_chunk(j.nbatch)
                                                   : lds_coils;
         const int gc = std::min(chunk_for(pl->p.grid_chunk, j.nbatch, gc_auto),
-                                gmode == kGridTiles ? std::min(lds_coils, kTilesCoils) : lds_coils);
+                                gmode == kGridTiles ? 8 * kTilesBlocks : lds_coils);
         if (mode == kInterpStaged) {
             // one item per (tile, segment) covers every coil; the region is
             // loaded `ic` coils at a time
@@ -285,7 +328,7 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
             // coil-minor sample copy: chunks of mc coils padded to cw lanes
             // (not for tables whose gridding reads the samples in place:
             // low-rank gridding, or tables only used to interpolate)
-            if (no_copy || force_gather) {
+            if (lr_coeffs > 0 || force_gather) {
                 st_none = true;
             } else if (mc >= 2) {
                 st_cw = std::max(st_cw, cw);
@@ -299,46 +342,68 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
             continue;
         }
         max_gc = std::max(max_gc, gc);
-        if (gmode == kGridTiles) {
-            // coil-minor sample copy in chunks of gc coils padded to cw
-            // (scalar-loaded records); none for low-rank or gather tables,
-            // whose gridding takes the LDS-atomic kernel over the same bins
-            if (no_copy || force_gather) {
-                st_none = true;
-            } else {
-                st_cw = std::max(st_cw, gc <= 2 ? 2 : gc <= 4 ? 4 : 8);
-                const int64_t pblk = (j.npts + kBlock - 1) / kBlock;
-                for (int c0 = 0; c0 < j.nbatch; c0 += gc)
+        if (tcopy) {  // one record chunk per item chunk, kTilesCopyCoils coils per copy item
+            const int64_t pblk = (j.npts + kBlock - 1) / kBlock;
+            st_cw = std::max(st_cw, (gc + 1) / 2 * 2);  // whole 16-byte pieces
+            for (int c0 = 0; c0 < j.nbatch; c0 += gc)
+                for (int c = c0; c < c0 + gc; c += kTilesCopyCoils)
                     for (int64_t b = 0; b < pblk; ++b)
-                        tr.push_back(Item{(int)ji, (int)b, c0, std::min(j.nbatch, c0 + gc), c0 / gc, 0, 0, -1});
-            }
+                        tr.push_back(Item{(int)ji, (int)b, std::min(c, j.nbatch),
+                                          std::min({j.nbatch, c0 + gc, c + kTilesCopyCoils}), c0 / gc, c - c0, 0, -1});
         }
         const int64_t ntiles = (int64_t)j.NT[0] * j.NT[1] * j.NT[2];
         const int64_t fg = (j.bin_off - pl->d_bin_off) / std::max<int64_t>(pl->ntiles_total, 1);
         const int32_t *goff = pl->h_bin_off.data() + fg * pl->ntiles_total;
-        const int split = pl->p.grid_split == 0 ? (gmode == kGridTiles ? kTilesSplit : kGridSplitDefault)
-                          : pl->p.grid_split < 0 ? INT32_MAX : pl->p.grid_split;
+        const bool tiles = gmode == kGridTiles;
+        constexpr int waves = kBlock / kWave;
+        // entries per workgroup of a split tile; tiles: a tile of at most
+        // wave_max entries goes to one wave, of more to a workgroup's four
+        // waves, in whole steps of the kernel
+        const int64_t wave_max = tiles ? (pl->p.grid_split == 0  ? kTilesWave
+                                          : pl->p.grid_split < 0 ? INT32_MAX
+                                                                 : (pl->p.grid_split + waves - 1) / waves)
+                                       : 0;
+        const int64_t split = pl->p.grid_split == 0  ? (tiles ? wave_max * waves * tiles_times : kGridSplitDefault)
+                              : pl->p.grid_split < 0 ? INT32_MAX
+                                                     : pl->p.grid_split;
         const int64_t cells = (int64_t)j.T[0] * j.T[1] * j.T[2];  // partial size per coil
-        for (int64_t tl = 0; tl < ntiles; ++tl) {
+        std::vector<int32_t> order;
+        if (tiles) order = brick_order(j.NT, j.ndim);
+        for (int64_t ti = 0; ti < ntiles; ++ti) {
+            const int64_t tl = tiles ? order[ti] : ti;
             const int32_t b0 = goff[tl], b1 = goff[tl + 1];
             const int nparts = (int)std::max<int64_t>(1, ((int64_t)(b1 - b0) + split - 1) / split);
             for (int c0 = 0; c0 < j.nbatch; c0 += gc) {
                 const int c1 = std::min(j.nbatch, c0 + gc);
-                if (nparts == 1) {
+                if (nparts == 1 && (!tiles || b1 - b0 <= wave_max)) {
                     grid.push_back(Item{(int)ji, (int)tl, c0, c1, b0, b1, 0, -1});
                     continue;
                 }
-                const int slot = (int)slot_base.size();
-                slot_base.push_back(scratch);
-                scratch += (int64_t)nparts * 2 * (c1 - c0) * cells;
+                const int slot = nparts > 1 ? (int)slot_base.size() : -1;
+                if (nparts > 1) {
+                    slot_base.push_back(scratch);
+                    scratch += (int64_t)nparts * 2 * (c1 - c0) * cells;
+                }
                 const int32_t per = (b1 - b0 + nparts - 1) / nparts;
                 for (int q = 0; q < nparts; ++q) {
                     const int32_t e0 = b0 + q * per, e1 = std::min(b1, e0 + per);
-                    grid.push_back(Item{(int)ji, (int)tl, c0, c1, e0, e1, q, slot});
+                    if (!tiles) {
+                        grid.push_back(Item{(int)ji, (int)tl, c0, c1, e0, e1, q, slot});
+                        continue;
+                    }
+                    const int32_t share = ((e1 - e0 + waves - 1) / waves + 15) / 16 * 16;
+                    for (int w = 0; w < waves; ++w)
+                        joined.push_back(Item{(int)ji, (int)tl | kTilesJoin, c0, c1, std::min(e1, e0 + w * share),
+                                              std::min(e1, e0 + (w + 1) * share), q, slot});
                 }
-                tile_fold_items((int)ji, (int)tl, c0, c1, slot, nparts, (int64_t)(c1 - c0) * cells, kBlock, fold);
+                if (nparts > 1)
+                    tile_fold_items((int)ji, (int)tl, c0, c1, slot, nparts, (int64_t)(c1 - c0) * cells, kBlock, fold);
             }
         }
+    }
+    if (gmode == kGridTiles) {
+        tiles_deal(joined, grid);
+        t.wpad = plan_of.empty() ? 0 : plan_of[0]->wpad;
     }
     t.scratch_floats = scratch;
     t.grid_coils = max_gc;
@@ -347,15 +412,13 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
         // every job gets its copy at st_cw coils per record
         int64_t off = 0;
         for (size_t ji = 0; ji < jobs.size(); ++ji) {
-            const int mc = gmode == kGridTiles ? std::min(chunk_for(plan_of[ji]->p.grid_chunk, jobs[ji].nbatch,
-                                                                    std::min(lds_coils, kTilesCoils)),
-                                                          std::min(lds_coils, kTilesCoils))
-                                               : std::min(chunk_for(plan_of[ji]->p.grid_chunk, jobs[ji].nbatch,
-                                                                    kMatrixChunk),
-                                                          kMatrixCoils);
+            const int nb = jobs[ji].nbatch, chunk = plan_of[ji]->p.grid_chunk;
+            const int mc = gmode == kGridMatrix
+                               ? std::min(chunk_for(chunk, nb, kMatrixChunk), kMatrixCoils)
+                               : std::min(chunk_for(chunk, nb, tiles_chunk(nb)), 8 * kTilesBlocks);
             jobs_st[ji].st_off = off;
-            jobs_st[ji].st_chunk = mc;
-            off += (int64_t)((jobs[ji].nbatch + mc - 1) / mc) * jobs[ji].npts * st_cw;
+            jobs_st[ji].tchunk = mc;
+            off += (int64_t)((nb + mc - 1) / mc) * jobs[ji].npts * st_cw;
         }
         t.st_cw = st_cw;
         t.st_cpl = mat_cpl;
@@ -374,7 +437,7 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
     const int64_t copy_bytes = t.d_st ? (int64_t)(sizeof(Item) * std::max<size_t>(tr.size(), 1) +
                                                   sizeof(float2) * std::max<int64_t>(t.st_elems, 1))
                                       : 0;
-    t.grid_lds = gmode == kGridMatrix ? 0 : grid_lds_bytes(max_gc, max_plane, wc, lmode, gndim);
+    t.grid_lds = lds_grid ? grid_lds_bytes(max_gc, max_plane, wc, gmode, gndim) : 0;
     t.interp_lds = mode == kInterpStaged ? region_coil * (size_t)max_ic + rows_bytes : 0;
     t.interp_coils = max_ic;
     const int rc = upload_tables(jobs_st, interp, grid, fold, slot_base, t);
@@ -461,6 +524,7 @@ void destroy(tn_plan *pl) {
     if (pl->d_mrow) (void)hipFree(pl->d_mrow);
     if (pl->d_mnz) (void)hipFree(pl->d_mnz);
     if (pl->d_taps) (void)hipFree(pl->d_taps);
+    if (pl->d_tent) (void)hipFree(pl->d_tent);
     for (int a = 0; a < 3; ++a)
         if (pl->d_fft_tw[a]) (void)hipFree(pl->d_fft_tw[a]);
     for (int d = 0; d < 3; ++d)
@@ -471,23 +535,26 @@ void destroy(tn_plan *pl) {
 
 enum TableUse { kTablesPlain = 0, kTablesGather = 1, kTablesLowRank = 2 };
 
-tn::LaunchTables *plan_tables(tn_plan *plan, int64_t nbatch, int *rc, int use = kTablesPlain) {
+// Tables of a plan for `nbatch` coils; low-rank tables hold nbatch * ncoeff
+// accumulator coils.
+tn::LaunchTables *plan_tables(tn_plan *plan, int64_t nbatch, int *rc, int use = kTablesPlain, int ncoeff = 1) {
     auto &cache = use == kTablesGather ? plan->cache_gather : use == kTablesLowRank ? plan->cache_lowrank : plan->cache;
-    auto it = cache.find(nbatch);
+    const int64_t key = use == kTablesLowRank ? nbatch << 32 | ncoeff : nbatch;
+    auto it = cache.find(key);
     if (it != cache.end()) {
         *rc = TN_OK;
         return &it->second;
     }
     std::vector<Job> jobs;
-    make_jobs(plan, nbatch, 0, 0, 0, jobs);
+    make_jobs(plan, nbatch * ncoeff, 0, 0, 0, jobs);
     std::vector<const tn_plan *> owners(jobs.size(), plan);
     LaunchTables t;
-    *rc = build_tables_for(jobs, owners, t, use == kTablesGather, use == kTablesLowRank);
+    *rc = build_tables_for(jobs, owners, t, use == kTablesGather, use == kTablesLowRank ? ncoeff : 0);
     if (*rc != TN_OK) {
         free_tables(t);
         return nullptr;
     }
-    return &(cache[nbatch] = t);
+    return &(cache[key] = t);
 }
 
 // Shared checks of the low-rank entry points: one-frame plan whose samples
@@ -507,6 +574,18 @@ int check_lowrank(const tn_plan *plan, int64_t nbatch, int32_t ncoeff, int32_t f
     lr.nframes = (int32_t)(plan->p.npts / frame_npts);
     lr.frame_npts = frame_npts;
     return TN_OK;
+}
+
+// Whether two plans of different gridding variants may share a batch: both
+// chosen automatically among the tile and the matrix gridding, or one of
+// those chosen and the matrix asked for (automatic plans and explicit matrix
+// plans batch together).
+bool batch_modes_mix(const tn_plan *a, const tn_plan *b) {
+    auto ok = [](const tn_plan *p) {
+        return (p->p.grid_mode == kGridAuto && (p->grid_mode == kGridTiles || p->grid_mode == kGridMatrix)) ||
+               p->p.grid_mode == kGridMatrix;
+    };
+    return ok(a) && ok(b);
 }
 
 // Checks that the current device is the plan's device.
@@ -550,39 +629,41 @@ int tn_plan_create(const tn_plan_params *params, const float *coord_dev, tn_stre
             delete pl;
             return fail(TN_E_ARG, "grid_mode 2 supports at most %d taps per z plane (got %d)", kRunsMaxTaps, taps);
         }
-        // automatic: the sparse gridding matrix when it fits kMatrixAutoBytes
-        // (8 bytes per sample and tap), else register tiles (3D), else
-        // register runs when the taps of a z plane fit the registers, else
-        // per-sample LDS atomics
+        // automatic: the tile gridding where it serves the plan, else the
+        // sparse gridding matrix when it fits kMatrixAutoBytes (8 bytes per
+        // sample and tap), else register runs when the taps of a z plane fit
+        // the registers, else per-sample LDS atomics
         const int64_t nnz = (int64_t)params->nframes * params->npts * params->width[0] * params->width[1] *
                             params->width[2];
         const int64_t nrows = (int64_t)params->nframes * params->grid[0] * params->grid[1] * params->grid[2];
         const bool matrix_ok = nnz < INT32_MAX && (uint64_t)nnz * sizeof(int2) <= kMatrixAutoBytes &&
                                nrows < (int64_t)UINT32_MAX && params->npts <= ((int64_t)1 << 28);
-        // then register tiles where they fit (3D)
         const bool tiles_ok = tiles_fit(*params);
         if (params->grid_mode == kGridTiles && !tiles_ok) {
             delete pl;
             return fail(TN_E_ARG,
-                        "grid_mode 4 (register tiles) needs a 3D plan with at most %d taps per axis and grid "
-                        "lengths that are multiples of the %dx%dx%d tile with at least two tiles per axis",
-                        kTilesMaxWidth, kTilesT[0], kTilesT[1], kTilesT[2]);
+                        "grid_mode 4 (register tiles) needs a 3D plan with at most 4 taps per axis and grid "
+                        "lengths that are multiples of 8 x 8 x 4 with at least two such blocks per axis");
         }
         pl->grid_mode = params->grid_mode == kGridSpread   ? kGridSpread
                         : params->grid_mode == kGridMatrix ? kGridMatrix
                         : params->grid_mode == kGridRuns   ? kGridRuns
                         : params->grid_mode == kGridTiles  ? kGridTiles
+                        : tiles_serve(*params)             ? kGridTiles
                         : matrix_ok                        ? kGridMatrix
                         : tiles_ok                         ? kGridTiles
                         : runs_ok                          ? kGridRuns
                                                            : kGridSpread;
         if (pl->grid_mode == kGridTiles) {  // the tile the kernel is built for, whatever was asked
             pl->ntiles_total = 1;
+            int wmax = 1;
             for (int d = 0; d < 3; ++d) {
-                pl->tile[d] = kTilesT[2 - d];
-                pl->ntiles[d] = params->grid[d] / pl->tile[d];
+                pl->tile[d] = tiles_dim(params->ndim, 2 - d);
+                pl->ntiles[d] = (params->grid[d] + pl->tile[d] - 1) / pl->tile[d];
                 pl->ntiles_total *= pl->ntiles[d];
+                wmax = std::max(wmax, (int)params->width[d]);
             }
+            pl->wpad = tiles_pad(wmax);
         }
         // kernels wider than kStagedMaxWidth grid only through the matrix
         const int wmax = std::max(params->width[0], std::max(params->width[1], params->width[2]));
@@ -634,14 +715,15 @@ int64_t tn_plan_device_bytes(const tn_plan *plan) {
     const tn_plan_params &p = plan->p;
     const int64_t total = (int64_t)p.nframes * p.npts;
     int64_t b = sizeof(float) * std::max<int64_t>(total * p.ndim, 1);                     // coordinates
-    b += sizeof(float4) * std::max<int64_t>(plan->nentries, 1);                            // gridding bins
+    if (plan->d_entries) b += sizeof(float4) * std::max<int64_t>(plan->nentries, 1);       // gridding bins
     b += sizeof(int32_t) * (plan->ntiles_total * p.nframes + 1);
     b += sizeof(float4) * std::max<int64_t>(total, 1);                                     // interpolation bins
     b += sizeof(int32_t) * (plan->nitiles_total * p.nframes + 1);
     if (plan->d_mrow)                                                                      // gridding matrix
         b += sizeof(int32_t) * ((int64_t)p.grid[0] * p.grid[1] * p.grid[2] * p.nframes + 1) +
              sizeof(int2) * std::max<int64_t>(plan->mnnz, 1);
-    if (plan->d_taps) b += 4 * sizeof(float4) * total;                                    // tile gridding taps
+    if (plan->d_taps)                                                                      // tile gridding
+        b += sizeof(float) * tiles_tap_stride(p.ndim, plan->wpad) * total + sizeof(int2) * plan->nentries;
     for (int d = 0; d < 3; ++d)
         if (plan->d_apod[d]) b += sizeof(float) * p.shape[d];
     b += plan->fft_tw_bytes;
@@ -765,7 +847,7 @@ int tn_grid_lowrank(tn_plan *plan, const void *samp, void *grid, int64_t nbatch,
     rc = check_device(plan->device);
     if (rc) return rc;
     // accumulator coils are (coil, coeff) pairs
-    LaunchTables *t = plan_tables(plan, nbatch * ncoeff, &rc, kTablesLowRank);
+    LaunchTables *t = plan_tables(plan, nbatch, &rc, kTablesLowRank, ncoeff);
     if (!t) return rc;
     return launch_grid(*t, (const float2 *)samp, (float2 *)grid, weight, (hipStream_t)stream, lr);
 }
@@ -840,8 +922,15 @@ int tn_batch_create(tn_plan *const *plans, const int64_t *nbatch, const int64_t 
         return fail(TN_E_ARG, "NULL argument");
     *out = nullptr;
     if (njobs < 1) return fail(TN_E_ARG, "njobs must be >= 1");
-    std::vector<Job> jobs;
-    std::vector<const tn_plan *> owners;
+    // one table per gridding variant (and tap record size) among the plans: automatic plans may
+    // differ (the kernel width and the plan's size decide), variants asked for
+    // may not
+    struct Part {
+        int mode, wpad;
+        std::vector<Job> jobs;
+        std::vector<const tn_plan *> owners;
+    };
+    std::vector<Part> parts;
     int device = plans[0] ? plans[0]->device : -1;
     int ndim = plans[0] ? plans[0]->p.ndim : 0;
     for (int k = 0; k < njobs; ++k) {
@@ -851,20 +940,23 @@ int tn_batch_create(tn_plan *const *plans, const int64_t *nbatch, const int64_t 
         if (pl->p.ndim != ndim) return fail(TN_E_ARG, "plans mix 2D and 3D");
         if (nbatch[k] < 1 || nbatch[k] >= INT32_MAX) return fail(TN_E_ARG, "nbatch[%d] < 1", k);
         if (grid_offset[k] < 0 || samp_offset[k] < 0) return fail(TN_E_ARG, "negative offset");
-        const size_t before = jobs.size();
-        make_jobs(pl, nbatch[k], grid_offset[k], samp_offset[k],
-                  weight_offset ? weight_offset[k] : -1, jobs);
-        owners.resize(jobs.size(), pl);
-        (void)before;
+        if (pl->grid_mode != plans[0]->grid_mode && !batch_modes_mix(pl, plans[0]))
+            return fail(TN_E_ARG, "batched plans must share the gridding variant");
+        auto part = std::find_if(parts.begin(), parts.end(), [&](const Part &q) { return q.mode == pl->grid_mode && q.wpad == pl->wpad; });
+        if (part == parts.end()) part = parts.insert(parts.end(), Part{pl->grid_mode, pl->wpad, {}, {}});
+        make_jobs(pl, nbatch[k], grid_offset[k], samp_offset[k], weight_offset ? weight_offset[k] : -1, part->jobs);
+        part->owners.resize(part->jobs.size(), pl);
     }
     int rc = check_device(device);
     if (rc) return rc;
     tn_batch *b = new tn_batch();
     b->device = device;
     b->plans.assign(plans, plans + njobs);
-    rc = build_tables_for(jobs, owners, b->tables);
+    b->tables.resize(parts.size());
+    for (size_t q = 0; q < parts.size() && rc == TN_OK; ++q)
+        rc = build_tables_for(parts[q].jobs, parts[q].owners, b->tables[q]);
     if (rc) {
-        free_tables(b->tables);
+        for (LaunchTables &t : b->tables) free_tables(t);
         delete b;
         return rc;
     }
@@ -878,7 +970,7 @@ int tn_batch_destroy(tn_batch *batch) {
     int cur = 0;
     (void)hipGetDevice(&cur);
     (void)hipSetDevice(batch->device);
-    free_tables(batch->tables);
+    for (LaunchTables &t : batch->tables) free_tables(t);
     (void)hipSetDevice(cur);
     delete batch;
     return TN_OK;
@@ -890,8 +982,11 @@ int tn_batch_interp(tn_batch *batch, const void *grid_base, void *samp_base,
     if (!batch || !grid_base || !samp_base) return fail(TN_E_ARG, "NULL argument");
     int rc = check_device(batch->device);
     if (rc) return rc;
-    return launch_interp(batch->tables, (const float2 *)grid_base, (float2 *)samp_base, weight_base,
-                         (hipStream_t)stream);
+    for (const LaunchTables &t : batch->tables) {
+        rc = launch_interp(t, (const float2 *)grid_base, (float2 *)samp_base, weight_base, (hipStream_t)stream);
+        if (rc) return rc;
+    }
+    return TN_OK;
 }
 
 int tn_batch_grid(tn_batch *batch, const void *samp_base, void *grid_base, const float *weight_base,
@@ -900,8 +995,11 @@ int tn_batch_grid(tn_batch *batch, const void *samp_base, void *grid_base, const
     if (!batch || !grid_base || !samp_base) return fail(TN_E_ARG, "NULL argument");
     int rc = check_device(batch->device);
     if (rc) return rc;
-    return launch_grid(batch->tables, (const float2 *)samp_base, (float2 *)grid_base, weight_base,
-                       (hipStream_t)stream);
+    for (const LaunchTables &t : batch->tables) {
+        rc = launch_grid(t, (const float2 *)samp_base, (float2 *)grid_base, weight_base, (hipStream_t)stream);
+        if (rc) return rc;
+    }
+    return TN_OK;
 }
 
 }  // extern "C"

@@ -49,11 +49,31 @@ constexpr int kGridPad = 4;      // accumulator row padding (floats)
 // set per z plane), over the tile's entries in sample order with per-sample
 // taps from a plan table.
 enum GridMode { kGridAuto = 0, kGridSpread = 1, kGridRuns = 2, kGridMatrix = 3, kGridTiles = 4 };
-constexpr int kTilesT[3] = {8, 8, 4};  // register-tile gridding tile (x, y, z): 64 lanes x 4 planes
-constexpr int kTilesMaxWidth = 4;      // taps per axis the register tiles hold
-constexpr int kTilesCoils = 8;         // coils per register-tile item (4 planes x 8 coils x 2 floats)
-constexpr int kTilesSplit = 384;       // default entries per register-tile item (kooshball 128^3, osf 2:
-                                       // 3.30 ms against 3.52 at 256, 3.38 at 512, 3.86 at 1024)
+// Tile gridding (matrix cores): a tile is four patches of 4x4 cells, the z
+// planes of a 4x4x4 tile in 3D and the quadrants of an 8x8 tile in 2D.
+__host__ __device__ constexpr int tiles_dim(int ndim, int axis) {  // axis: 0 x, 1 y, 2 z
+    return ndim == 3 ? 4 : axis < 2 ? 8 : 1;
+}
+constexpr int kTilesMaxWidth = 6;  // most taps per axis
+constexpr int kTilesBlocks = 4;    // most blocks of 8 coils per item
+constexpr int kTilesCopyCoils = 8; // coils per workgroup of the coil-minor copy
+// Most entries of a tile that one wave takes by default; larger tiles go to a
+// workgroup's four waves. Short chains keep the sums as exact as the matrix
+// rows (61x101x84 kooshball, error against 64 bits: 7.9e-7 at 96, 8.7e-7 at
+// 192, 1.2e-6 at 384; the matrix 7.9e-7) and small problems balanced
+// (CG-SENSE, 195 k entries: 1.95 ms a solve at 64-96, 2.02 at 160, 2.16 at
+// 256); the large kooshball (27 M entries) takes 4% longer than at 384.
+constexpr int kTilesWave = 96;
+// samples of a table (bytes) from which the gridding reads a coil-minor copy:
+// in place, the records of an entry's coils lie in different rows and a wave's
+// loads touch four times the cache lines, which costs nothing while the samples
+// stay in the L2s (12 coils, 31 MB: 46 us against 37 + 15 for the copy) and
+// most of the time beyond (kooshball, 328 MB: 1.63 ms against 0.98 + 0.11)
+constexpr int64_t kTilesCopyBytes = 48ll << 20;
+// Tap record of a sample: the taps of each axis, padded with zeros to wpad
+// words (16-byte aligned).
+__host__ __device__ constexpr int tiles_pad(int wmax) { return wmax <= 4 ? 4 : 8; }
+__host__ __device__ constexpr int tiles_tap_stride(int ndim, int wpad) { return ndim * wpad; }
 constexpr int kMatrixLongRow = 128;  // default (2D): rows with more entries get a whole workgroup
 constexpr int kMatrixLongRow3d = 256;  // default (3D): kooshball 128^3 at osf 2: 3.74 ms against 4.33 (128), 4.30 (512)
 constexpr int kMatrixChunk = 16;     // default coils per item (record width of the coil-minor copy)
@@ -93,7 +113,7 @@ struct alignas(16) Job {
     int32_t NT[3];      // tiles per axis
     int32_t IT[3];      // staged-interpolation tile
     int32_t INT_[3];    // staged-interpolation tiles per axis
-    int32_t st_chunk;   // tile gridding: coils per chunk of the coil-minor copy
+    int32_t tchunk;     // tile gridding: coils per chunk of the coil-minor copy
     int32_t pad1;
     float beta[3];
     float inv_scale;
@@ -116,8 +136,9 @@ struct alignas(16) Job {
     int64_t samp_bstride;
     int64_t w_off;            // offset into the weight base (-1: no weight)
     int64_t st_off;           // matrix / tile gridding: this job's coil-minor sample copy in the table's buffer
-    const float4 *taps;       // tile gridding: per sample of this frame, (x taps), (y taps), (z taps),
-                              // (footprint origin x, y, z as int bits, 0)
+    const int2 *tent;         // tile gridding: (sample, tile-local footprint origin x, y, z + 16 in bytes 0-2),
+                              // sorted by tile, samples ascending; bin_off holds the offsets
+    const float *taps;        // tile gridding: tap records of this frame's samples
 };
 
 // Low-rank subspace arguments of a launch (ncoeff == 0: plain transform).
@@ -150,13 +171,14 @@ struct LaunchTables {
     size_t interp_lds = 0;     // dynamic LDS bytes for the staged interpolation
     int interp_coils = 1;      // coils per LDS region load (staged interpolation)
     int grid_mode = kGridSpread;  // gridding variant (matches the plans' entry order)
-    // matrix gridding over a coil-minor copy of the samples: chunks of
-    // st_cw coils, [chunk][sample][st_cw] per job, built by the transpose items
+    // matrix and tile gridding over a coil-minor copy of the samples: chunks of
+    // st_cw coils, [chunk][sample][st_cw] per job, built by the copy items
     Item *d_tr = nullptr;
     int64_t n_tr = 0;
     float2 *d_st = nullptr;
     int64_t st_elems = 0;
     int st_cw = 0;  // 0: the lane-per-cell matrix kernel reads the samples in place
+    int wpad = 0;   // tile gridding: words per axis of the tap records
     int st_cpl = 1; // coils per lane of the matrix kernel over the copy (1 or 2)
     int64_t device_bytes = 0;  // bytes of the device allocations above
 };
@@ -193,7 +215,9 @@ struct tn_plan {
     float2 *d_fft_tw[3] = {nullptr, nullptr, nullptr};  // pruned FFT twiddles exp(-2 pi i m / G), (x, y, z); null: none
     int64_t fft_tw_bytes = 0;
     int64_t mnnz = 0;
-    float4 *d_taps = nullptr;   // tile gridding: 4 float4 per sample (taps per axis, origin)
+    int2 *d_tent = nullptr;     // tile gridding entries
+    float *d_taps = nullptr;    // tile gridding: tap records, tiles_tap_stride words per sample
+    int wpad = 0;
     std::map<int64_t, tn::LaunchTables> cache;
     std::map<int64_t, tn::LaunchTables> cache_gather;  // gather-mode tables (low-rank interpolation)
     std::map<int64_t, tn::LaunchTables> cache_lowrank; // tables of the low-rank gridding (no coil-minor copy)
@@ -201,7 +225,7 @@ struct tn_plan {
 
 struct tn_batch {
     int device = 0;
-    tn::LaunchTables tables;
+    std::vector<tn::LaunchTables> tables;  // one per gridding variant among the plans
     std::vector<tn_plan *> plans;
 };
 
@@ -227,23 +251,26 @@ int launch_grid(const LaunchTables &t, const float2 *samp, float2 *grid,
 int static_scratch(int device, float **out);
 int launch_interp_lowrank(const LaunchTables &t, const float2 *grid, float2 *samp,
                           const float *weight, hipStream_t stream, LowRank lr);
-int launch_fold(const LaunchTables &t, float2 *grid, hipStream_t stream);
+// Sums the partial tiles of split gridding tiles (nothing when none are split).
+int launch_fold(const LaunchTables &t, float2 *grid, const float *scratch, hipStream_t stream);
 int launch_apod_pad(const tn_plan *plan, const float2 *image, float2 *grid,
                     int64_t nimg, hipStream_t stream);
 int launch_crop_apod(const tn_plan *plan, const float2 *grid, float2 *image,
                      int64_t nimg, hipStream_t stream);
 int build_bins(tn_plan *plan, hipStream_t stream);
-// Whether register-tile gridding can serve a plan of these parameters: 3D,
-// at most kTilesMaxWidth taps per axis, grids of whole tiles with at least
-// two tiles per axis (a footprint then meets a tile at most once).
+// Whether an explicit grid_mode 4 is accepted: 3D, at most 4 taps per axis,
+// grids of whole 8x8x4 blocks with at least two per axis. (The automatic mode
+// uses the tile gridding beyond that, where tiles_serve says so.)
 inline bool tiles_fit(const tn_plan_params &p) {
     if (p.ndim != 3) return false;
-    for (int d = 0; d < 3; ++d) {
-        const int T = kTilesT[2 - d];  // params are (z, y, x)
-        if (p.width[d] > kTilesMaxWidth || p.grid[d] % T != 0 || p.grid[d] < 2 * T) return false;
-    }
+    const int block[3] = {4, 8, 8};  // params are (z, y, x)
+    for (int d = 0; d < 3; ++d)
+        if (p.width[d] > 4 || p.grid[d] % block[d] != 0 || p.grid[d] < 2 * block[d]) return false;
     return true;
 }
+bool tiles_serve(const tn_plan_params &p);
+int launch_tiles(const LaunchTables &t, const float2 *samp, float2 *grid, const float *weight, hipStream_t stream,
+                 const LowRank &lr, float *scratch);
 int build_matrix(tn_plan *plan, hipStream_t stream);
 // Pruned, fused oversampled-grid FFT stages (2D plans with supported lengths).
 bool fft_supported(const tn_plan *plan);

@@ -165,21 +165,69 @@ __global__ void matrix_emit_kernel(BinGeom geo, const float *__restrict__ coord,
     }
 }
 
-// Per-sample taps of the register-tile gridding (3D, at most
-// kTilesMaxWidth taps per axis): float4 x taps, y taps, z taps (zeros past
-// the axis width) and the footprint origin (x, y, z) as int bits, the same
-// taps and wrapped origin the other gridding variants evaluate.
-__global__ void tiles_taps_kernel(BinGeom geo, const float *__restrict__ coord, float4 *__restrict__ taps) {
+// Tile gridding: the pieces of sample i's footprint per axis (unused axes:
+// tile 0, origin 0); returns their product, the sample's entry count.
+__device__ __forceinline__ int tile_pieces(const BinGeom &geo, const float *c, int (&nt)[3],
+                                           int (&tile)[3][kMaxPieces], int (&local)[3][kMaxPieces]) {
+    int n = 1;
+    for (int d = 0; d < 3; ++d) {
+        nt[d] = 1;
+        tile[d][0] = local[d][0] = 0;
+        if (d < geo.ndim)
+            nt[d] = axis_pieces(axis_base(geo.ax[d], c[d]), geo.ax[d].W, geo.ax[d].G, geo.ax[d].T, tile[d], local[d]);
+        n *= nt[d];
+    }
+    return n;
+}
+
+__global__ void tiles_count_kernel(BinGeom geo, const float *__restrict__ coord, int32_t *__restrict__ counts) {
     const int64_t total = geo.npts * geo.nframes;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
          i += (int64_t)gridDim.x * blockDim.x) {
-        int base[3];
-        float w[3][kTilesMaxWidth];
-        for (int d = 0; d < 3; ++d)
-            axis_taps<kTilesMaxWidth>(coord[i * 3 + d], geo.ax[d].W, geo.ax[d].G, geo.ax[d].shift, beta_of(geo, d),
-                                      base[d], w[d]);
-        for (int d = 0; d < 3; ++d) taps[4 * i + d] = make_float4(w[d][0], w[d][1], w[d][2], w[d][3]);
-        taps[4 * i + 3] = make_float4(__int_as_float(base[0]), __int_as_float(base[1]), __int_as_float(base[2]), 0.0f);
+        int nt[3], tile[3][kMaxPieces], local[3][kMaxPieces];
+        counts[i] = tile_pieces(geo, coord + i * geo.ndim, nt, tile, local);
+    }
+}
+
+// Tile gridding entries of every sample, keyed by (frame, tile): value =
+// (sample within its frame, tile-local origin + 16 per axis in bytes).
+__global__ void tiles_emit_kernel(BinGeom geo, const float *__restrict__ coord, const int32_t *__restrict__ offsets,
+                                  uint32_t *__restrict__ keys, uint64_t *__restrict__ vals) {
+    const int64_t total = geo.npts * geo.nframes;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t frame = i / geo.npts;
+        const uint32_t p = (uint32_t)(i - frame * geo.npts);
+        int nt[3], tile[3][kMaxPieces], local[3][kMaxPieces];
+        tile_pieces(geo, coord + i * geo.ndim, nt, tile, local);
+        int32_t pos = offsets[i];
+        for (int a = 0; a < nt[2]; ++a)
+            for (int b = 0; b < nt[1]; ++b)
+                for (int c = 0; c < nt[0]; ++c) {
+                    const int64_t t = ((int64_t)tile[2][a] * geo.NT[1] + tile[1][b]) * geo.NT[0] + tile[0][c];
+                    const uint32_t loc = (uint32_t)(local[0][c] + 16) | (uint32_t)(local[1][b] + 16) << 8 |
+                                         (uint32_t)(local[2][a] + 16) << 16;
+                    keys[pos] = (uint32_t)(frame * geo.ntiles + t);
+                    vals[pos] = ((uint64_t)loc << 32) | p;
+                    ++pos;
+                }
+    }
+}
+
+// Tap records of the tile gridding (tiles_tap_stride): the taps
+// the other gridding variants evaluate, padded with zeros.
+template <int WP>
+__global__ void tiles_taps_kernel(BinGeom geo, const float *__restrict__ coord, float *__restrict__ taps) {
+    const int64_t total = geo.npts * geo.nframes;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        float *t = taps + i * tiles_tap_stride(geo.ndim, WP);
+        for (int d = 0; d < geo.ndim; ++d) {
+            int base;
+            float w[WP];
+            axis_taps<WP>(coord[i * geo.ndim + d], geo.ax[d].W, geo.ax[d].G, geo.ax[d].shift, beta_of(geo, d), base, w);
+            for (int k = 0; k < WP; ++k) t[d * WP + k] = w[k];
+        }
     }
 }
 
@@ -423,7 +471,79 @@ int order_by_origin(const BinGeom &geo, const uint32_t *bin_keys, int64_t n, flo
     return TN_OK;
 }
 
+// Entries (sorted by (frame, tile), each tile's samples ascending: the sums'
+// fixed order) and tap records of the tile gridding.
+int build_tiles(tn_plan *plan, const BinGeom &geo, int64_t nbins, hipStream_t stream) {
+    const int64_t total = geo.npts * geo.nframes;
+    DevBuf counts, offsets, tmp;
+    TN_HIP(hipMalloc(&counts.p, sizeof(int32_t) * total));
+    TN_HIP(hipMalloc(&offsets.p, sizeof(int32_t) * total));
+    hipLaunchKernelGGL(tiles_count_kernel, dim3(grid_blocks(total)), dim3(kBlock), 0, stream, geo, plan->d_coord,
+                       (int32_t *)counts.p);
+    TN_HIP(hipGetLastError());
+    size_t scan_bytes = 0, sort_bytes = 0;
+    TN_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, scan_bytes, (int32_t *)counts.p, (int32_t *)offsets.p, (int)total,
+                                            stream));
+    TN_HIP(hipMalloc(&tmp.p, scan_bytes));
+    TN_HIP(hipcub::DeviceScan::ExclusiveSum(tmp.p, scan_bytes, (int32_t *)counts.p, (int32_t *)offsets.p, (int)total,
+                                            stream));
+    int32_t last[2] = {0, 0};
+    TN_HIP(hipMemcpyAsync(&last[0], (int32_t *)offsets.p + (total - 1), sizeof(int32_t), hipMemcpyDeviceToHost, stream));
+    TN_HIP(hipMemcpyAsync(&last[1], (int32_t *)counts.p + (total - 1), sizeof(int32_t), hipMemcpyDeviceToHost, stream));
+    TN_HIP(hipStreamSynchronize(stream));
+    const int64_t n = (int64_t)last[0] + last[1];
+    plan->nentries = n;
+    int end_bit = 1;
+    while (end_bit < 32 && ((uint64_t)1 << end_bit) < (uint64_t)nbins) ++end_bit;
+    DevBuf keys, vals, keys_sorted, sort_tmp;
+    TN_HIP(hipMalloc(&keys.p, sizeof(uint32_t) * n));
+    TN_HIP(hipMalloc(&vals.p, sizeof(uint64_t) * n));
+    TN_HIP(hipMalloc(&keys_sorted.p, sizeof(uint32_t) * n));
+    TN_HIP(hipMalloc(&plan->d_tent, sizeof(int2) * n));
+    hipLaunchKernelGGL(tiles_emit_kernel, dim3(grid_blocks(total)), dim3(kBlock), 0, stream, geo, plan->d_coord,
+                       (const int32_t *)offsets.p, (uint32_t *)keys.p, (uint64_t *)vals.p);
+    TN_HIP(hipGetLastError());
+    TN_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, (uint32_t *)keys.p, (uint32_t *)keys_sorted.p,
+                                              (uint64_t *)vals.p, (uint64_t *)plan->d_tent, (int)n, 0, end_bit, stream));
+    TN_HIP(hipMalloc(&sort_tmp.p, sort_bytes));
+    TN_HIP(hipcub::DeviceRadixSort::SortPairs(sort_tmp.p, sort_bytes, (uint32_t *)keys.p, (uint32_t *)keys_sorted.p,
+                                              (uint64_t *)vals.p, (uint64_t *)plan->d_tent, (int)n, 0, end_bit, stream));
+    hipLaunchKernelGGL(bin_offsets_kernel, dim3(grid_blocks(n + 1)), dim3(kBlock), 0, stream,
+                       (const uint32_t *)keys_sorted.p, n, nbins, plan->d_bin_off);
+    TN_HIP(hipGetLastError());
+    TN_HIP(hipMalloc(&plan->d_taps, sizeof(float) * tiles_tap_stride(geo.ndim, plan->wpad) * total));
+    hipLaunchKernelGGL(plan->wpad == 4 ? tiles_taps_kernel<4> : tiles_taps_kernel<8>, dim3(grid_blocks(total)),
+                       dim3(kBlock), 0, stream, geo, plan->d_coord, plan->d_taps);
+    TN_HIP(hipGetLastError());
+    TN_HIP(hipMemcpyAsync(plan->h_bin_off.data(), plan->d_bin_off, sizeof(int32_t) * (nbins + 1), hipMemcpyDeviceToHost,
+                          stream));
+    TN_HIP(hipStreamSynchronize(stream));  // temporaries are freed on scope exit
+    return TN_OK;
+}
+
 }  // namespace
+
+// The automatic mode grids through the tiles where the kernel has at most
+// kTilesMaxWidth taps per axis and the entries (8 bytes each, at most the
+// product of the pieces a footprint can have) and tap records fit the budget
+// and 32-bit offsets.
+bool tiles_serve(const tn_plan_params &p) {
+    uint64_t pieces = 1;
+    int wmax = 1;
+    for (int d = 3 - p.ndim; d < 3; ++d) {
+        const int T = tiles_dim(p.ndim, 2 - d);
+        wmax = std::max(wmax, p.width[d]);
+        pieces *= (p.width[d] + T - 2) / T + 2;  // tiles met, one more for a wrap
+    }
+    const uint64_t total = (uint64_t)p.nframes * (uint64_t)p.npts;
+    uint64_t tiles = p.nframes;
+    for (int d = 0; d < 3; ++d) {
+        const int T = tiles_dim(p.ndim, 2 - d);
+        tiles *= (p.grid[d] + T - 1) / T;
+    }
+    return wmax <= kTilesMaxWidth && total * pieces < (uint64_t)INT32_MAX && tiles < (uint64_t)INT32_MAX / 2 &&
+           total * 4 * tiles_tap_stride(p.ndim, tiles_pad(wmax)) + total * pieces * 8 <= 4 * kMatrixAutoBytes;
+}
 
 int build_bins(tn_plan *plan, hipStream_t stream) {
     const BinGeom geo = make_geom(plan);
@@ -450,7 +570,10 @@ int build_bins(tn_plan *plan, hipStream_t stream) {
     }
 
     // ---- gridding bins: every tile a footprint touches --------------------
-    if (plan->grid_mode == kGridMatrix) {  // gridding reads the matrix instead
+    if (plan->grid_mode == kGridTiles) {
+        int rc = build_tiles(plan, geo, nbins, stream);
+        if (rc) return rc;
+    } else if (plan->grid_mode == kGridMatrix) {  // gridding reads the matrix instead
         TN_HIP(hipMemsetAsync(plan->d_bin_off, 0, sizeof(int32_t) * (nbins + 1), stream));
         plan->nentries = 0;
         int rc = build_matrix(plan, stream);
@@ -484,20 +607,9 @@ int build_bins(tn_plan *plan, hipStream_t stream) {
                            plan->d_coord, (const int32_t *)offsets.p, (uint32_t *)keys.p,
                            (int32_t *)vals.p);
         TN_HIP(hipGetLastError());
-        // register tiles: each tile's entries in sample order (the stable
-        // sort's), the sums' fixed order
         int rc = sort_entries(geo, plan->d_coord, keys.p, vals.p, n, plan->d_bin_off,
-                              &plan->d_entries, stream,
-                              plan->grid_mode == kGridRuns    ? kOrderOrigin
-                              : plan->grid_mode == kGridTiles ? kOrderSample
-                                                              : kOrderSpread);
+                              &plan->d_entries, stream, plan->grid_mode == kGridRuns ? kOrderOrigin : kOrderSpread);
         if (rc) return rc;
-        if (plan->grid_mode == kGridTiles) {
-            TN_HIP(hipMalloc(&plan->d_taps, sizeof(float4) * 4 * total));
-            hipLaunchKernelGGL(tiles_taps_kernel, dim3(grid_blocks(total)), dim3(kBlock), 0, stream, geo,
-                               plan->d_coord, plan->d_taps);
-            TN_HIP(hipGetLastError());
-        }
         plan->h_bin_off.assign(nbins + 1, 0);
         TN_HIP(hipMemcpyAsync(plan->h_bin_off.data(), plan->d_bin_off, sizeof(int32_t) * (nbins + 1),
                               hipMemcpyDeviceToHost, stream));

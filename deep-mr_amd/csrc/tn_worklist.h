@@ -7,7 +7,38 @@
 #include <cstdint>
 #include <vector>
 
+#ifdef __HIPCC__
+#define TN_HOST_DEVICE __host__ __device__
+#else
+#define TN_HOST_DEVICE
+#endif
+
 namespace tn {
+
+// Pieces of a kernel footprint along one axis for the tile gridding: the
+// cells base .. base + W - 1 (mod G, W <= G, 0 <= base < G) as (tile, local
+// origin) pairs: cell c of a tile is tap c - local of the footprint where that
+// lies in [0, W). Cells before the wrap give the tiles they meet the origin
+// base - t T, wrapped cells base - G - t T; a tile can hold both a first and a
+// wrapped piece (grids shorter than T + W - 1), whose cells are disjoint.
+// local is in [-(W - 1), T - 1]. Returns the number of pieces, at most
+// kMaxPieces for W <= 8 and T >= 4.
+constexpr int kMaxPieces = 6;
+TN_HOST_DEVICE inline int axis_pieces(int base, int W, int G, int T, int (&tile)[kMaxPieces],
+                                      int (&local)[kMaxPieces]) {
+    int n = 0;
+    const int end = base + W;
+    const int stop = end < G ? end : G;
+    for (int t = base / T; t * T < stop && n < kMaxPieces; ++t) {
+        tile[n] = t;
+        local[n++] = base - t * T;
+    }
+    for (int t = 0; t * T < end - G && n < kMaxPieces; ++t) {
+        tile[n] = t;
+        local[n++] = base - G - t * T;
+    }
+    return n;
+}
 
 constexpr int kMatrixCoils = 16;   // widest record of the matrix gridding (coils per item)
 constexpr int kMatrixStage = 1024; // entries of a run of cells staged in LDS (also the longest short row), 3D
@@ -48,6 +79,66 @@ inline void tile_fold_items(int job, int tile, int c0, int c1, int slot, int npa
     for (int64_t k = 0; k < nsub && k * per < elems; ++k)
         fold.push_back(Item{job, tile, c0, c1, slot, nparts, (int32_t)(k * per),
                             (int32_t)std::min(elems, (k + 1) * per)});
+}
+
+constexpr int kTilesGroup = 4;  // tile-gridding items (waves) per workgroup
+constexpr int kDealXcds = 8;    // XCDs the hardware deals workgroups to in turn
+constexpr int kTilesBase = 24;  // a tile's own cost in entries, for the balance over the XCDs
+constexpr int32_t kTilesJoin = 1 << 30;  // flag of an item's unit: the workgroup's four items share the tile
+
+// Tiles of a frame in bricks (x fastest inside and over the bricks), so that
+// neighbours along every axis are near each other in the work list.
+inline std::vector<int32_t> brick_order(const int32_t (&nt)[3], int ndim) {
+    const int b[3] = {8, ndim == 3 ? 4 : 8, ndim == 3 ? 4 : 1};  // x, y, z
+    std::vector<int32_t> order;
+    order.reserve((size_t)nt[0] * nt[1] * nt[2]);
+    for (int z0 = 0; z0 < nt[2]; z0 += b[2])
+        for (int y0 = 0; y0 < nt[1]; y0 += b[1])
+            for (int x0 = 0; x0 < nt[0]; x0 += b[0])
+                for (int z = z0; z < std::min(nt[2], z0 + b[2]); ++z)
+                    for (int y = y0; y < std::min(nt[1], y0 + b[1]); ++y)
+                        for (int x = x0; x < std::min(nt[0], x0 + b[0]); ++x)
+                            order.push_back((z * nt[1] + y) * nt[0] + x);
+    return order;
+}
+
+// Work list of the tile gridding, four items per workgroup: first the
+// workgroups that share a tile (`joined`), as listed (the hardware deals
+// workgroups to the XCDs in turn, which spreads a hot tile's parts over all of
+// them), then the other tiles (`grid`, which becomes the whole list) in one
+// contiguous range per XCD, so that neighbouring tiles, which read many of the
+// same samples, share an L2. The ranges hold equal work (entries, plus
+// kTilesBase for a tile's own cost), not equal numbers of tiles: on a kooshball
+// the XCDs of the dense centre otherwise worked 1.7 times as long as the
+// average one. Shorter ranges are filled up with empty items (job -1).
+inline void tiles_deal(std::vector<Item> &joined, std::vector<Item> &grid) {
+    constexpr int64_t per = kTilesGroup, kXcds = kDealXcds;
+    const Item none{-1, 0, 0, 0, 0, 0, 0, -1};
+    std::vector<Item> rest;
+    rest.swap(grid);
+    grid.swap(joined);
+    if (rest.empty()) return;
+    while (grid.size() % (per * kXcds)) grid.push_back(none);
+    const int64_t wg = ((int64_t)rest.size() + per - 1) / per;
+    double total = 0;
+    for (const Item &it : rest) total += kTilesBase + (it.e1 - it.e0);
+    int64_t first[kXcds + 1] = {0}, longest = 0;  // workgroup ranges
+    double sum = 0;
+    int x = 0;
+    for (int64_t w = 0; w < wg; ++w) {
+        while (x + 1 < kXcds && sum >= total * (x + 1) / kXcds) first[++x] = w;
+        for (int64_t q = w * per; q < std::min<int64_t>((w + 1) * per, (int64_t)rest.size()); ++q)
+            sum += kTilesBase + (rest[q].e1 - rest[q].e0);
+    }
+    while (x < kXcds) first[++x] = wg;
+    for (x = 0; x < kXcds; ++x) longest = std::max(longest, first[x + 1] - first[x]);
+    grid.reserve(grid.size() + longest * kXcds * per);
+    for (int64_t w = 0; w < longest; ++w)
+        for (x = 0; x < kXcds; ++x)
+            for (int64_t q = 0; q < per; ++q) {
+                const int64_t from = (first[x] + w) * per + q;
+                grid.push_back(first[x] + w < first[x + 1] && from < (int64_t)rest.size() ? rest[from] : none);
+            }
 }
 
 // Matrix-gridding work of one frame, independent of the coils: a run of

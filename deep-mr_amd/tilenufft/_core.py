@@ -236,7 +236,7 @@ class NativePlan:
         return n
 
     def grid_mode_effective(self):
-        """The gridding variant the library chose (1, 2 or 3)."""
+        """The gridding variant the library chose (1 to 4)."""
         m = int(_lib.load().tn_plan_grid_mode(self.handle))
         if m < 0:
             _lib.check(m, "tn_plan_grid_mode")

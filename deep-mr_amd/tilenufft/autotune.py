@@ -27,11 +27,12 @@ def default_candidates(ndim):
     else:
         tiles = [(8, 8, 8), (8, 16, 16), (16, 16, 16), (8, 8, 32), (16, 16, 32)]
         itiles = [(4, 8, 8), (8, 8, 8), (8, 8, 16), (8, 16, 16)]
-    # register tiles (grid_mode 4) are 3D only; plans they do not fit skip them
+    # the tile gridding is grid_mode 4 in 3D, where the grid fits it, and else
+    # what the automatic mode (0) picks for kernels of up to 6 taps
     return dict(tiles=tiles, grid_chunks=[0, 1, 2, 4, 8, 16], interp_chunks=[1, 2, 4, 8, 16],
                 itiles=itiles, staged_chunks=[2, 4, 8, 16], grid_splits=[512, 1024, 2048, 4096],
                 matrix_splits=[64, 128, 256], tiles_splits=[256, 384, 512, 1024],
-                grid_modes=[3, 2, 1] if ndim == 2 else [3, 4, 2, 1])
+                grid_modes=[0, 3, 2, 1] if ndim == 2 else [3, 4, 0, 2, 1])
 
 
 def _cache_path():
@@ -96,10 +97,14 @@ def tune_batch(plans, ncoils, candidates=None, reps=5, use_cache=True, verbose=F
         # 1) gridding variant x tile, automatic chunks
         best_tile, best_t, best_gm = None, float("inf"), 0
         for gm in cand.get("grid_modes", [0]):
-            # the matrix and register-tile griddings do not use the gridding tile
-            for tile in (cand["tiles"][:1] if gm in (3, 4) else cand["tiles"]):
+            # the matrix and tile griddings do not use the gridding tile
+            for tile in (cand["tiles"][:1] if gm in (0, 3, 4) else cand["tiles"]):
+                if gm == 0 and best_gm == 4:
+                    continue  # the same variant
                 try:
                     _apply(plans, tile, 0, 0, gmode=gm)
+                    if gm == 0 and plans[0].interpolator.grid_mode_effective() != 4:
+                        continue  # a variant tried under its own number
                     b = BatchedNUFFT(plans, ncoils)
                     t = _time(lambda: b.gridding(b.grid), reps, dev)
                 except RuntimeError as exc:  # variant unsupported for this width
@@ -125,7 +130,7 @@ def tune_batch(plans, ncoils, candidates=None, reps=5, use_cache=True, verbose=F
         best_split = 0
         # (for the matrix gridding: the row length above which a whole
         # workgroup sums one cell)
-        splits = "matrix_splits" if best_gm == 3 else "tiles_splits" if best_gm == 4 else "grid_splits"
+        splits = "matrix_splits" if best_gm == 3 else "tiles_splits" if best_gm in (0, 4) else "grid_splits"
         for sp in cand.get(splits, []):
             _apply(plans, best_tile, 0, best_gc, split=sp, gmode=best_gm)
             b = BatchedNUFFT(plans, ncoils)

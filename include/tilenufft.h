@@ -67,8 +67,10 @@ typedef struct tn_plan_params {
     int32_t grid_split;   /* max samples per gridding workgroup before a hot tile
                              is split across workgroups (partials folded in a
                              fixed order); 0 = automatic, < 0 = never split   */
-    int32_t grid_mode;    /* gridding variant: 0 automatic (3 when its matrix
-                             fits in 4 GiB, else 4 where it fits, else 2
+    int32_t grid_mode;    /* gridding variant: 0 automatic (tiles as for 4, in
+                             2D and 3D, for widths <= 6 and any grid, where
+                             their entries fit the plan-memory budget, else 3
+                             when its matrix fits in 4 GiB, else 2
                              when W_y * W_x <= 36, else 1), 1 one LDS atomic per
                              tap and sample (entries spread over footprint
                              origins), 2 per-lane runs of origin-sorted
@@ -80,13 +82,16 @@ typedef struct tn_plan_params {
                              grid_chunk = coils per record, <= 16 (0: 16),
                              grid_split = row length above which one cell
                              is summed by a workgroup of its own; 4 (3D,
-                             widths <= 4, grid lengths multiples of the
-                             8x8x4 (x, y, z) tile with two or more tiles
-                             per axis) one wave per tile summing its cells
-                             in registers over the tile's samples in
-                             ascending order, per-sample taps from a plan
-                             table (64 bytes per sample), coil-minor
-                             records; grid_chunk <= 8 (0: 8); tile ignored */
+                             widths <= 4, grid lengths multiples of
+                             8x8x4 (x, y, z) with two or more such blocks
+                             per axis) one wave per 4x4x4 tile (2D,
+                             automatic: 8x8), its cells' sums formed by the
+                             matrix cores over the tile's samples in
+                             ascending order with per-sample taps from a
+                             plan table (4 bytes per padded tap and axis);
+                             a tile of many samples takes a workgroup's
+                             four waves; grid_chunk <= 32 (0: equal
+                             chunks of at most 32); tile ignored        */
     float inv_scale;    /* 1 / kernel scaling (src/deepmr/fft/_interp/plan.py:190) */
     const float *apod[3]; /* host apodization vectors of length shape[d], or
                              NULL for ones (src/deepmr/fft/nufft.py:423-447)   */
