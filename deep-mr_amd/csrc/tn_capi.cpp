@@ -830,7 +830,10 @@ int tn_interp_lowrank(tn_plan *plan, const void *grid, void *samp, int64_t nbatc
     if (rc) return rc;
     rc = check_device(plan->device);
     if (rc) return rc;
-    LaunchTables *t = plan_tables(plan, nbatch, &rc, kTablesGather);
+    // the low-rank table's interpolation items hold (coil, coefficient) planes;
+    // plans that do not stage their interpolation gather, by coil
+    LaunchTables *t = plan_tables(plan, nbatch, &rc, kTablesLowRank, ncoeff);
+    if (t && t->interp_mode != kInterpStaged) t = plan_tables(plan, nbatch, &rc, kTablesGather);
     if (!t) return rc;
     return launch_interp_lowrank(*t, (const float2 *)grid, (float2 *)samp, weight, (hipStream_t)stream, lr);
 }
