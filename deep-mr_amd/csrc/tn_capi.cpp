@@ -525,8 +525,7 @@ void destroy(tn_plan *pl) {
     if (pl->d_mnz) (void)hipFree(pl->d_mnz);
     if (pl->d_taps) (void)hipFree(pl->d_taps);
     if (pl->d_tent) (void)hipFree(pl->d_tent);
-    for (int a = 0; a < 3; ++a)
-        if (pl->d_fft_tw[a]) (void)hipFree(pl->d_fft_tw[a]);
+    if (pl->d_fft) (void)hipFree(pl->d_fft);
     for (int d = 0; d < 3; ++d)
         if (pl->d_apod[d]) (void)hipFree(pl->d_apod[d]);
     (void)hipSetDevice(cur);
@@ -726,7 +725,7 @@ int64_t tn_plan_device_bytes(const tn_plan *plan) {
         b += sizeof(float) * tiles_tap_stride(p.ndim, plan->wpad) * total + sizeof(int2) * plan->nentries;
     for (int d = 0; d < 3; ++d)
         if (plan->d_apod[d]) b += sizeof(float) * p.shape[d];
-    b += plan->fft_tw_bytes;
+    b += plan->fft_bytes;
     for (const auto &kv : plan->cache) b += kv.second.device_bytes;
     for (const auto &kv : plan->cache_gather) b += kv.second.device_bytes;
     for (const auto &kv : plan->cache_lowrank) b += kv.second.device_bytes;
@@ -875,13 +874,17 @@ int tn_crop_apod(tn_plan *plan, const void *grid, void *image, int64_t nimg, tn_
     return launch_crop_apod(plan, (const float2 *)grid, (float2 *)image, nimg, (hipStream_t)stream);
 }
 
-int tn_plan_has_fft(const tn_plan *plan) { return plan && plan->d_fft_tw[0] ? 1 : 0; }
+int tn_plan_has_fft(const tn_plan *plan) { return plan && plan->d_fft && plan->fft_direct ? 1 : 0; }
+
+int tn_plan_has_transform(const tn_plan *plan) { return plan && plan->d_fft ? 1 : 0; }
 
 int tn_fft_forward(tn_plan *plan, const void *image, void *grid, int64_t nimg, tn_stream stream) {
     clear_error();
     if (!plan) return fail(TN_E_ARG, "plan is NULL");
     if (nimg < 0) return fail(TN_E_ARG, "nimg must be >= 0");
     if (nimg > 0 && (!image || !grid)) return fail(TN_E_ARG, "NULL data pointer");
+    if (!tn_plan_has_fft(plan))
+        return fail(TN_E_ARG, "the plan has no pruned FFT (2D and 3D plans with common oversampled grid lengths, 16..1024)");
     int rc = check_device(plan->device);
     if (rc) return rc;
     return launch_fft_forward(plan, (const float2 *)image, (float2 *)grid, nimg, (hipStream_t)stream);
@@ -892,6 +895,8 @@ int tn_fft_adjoint(tn_plan *plan, void *grid, void *image, int64_t nimg, tn_stre
     if (!plan) return fail(TN_E_ARG, "plan is NULL");
     if (nimg < 0) return fail(TN_E_ARG, "nimg must be >= 0");
     if (nimg > 0 && (!image || !grid)) return fail(TN_E_ARG, "NULL data pointer");
+    if (!tn_plan_has_fft(plan))
+        return fail(TN_E_ARG, "the plan has no pruned FFT (2D and 3D plans with common oversampled grid lengths, 16..1024)");
     int rc = check_device(plan->device);
     if (rc) return rc;
     return launch_fft_adjoint(plan, (float2 *)grid, (float2 *)image, nimg, (hipStream_t)stream);
@@ -902,6 +907,8 @@ int tn_fft_z_forward(tn_plan *plan, const void *image, void *zout, int64_t nimg,
     if (!plan) return fail(TN_E_ARG, "plan is NULL");
     if (nimg < 0) return fail(TN_E_ARG, "nimg must be >= 0");
     if (nimg > 0 && (!image || !zout)) return fail(TN_E_ARG, "NULL data pointer");
+    if (plan->p.ndim != 3 || !tn_plan_has_fft(plan))
+        return fail(TN_E_ARG, "the plan has no z stage (3D plans with pruned FFT stages)");
     int rc = check_device(plan->device);
     if (rc) return rc;
     return launch_fft_z_forward(plan, (const float2 *)image, (float2 *)zout, nimg, (hipStream_t)stream);
@@ -912,9 +919,41 @@ int tn_fft_z_adjoint(tn_plan *plan, const void *zin, void *image, int64_t nimg, 
     if (!plan) return fail(TN_E_ARG, "plan is NULL");
     if (nimg < 0) return fail(TN_E_ARG, "nimg must be >= 0");
     if (nimg > 0 && (!image || !zin)) return fail(TN_E_ARG, "NULL data pointer");
+    if (plan->p.ndim != 3 || !tn_plan_has_fft(plan))
+        return fail(TN_E_ARG, "the plan has no z stage (3D plans with pruned FFT stages)");
     int rc = check_device(plan->device);
     if (rc) return rc;
     return launch_fft_z_adjoint(plan, (const float2 *)zin, (float2 *)image, nimg, (hipStream_t)stream);
+}
+
+int tn_transform_forward(tn_plan *plan, const void *image, void *grid, void *work, int64_t nimg, tn_stream stream) {
+    clear_error();
+    if (!plan) return fail(TN_E_ARG, "plan is NULL");
+    if (!plan->d_fft) return fail(TN_E_ARG, "the plan has no FFT stages");
+    if (nimg < 0) return fail(TN_E_ARG, "nimg must be >= 0");
+    const bool d3 = plan->p.ndim == 3;
+    if (nimg > 0 && (!image || !grid || (d3 && !work))) return fail(TN_E_ARG, "NULL data pointer");
+    int rc = check_device(plan->device);
+    if (rc) return rc;
+    hipStream_t s = (hipStream_t)stream;
+    if (!d3) return launch_fft_forward(plan, (const float2 *)image, (float2 *)grid, nimg, s);
+    rc = launch_fft_z_forward(plan, (const float2 *)image, (float2 *)work, nimg, s);
+    return rc ? rc : launch_fft_forward(plan, (const float2 *)work, (float2 *)grid, nimg * plan->p.grid[0], s);
+}
+
+int tn_transform_adjoint(tn_plan *plan, void *grid, void *image, void *work, int64_t nimg, tn_stream stream) {
+    clear_error();
+    if (!plan) return fail(TN_E_ARG, "plan is NULL");
+    if (!plan->d_fft) return fail(TN_E_ARG, "the plan has no FFT stages");
+    if (nimg < 0) return fail(TN_E_ARG, "nimg must be >= 0");
+    const bool d3 = plan->p.ndim == 3;
+    if (nimg > 0 && (!image || !grid || (d3 && !work))) return fail(TN_E_ARG, "NULL data pointer");
+    int rc = check_device(plan->device);
+    if (rc) return rc;
+    hipStream_t s = (hipStream_t)stream;
+    if (!d3) return launch_fft_adjoint(plan, (float2 *)grid, (float2 *)image, nimg, s);
+    rc = launch_fft_adjoint(plan, (float2 *)grid, (float2 *)work, nimg * plan->p.grid[0], s);
+    return rc ? rc : launch_fft_z_adjoint(plan, (const float2 *)work, (float2 *)image, nimg, s);
 }
 
 int tn_batch_create(tn_plan *const *plans, const int64_t *nbatch, const int64_t *grid_offset,

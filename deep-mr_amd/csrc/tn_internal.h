@@ -183,6 +183,28 @@ struct LaunchTables {
     int64_t device_bytes = 0;  // bytes of the device allocations above
 };
 
+// Line transforms of one axis: N pixels <-> L grid points, by a kernel of
+// length L (M = 0), by radices at run time (M = 0, radices.n > 0), or as chirp
+// transforms by convolutions of length M (see tn_chirp.hip).
+struct ChirpTable {  // one direction
+    const float2 *in = nullptr;   // factors of the inputs
+    const float2 *out = nullptr;  // factors of the outputs
+    const float2 *b = nullptr;    // transform of the chirp, divided by M
+};
+// Radices of a length with small factors (see tn_smooth.hip).
+constexpr int kSmoothPasses = 6;
+struct SmoothRadices {
+    int n = 0;  // passes, 0: not such an axis
+    int r[kSmoothPasses] = {};
+    int pitch = 0;  // LDS float2 per column
+};
+struct FftAxis {
+    int N = 1, L = 1, M = 0;
+    SmoothRadices radices;
+    const float2 *tw = nullptr;  // exp(-2 pi i m / L), or / M
+    ChirpTable fwd, inv;
+};
+
 }  // namespace tn
 
 struct tn_plan {
@@ -212,8 +234,10 @@ struct tn_plan {
     int grid_mode = tn::kGridSpread;  // effective gridding variant (entry order)
     int32_t *d_mrow = nullptr;  // matrix gridding: row offsets, (nframes * cells + 1)
     int2 *d_mnz = nullptr;      // matrix gridding: (sample, weight bits) sorted by (frame, cell)
-    float2 *d_fft_tw[3] = {nullptr, nullptr, nullptr};  // pruned FFT twiddles exp(-2 pi i m / G), (x, y, z); null: none
-    int64_t fft_tw_bytes = 0;
+    tn::FftAxis axis[3];        // line transforms of the FFT stages, (x, y, z)
+    float2 *d_fft = nullptr;    // their tables; null: no FFT stages
+    bool fft_direct = false;    // every axis has a kernel of its own length (the pruned stages)
+    int64_t fft_bytes = 0;
     int64_t mnnz = 0;
     int2 *d_tent = nullptr;     // tile gridding entries
     float *d_taps = nullptr;    // tile gridding: tap records, tiles_tap_stride words per sample
@@ -272,13 +296,28 @@ bool tiles_serve(const tn_plan_params &p);
 int launch_tiles(const LaunchTables &t, const float2 *samp, float2 *grid, const float *weight, hipStream_t stream,
                  const LowRank &lr, float *scratch);
 int build_matrix(tn_plan *plan, hipStream_t stream);
-// Pruned, fused oversampled-grid FFT stages (2D plans with supported lengths).
-bool fft_supported(const tn_plan *plan);
+// Pruned, fused oversampled-grid FFT stages (2D and 3D plans).
 int build_fft(tn_plan *plan, hipStream_t stream);
 int launch_fft_forward(const tn_plan *plan, const float2 *image, float2 *grid, int64_t nimg, hipStream_t stream);
 int launch_fft_adjoint(const tn_plan *plan, float2 *grid, float2 *image, int64_t nimg, hipStream_t stream);
 int launch_fft_z_forward(const tn_plan *plan, const float2 *image, float2 *zout, int64_t nimg, hipStream_t stream);
 int launch_fft_z_adjoint(const tn_plan *plan, const float2 *zin, float2 *image, int64_t nimg, hipStream_t stream);
+// Lengths with factors up to 17 (tn_smooth.hip).
+bool smooth_radices(int L, SmoothRadices &f);
+int smooth_prepare(const FftAxis &a);
+int smooth_rows(const FftAxis &a, bool inverse, float2 *data, int64_t nlines, hipStream_t stream);
+int smooth_cols(const FftAxis &a, bool inverse, const float2 *src, float2 *dst, int64_t nimg, int cols, int pitch,
+                int hx, const float *apx, const float *apy, float scale, hipStream_t stream);
+// Chirp transforms (tn_chirp.hip): the convolution length of an axis (0:
+// none), its tables in float2 (appended to `host`; chirp_bind sets the
+// pointers for a table that starts at `base`), and the stages.
+int chirp_length(int N, int L);
+void chirp_tables(const FftAxis &a, std::vector<float2> &host);
+void chirp_bind(FftAxis &a, const float2 *base);
+int chirp_prepare(const FftAxis &a);
+int chirp_rows(const FftAxis &a, bool inverse, float2 *data, int64_t nlines, hipStream_t stream);
+int chirp_cols(const FftAxis &a, bool inverse, const float2 *src, float2 *dst, int64_t nimg, int cols, int pitch,
+               int hx, const float *apx, const float *apy, float scale, hipStream_t stream);
 int count_footprint(tn_plan *plan, hipStream_t stream);
 
 // Variant selection shared by the table builder and the launchers.

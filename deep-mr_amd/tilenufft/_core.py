@@ -335,6 +335,37 @@ class NativePlan:
         return image
 
 
+    @property
+    def has_transform(self):
+        """True when the plan has FFT stages of its own: kernels of the grid
+        lengths (has_fft), or of any length with factors up to 17 (G <= 1024),
+        or chirp transforms (N + G - 1 <= 1536); not for 1D plans."""
+        return bool(_lib.load().tn_plan_has_transform(self.handle))
+
+    def _transform_work(self, nimg):
+        if self.ndim < 3:
+            return None
+        return torch.empty((nimg, self.grid[0], *self.shape[1:]), dtype=torch.complex64, device=self.device)
+
+    def transform_forward(self, image, grid, nimg):
+        """image (nimg, *N) -> grid (nimg, *G): apodize, pad and forward DFT
+        (3D: z first, through a (nimg, Gz, Ny, Nx) workspace)."""
+        with torch.cuda.device(self.device):
+            work = self._transform_work(nimg)
+            _lib.check(_lib.load().tn_transform_forward(self.handle, ptr(image), ptr(grid), ptr(work), int(nimg),
+                                                        stream_ptr(self.device)), "tn_transform_forward")
+        return grid
+
+    def transform_adjoint(self, grid, image, nimg):
+        """grid (nimg, *G) -> image (nimg, *N): inverse DFT (1 / prod(G)), crop
+        and apodize; ``grid`` is overwritten."""
+        with torch.cuda.device(self.device):
+            work = self._transform_work(nimg)
+            _lib.check(_lib.load().tn_transform_adjoint(self.handle, ptr(grid), ptr(image), ptr(work), int(nimg),
+                                                        stream_ptr(self.device)), "tn_transform_adjoint")
+        return image
+
+
 def _destroy(handle, device):
     try:
         with torch.cuda.device(device):

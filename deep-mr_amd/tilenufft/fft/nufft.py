@@ -5,9 +5,9 @@ Mirrors ``src/deepmr/fft/nufft.py``: ``plan_nufft``, ``apply_nufft``,
 argument meaning, tensor layouts, dtype casts and numpy-in / numpy-out
 behaviour. The compute chain per direction is three device steps:
 
-  forward  tn_fft_forward (apodize, pad, pruned 2D DFT) -> tn_interp
-  adjoint  tn_grid -> tn_fft_adjoint (pruned inverse 2D DFT, crop, apodize)
-  (plans without the pruned FFT stages, e.g. 3D: tn_apod_pad / tn_crop_apod
+  forward  tn_transform_forward (apodize, pad, pruned DFT) -> tn_interp
+  adjoint  tn_grid -> tn_transform_adjoint (pruned inverse DFT, crop, apodize)
+  (plans without FFT stages, 1D and very long axes: tn_apod_pad / tn_crop_apod
   around torch.fft on the device)
 
 The centring shifts of deepmr's ``fft``/``ifft`` and the zero-pad / crop are
@@ -404,8 +404,8 @@ def _apply_nufft(image, nufft_plan, basis_adjoint, weight, device, threadsperblo
     native = plan.interpolator
     with torch.cuda.device(dev):
         grid = torch.empty((nimg, *plan.os_shape), dtype=torch.complex64, device=dev)
-        if native.has_fft:
-            k = native.fft_forward(x, grid, nimg)
+        if native.has_transform:
+            k = native.transform_forward(x, grid, nimg)
         else:
             native.apod_pad(x, grid, nimg)
             k = torch.fft.fftn(grid, dim=tuple(range(-ndim, 0)))
@@ -476,8 +476,8 @@ def _apply_nufft_adj(kspace, nufft_plan, basis, weight, device, threadsperblock)
     with torch.cuda.device(dev):
         nimg = nbatch * nimgax
         img = torch.empty((nimg, *plan.shape), dtype=torch.complex64, device=dev)
-        if plan.interpolator.has_fft:
-            plan.interpolator.fft_adjoint(grid, img, nimg)
+        if plan.interpolator.has_transform:
+            plan.interpolator.transform_adjoint(grid, img, nimg)
         else:
             img_g = torch.fft.ifftn(grid, dim=tuple(range(-ndim, 0)))
             plan.interpolator.crop_apod(img_g, img, nimg)

@@ -486,16 +486,16 @@ class ReconServer:
 
 
 def _fft_forward(native, images, grid, nimg):
-    if native.has_fft:
-        native.fft_forward(images, grid, nimg)
+    if native.has_transform:
+        native.transform_forward(images, grid, nimg)
     else:
         native.apod_pad(images, grid, nimg)
         grid.copy_(torch.fft.fftn(grid, dim=(-2, -1)))
 
 
 def _fft_adjoint(native, grid, images, nimg):
-    if native.has_fft:
-        native.fft_adjoint(grid, images, nimg)
+    if native.has_transform:
+        native.transform_adjoint(grid, images, nimg)
     else:
         native.crop_apod(torch.fft.ifftn(grid, dim=(-2, -1)), images, nimg)
 

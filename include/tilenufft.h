@@ -245,6 +245,20 @@ int tn_fft_z_forward(tn_plan *plan, const void *image, void *zout, int64_t nimg,
 int tn_fft_z_adjoint(tn_plan *plan, const void *zin, void *image, int64_t nimg,
                      tn_stream stream);
 
+/* 1 when the plan has FFT stages of any kind: 2D and 3D plans whose axes each
+ * have a kernel of their grid length (as tn_plan_has_fft), a length G <= 1024
+ * with factors up to 17, or a chirp transform (G >= 2, N + G - 1 <= 1536). */
+int tn_plan_has_transform(const tn_plan *plan);
+
+/* The whole FFT stage of such a plan, 2D or 3D: image (nimg, *N) -> grid
+ * (nimg, *G) as tn_apod_pad followed by an unnormalised FFT, and grid -> image
+ * as an inverse FFT followed by tn_crop_apod (the grid is overwritten). 3D
+ * plans take a workspace of nimg * Gz * Ny * Nx complex values (2D: NULL). */
+int tn_transform_forward(tn_plan *plan, const void *image, void *grid, void *work,
+                         int64_t nimg, tn_stream stream);
+int tn_transform_adjoint(tn_plan *plan, void *grid, void *image, void *work,
+                         int64_t nimg, tn_stream stream);
+
 /* ---- batched launches over several plans (ragged work queue) ----------
  * A batch binds `njobs` (plan, nbatch, grid offset, sample offset) tuples to
  * single launches: one interpolation launch and one gridding launch cover
