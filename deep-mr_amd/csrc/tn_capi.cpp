@@ -537,6 +537,10 @@ enum TableUse { kTablesPlain = 0, kTablesGather = 1, kTablesLowRank = 2 };
 // Tables of a plan for `nbatch` coils; low-rank tables hold nbatch * ncoeff
 // accumulator coils.
 tn::LaunchTables *plan_tables(tn_plan *plan, int64_t nbatch, int *rc, int use = kTablesPlain, int ncoeff = 1) {
+    if (plan->stages_only) {
+        *rc = fail(TN_E_ARG, "the plan holds FFT stages only, no samples");
+        return nullptr;
+    }
     auto &cache = use == kTablesGather ? plan->cache_gather : use == kTablesLowRank ? plan->cache_lowrank : plan->cache;
     const int64_t key = use == kTablesLowRank ? nbatch << 32 | ncoeff : nbatch;
     auto it = cache.find(key);
@@ -703,6 +707,37 @@ int tn_plan_create(const tn_plan_params *params, const float *coord_dev, tn_stre
     return TN_OK;
 }
 
+int tn_stages_create(int32_t ndim, const int32_t *shape, const int32_t *grid, tn_stream stream, tn_plan **out) {
+    clear_error();
+    if (!out || !shape || !grid) return fail(TN_E_ARG, "NULL argument");
+    *out = nullptr;
+    tn_plan_params p{};
+    p.ndim = ndim;
+    p.nframes = 1;
+    for (int d = 0; d < 3; ++d) {
+        const bool used = ndim >= 2 && ndim <= 3 && d >= 3 - ndim;
+        p.shape[d] = used ? shape[d - (3 - ndim)] : 1;
+        p.grid[d] = used ? grid[d - (3 - ndim)] : 1;
+        p.width[d] = 1;
+    }
+    int rc = validate(&p);
+    if (rc) return rc;
+    tn_plan *pl = new tn_plan();
+    pl->p = p;
+    pl->stages_only = true;
+    if (hipGetDevice(&pl->device) != hipSuccess) {
+        delete pl;
+        return fail(TN_E_HIP, "hipGetDevice failed");
+    }
+    rc = build_fft(pl, (hipStream_t)stream);
+    if (rc) {
+        destroy(pl);
+        return rc;
+    }
+    *out = pl;
+    return TN_OK;
+}
+
 int tn_plan_destroy(tn_plan *plan) {
     clear_error();
     destroy(plan);
@@ -744,6 +779,7 @@ int64_t tn_plan_footprint_cells(const tn_plan *plan_c) {
     clear_error();
     tn_plan *plan = const_cast<tn_plan *>(plan_c);
     if (!plan) return fail(TN_E_ARG, "plan is NULL");
+    if (plan->stages_only) return fail(TN_E_ARG, "the plan holds FFT stages only, no samples");
     if (plan->footprint < 0) {
         int rc = check_device(plan->device);
         if (rc) return rc;
@@ -956,6 +992,20 @@ int tn_transform_adjoint(tn_plan *plan, void *grid, void *image, void *work, int
     return rc ? rc : launch_fft_z_adjoint(plan, (const float2 *)work, (float2 *)image, nimg, s);
 }
 
+int tn_convolve(tn_plan *plan, const void *image, const void *kern, int64_t nkern, void *out, void *work0, void *work1,
+                int64_t nimg, tn_stream stream) {
+    clear_error();
+    if (!plan) return fail(TN_E_ARG, "plan is NULL");
+    if (!plan->d_fft) return fail(TN_E_ARG, "the plan has no FFT stages");
+    if (nimg < 0 || nkern < 1) return fail(TN_E_ARG, "nimg must be >= 0 and nkern >= 1");
+    if (nimg > 0 && (!image || !kern || !out || !work1 || (plan->p.ndim == 3 && !work0)))
+        return fail(TN_E_ARG, "NULL data pointer");
+    int rc = check_device(plan->device);
+    if (rc) return rc;
+    return launch_convolve(plan, (const float2 *)image, (const float2 *)kern, nkern, (float2 *)out, (float2 *)work0,
+                           (float2 *)work1, nimg, (hipStream_t)stream);
+}
+
 int tn_batch_create(tn_plan *const *plans, const int64_t *nbatch, const int64_t *grid_offset,
                     const int64_t *samp_offset, const int64_t *weight_offset, int32_t njobs,
                     tn_batch **out) {
@@ -977,7 +1027,7 @@ int tn_batch_create(tn_plan *const *plans, const int64_t *nbatch, const int64_t 
     int ndim = plans[0] ? plans[0]->p.ndim : 0;
     for (int k = 0; k < njobs; ++k) {
         const tn_plan *pl = plans[k];
-        if (!pl) return fail(TN_E_ARG, "plan %d is NULL", k);
+        if (!pl || pl->stages_only) return fail(TN_E_ARG, "plan %d is NULL or holds no samples", k);
         if (pl->device != device) return fail(TN_E_ARG, "plans live on different devices");
         if (pl->p.ndim != ndim) return fail(TN_E_ARG, "plans mix 2D and 3D");
         if (nbatch[k] < 1 || nbatch[k] >= INT32_MAX) return fail(TN_E_ARG, "nbatch[%d] < 1", k);

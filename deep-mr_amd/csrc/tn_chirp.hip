@@ -52,6 +52,36 @@ __global__ __launch_bounds__(kBlock) void chirp_rows_kernel(float2 *__restrict__
         });
 }
 
+// The product rows (see fft_product_kernel): the chirp factors of the grid
+// points cancel between the two transforms.
+template <int M>
+__global__ __launch_bounds__(kBlock) void chirp_product_kernel(float2 *__restrict__ data, int64_t nlines, int L, int N,
+                                                               ChirpTable f, ChirpTable b,
+                                                               const float2 *__restrict__ tw,
+                                                               const float2 *__restrict__ kern, int64_t nk) {
+    constexpr int RL = rows_per_wave(M), pitch = fft_line(M);
+    __shared__ float2 lds[kBlock / kWave * RL][pitch];
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int64_t line0 = ((int64_t)blockIdx.x * (kBlock / kWave) + wave) * RL;
+    if (line0 >= nlines) return;  // no barriers below
+    // a row past the last one reads the last and writes nothing
+    auto row = [&](int l) { return data + min(line0 + l, nlines - 1) * N; };
+    const int64_t k0 = line0 % nk;
+    auto krow = [&](int l) { return kern + (k0 + l < nk ? k0 + l : (line0 + l) % nk) * L; };
+    const float2 zero = make_float2(0.0f, 0.0f);
+    float2 *buf = lds[wave * RL];
+    chirp_lines<M, RL>(
+        lane, tw, f.b, buf, pitch, [&](int l, int i) { return i < N ? cmul(row(l)[i], f.in[i]) : zero; },
+        [&](int l, int i, float2 v) { buf[l * pitch + lds_at<M>(i)] = v; });
+    __asm__ __volatile__("" ::: "memory");
+    chirp_lines<M, RL>(
+        lane, tw, b.b, buf, pitch,
+        [&](int l, int i) { return i < L ? cmul(buf[l * pitch + lds_at<M>(i)], krow(l)[i]) : zero; },
+        [&](int l, int i, float2 v) {
+            if (line0 + l < nlines && i < N) row(l)[i] = cmul(v, b.out[i]);
+        });
+}
+
 // Column stages, as the direct ones: image columns mx0 .. mx0 + C - 1 of
 // image b <-> grid columns (mx - hx) mod Gx. INV: grid -> image.
 template <int M, int C, bool INV>
@@ -120,10 +150,12 @@ __global__ __launch_bounds__(kBlock) void chirp_cols_kernel(const float2 *__rest
 }
 
 using RowFn = void (*)(float2 *, int64_t, int, int, int, int, int, ChirpTable, const float2 *);
+using ProductFn = void (*)(float2 *, int64_t, int, int, ChirpTable, ChirpTable, const float2 *, const float2 *, int64_t);
 using ColFn = void (*)(const float2 *, float2 *, int64_t, int, int, int, int, int, const float *, const float *,
                        ChirpTable, const float2 *, float);
 struct Fns {
     RowFn rows = nullptr;
+    ProductFn product = nullptr;
     ColFn cols[2] = {nullptr, nullptr};  // forward, inverse
     int C = 0;
     size_t lds = 0;
@@ -134,6 +166,7 @@ Fns fns_for() {
     Fns f;
     f.C = col_group(M);
     f.rows = chirp_rows_kernel<M>;
+    f.product = chirp_product_kernel<M>;
     f.cols[0] = chirp_cols_kernel<M, col_group(M), false>;
     f.cols[1] = chirp_cols_kernel<M, col_group(M), true>;
     f.lds = col_lds_bytes(M);
@@ -251,6 +284,13 @@ int chirp_rows(const FftAxis &a, bool inverse, float2 *data, int64_t nlines, hip
     hipLaunchKernelGGL(fns(a.M).rows, dim3(row_blocks(nlines, a.M)), dim3(kBlock), 0, stream, data, nlines, a.L,
                        inverse ? a.L : a.N, inverse ? 0 : h, inverse ? a.N : a.L, inverse ? h : 0,
                        inverse ? a.inv : a.fwd, a.tw);
+    TN_HIP(hipGetLastError());
+    return TN_OK;
+}
+
+int chirp_product(const FftAxis &a, float2 *data, int64_t nlines, const float2 *kern, int64_t nk, hipStream_t stream) {
+    hipLaunchKernelGGL(fns(a.M).product, dim3(row_blocks(nlines, a.M)), dim3(kBlock), 0, stream, data, nlines, a.L, a.N,
+                       a.fwd, a.inv, a.tw, kern, nk);
     TN_HIP(hipGetLastError());
     return TN_OK;
 }

@@ -63,6 +63,40 @@ __global__ __launch_bounds__(kBlock) void fft_rows_kernel(float2 *__restrict__ d
     }
 }
 
+// A row's whole share of a convolution, in place on rows of the N data columns:
+// padded to L, transformed, times the row's kernel values (rows repeat after
+// nk), transformed back and cropped, without leaving the wave's LDS lines.
+template <int L>
+__global__ __launch_bounds__(kBlock) void fft_product_kernel(float2 *__restrict__ data, int64_t nlines, int N,
+                                                             const float2 *__restrict__ kern, int64_t nk,
+                                                             const float2 *__restrict__ tw) {
+    constexpr int RL = rows_per_wave(L), pitch = fft_line(L);
+    __shared__ float2 lds[kBlock / kWave * RL][pitch];
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int64_t line0 = ((int64_t)blockIdx.x * (kBlock / kWave) + wave) * RL;
+    if (line0 >= nlines) return;  // no barriers below
+    // a row past the last one reads the last and writes nothing
+    auto line = [&](int l) { return min(line0 + l, nlines - 1); };
+    auto pixel = [&](int i) { return i + N / 2 < L ? i + N / 2 : i + N / 2 - L; };  // < N: data
+    const int64_t k0 = line0 % nk;
+    auto krow = [&](int l) { return kern + (k0 + l < nk ? k0 + l : (line0 + l) % nk) * L; };
+    float2 *buf = lds[wave * RL];
+    fft_lines<L, RL, false>(
+        lane, tw, buf, pitch,
+        [&](int l, int i) {
+            const int m = pixel(i);
+            return m < N ? data[line(l) * N + m] : make_float2(0.0f, 0.0f);
+        },
+        [&](int l, int i, float2 v) { buf[l * pitch + lds_at<L>(i)] = v; });
+    __asm__ __volatile__("" ::: "memory");  // other lanes' elements below: keep the reads behind the writes
+    fft_lines<L, RL, true>(
+        lane, tw, buf, pitch, [&](int l, int i) { return cmul(buf[l * pitch + lds_at<L>(i)], krow(l)[i]); },
+        [&](int l, int i, float2 v) {
+            const int m = pixel(i);
+            if (m < N && line0 + l < nlines) data[(line0 + l) * N + m] = v;
+        });
+}
+
 // Forward column stage: image columns mx0 .. mx0 + C - 1 of image b are
 // apodized (x then y, as the separate pre-pass does), placed at their grid
 // rows in LDS, transformed along y (length L = Gy; rows without data are
@@ -201,6 +235,7 @@ __global__ __launch_bounds__(kBlock) void fft_cols_inv_kernel(const float2 *__re
 }
 
 using RowFn = void (*)(float2 *, int64_t, int, const float2 *);
+using ProductFn = void (*)(float2 *, int64_t, int, const float2 *, int64_t, const float2 *);
 using ColFwdFn = void (*)(const float2 *, float2 *, int64_t, int, int, int, int, const float *, const float *,
                           const float2 *);
 using ColInvFn = void (*)(const float2 *, float2 *, int64_t, int, int, int, int, const float *, const float *,
@@ -209,6 +244,7 @@ using ColInvFn = void (*)(const float2 *, float2 *, int64_t, int, int, int, int,
 struct FftFns {
     int L = 0;
     RowFn row_fwd = nullptr, row_inv = nullptr;
+    ProductFn product = nullptr;
     ColFwdFn col_fwd = nullptr;
     ColInvFn col_inv = nullptr;
     int C = 0;
@@ -222,6 +258,7 @@ FftFns fns_for() {
     f.C = col_group(L);
     f.row_fwd = fft_rows_kernel<L, false>;
     f.row_inv = fft_rows_kernel<L, true>;
+    f.product = fft_product_kernel<L>;
     f.col_fwd = fft_cols_fwd_kernel<L, col_group(L)>;
     f.col_inv = fft_cols_inv_kernel<L, col_group(L)>;
     f.lds = col_lds_bytes(L);
@@ -267,6 +304,15 @@ int launch_rows(const FftAxis &a, bool inverse, float2 *data, int64_t nlines, hi
     const FftFns f = fft_fns(a.L);
     hipLaunchKernelGGL(inverse ? f.row_inv : f.row_fwd, dim3(row_blocks(nlines, a.L)), dim3(kBlock), 0, stream, data,
                        nlines, a.N, a.tw);
+    TN_HIP(hipGetLastError());
+    return TN_OK;
+}
+
+int launch_product(const FftAxis &a, float2 *data, int64_t nlines, const float2 *kern, int64_t nk, hipStream_t stream) {
+    if (a.M) return chirp_product(a, data, nlines, kern, nk, stream);
+    if (a.radices.n) return smooth_product(a, data, nlines, kern, nk, stream);
+    hipLaunchKernelGGL(fft_fns(a.L).product, dim3(row_blocks(nlines, a.L)), dim3(kBlock), 0, stream, data, nlines, a.N,
+                       kern, nk, a.tw);
     TN_HIP(hipGetLastError());
     return TN_OK;
 }
@@ -371,6 +417,29 @@ int launch_fft_z_adjoint(const tn_plan *plan, const float2 *zin, float2 *image, 
     const int cols = plan->p.shape[1] * plan->p.shape[2];
     return launch_cols(plan->axis[2], true, zin, image, nimg, cols, cols, 0, nullptr, plan->d_apod[0], stream,
                        (float)(1.0 / (double)plan->p.grid[0]));
+}
+
+// Convolution of nimg images with `kern` (nkern kernels of the grid's size in
+// FFT order, image i taking kernel i mod nkern): pad, DFT, product, inverse DFT,
+// crop. The placement cancels: the columns stay in image order. work0 (3D):
+// nimg * Gz * Ny * Nx, work1: nimg * (Gz) * Gy * Nx complex values.
+int launch_convolve(const tn_plan *plan, const float2 *image, const float2 *kern, int64_t nkern, float2 *out,
+                    float2 *work0, float2 *work1, int64_t nimg, hipStream_t stream) {
+    if (nimg == 0) return TN_OK;
+    const FftAxis &x = plan->axis[0], &y = plan->axis[1], &z = plan->axis[2];
+    const bool d3 = plan->p.ndim == 3;
+    const int plane = x.N * y.N;
+    const int64_t nplanes = d3 ? nimg * z.L : nimg;
+    const double cells = (double)x.L * y.L * (d3 ? z.L : 1);
+    int rc = TN_OK;
+    if (d3) rc = launch_cols(z, false, image, work0, nimg, plane, plane, 0, nullptr, nullptr, stream);
+    if (!rc) rc = launch_cols(y, false, d3 ? work0 : image, work1, nplanes, x.N, x.N, 0, nullptr, nullptr, stream);
+    if (!rc) rc = launch_product(x, work1, nplanes * y.L, kern, nkern * (d3 ? z.L : 1) * y.L, stream);
+    if (!rc)
+        rc = launch_cols(y, true, work1, d3 ? work0 : out, nplanes, x.N, x.N, 0, nullptr, nullptr, stream,
+                         (float)(1.0 / cells));
+    if (!rc && d3) rc = launch_cols(z, true, work0, out, nimg, plane, plane, 0, nullptr, nullptr, stream);
+    return rc;
 }
 
 }  // namespace tn

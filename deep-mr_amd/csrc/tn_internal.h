@@ -236,6 +236,7 @@ struct tn_plan {
     int2 *d_mnz = nullptr;      // matrix gridding: (sample, weight bits) sorted by (frame, cell)
     tn::FftAxis axis[3];        // line transforms of the FFT stages, (x, y, z)
     float2 *d_fft = nullptr;    // their tables; null: no FFT stages
+    bool stages_only = false;   // made by tn_stages_create: no samples, bins or tables
     bool fft_direct = false;    // every axis has a kernel of its own length (the pruned stages)
     int64_t fft_bytes = 0;
     int64_t mnnz = 0;
@@ -302,10 +303,13 @@ int launch_fft_forward(const tn_plan *plan, const float2 *image, float2 *grid, i
 int launch_fft_adjoint(const tn_plan *plan, float2 *grid, float2 *image, int64_t nimg, hipStream_t stream);
 int launch_fft_z_forward(const tn_plan *plan, const float2 *image, float2 *zout, int64_t nimg, hipStream_t stream);
 int launch_fft_z_adjoint(const tn_plan *plan, const float2 *zin, float2 *image, int64_t nimg, hipStream_t stream);
+int launch_convolve(const tn_plan *plan, const float2 *image, const float2 *kern, int64_t nkern, float2 *out,
+                    float2 *work0, float2 *work1, int64_t nimg, hipStream_t stream);
 // Lengths with factors up to 17 (tn_smooth.hip).
 bool smooth_radices(int L, SmoothRadices &f);
 int smooth_prepare(const FftAxis &a);
 int smooth_rows(const FftAxis &a, bool inverse, float2 *data, int64_t nlines, hipStream_t stream);
+int smooth_product(const FftAxis &a, float2 *data, int64_t nlines, const float2 *kern, int64_t nk, hipStream_t stream);
 int smooth_cols(const FftAxis &a, bool inverse, const float2 *src, float2 *dst, int64_t nimg, int cols, int pitch,
                 int hx, const float *apx, const float *apy, float scale, hipStream_t stream);
 // Chirp transforms (tn_chirp.hip): the convolution length of an axis (0:
@@ -316,6 +320,7 @@ void chirp_tables(const FftAxis &a, std::vector<float2> &host);
 void chirp_bind(FftAxis &a, const float2 *base);
 int chirp_prepare(const FftAxis &a);
 int chirp_rows(const FftAxis &a, bool inverse, float2 *data, int64_t nlines, hipStream_t stream);
+int chirp_product(const FftAxis &a, float2 *data, int64_t nlines, const float2 *kern, int64_t nk, hipStream_t stream);
 int chirp_cols(const FftAxis &a, bool inverse, const float2 *src, float2 *dst, int64_t nimg, int cols, int pitch,
                int hx, const float *apx, const float *apy, float scale, hipStream_t stream);
 int count_footprint(tn_plan *plan, hipStream_t stream);

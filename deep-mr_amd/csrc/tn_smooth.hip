@@ -186,6 +186,42 @@ __global__ __launch_bounds__(kBlock) void smooth_rows_kernel(float2 *__restrict_
     }
 }
 
+// The product rows (see fft_product_kernel), nl rows of N per wave.
+__global__ __launch_bounds__(kBlock) void smooth_product_kernel(float2 *__restrict__ data, int64_t nlines, int L, int N,
+                                                                SmoothRadices f, const float2 *__restrict__ tw, int nl,
+                                                                const float2 *__restrict__ kern, int64_t nk) {
+    extern __shared__ float2 lds[];  // per wave: two buffers of nl lines
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int64_t line0 = ((int64_t)blockIdx.x * (kBlock / kWave) + wave) * nl;
+    if (line0 >= nlines) return;  // no barriers below
+    const int pitch = fft_line(L);
+    float2 *a = lds + wave * 2 * nl * pitch, *b = a + nl * pitch;
+    nl = (int)min((int64_t)nl, nlines - line0);
+    const float il = 1.0f / (float)L;  // the quotients below are exact (t < 2^14)
+    const int total = nl * L;
+    auto pixel = [&](int i) { return i + N / 2 < L ? i + N / 2 : i + N / 2 - L; };  // < N: data
+#pragma unroll 4
+    for (int t = lane; t < total; t += kWave) {
+        const int l = (int)(((float)t + 0.5f) * il), i = t - l * L, m = pixel(i);
+        a[l * pitch + pad8(i)] = m < N ? data[(line0 + l) * N + m] : make_float2(0.0f, 0.0f);
+    }
+    float2 *res = smooth_lines(lane, f, L, nl, pitch, a, b, tw);
+    const int64_t k0 = line0 % nk;
+#pragma unroll 4
+    for (int t = lane; t < total; t += kWave) {  // swapped for the inverse
+        const int l = (int)(((float)t + 0.5f) * il), i = t - l * L;
+        const int64_t kr = k0 + l < nk ? k0 + l : (line0 + l) % nk;
+        float2 *v = res + l * pitch + pad8(i);
+        *v = swapped<true>(cmul(*v, kern[kr * L + i]));
+    }
+    res = smooth_lines(lane, f, L, nl, pitch, res, res == a ? b : a, tw);
+#pragma unroll 4
+    for (int t = lane; t < total; t += kWave) {
+        const int l = (int)(((float)t + 0.5f) * il), i = t - l * L, m = pixel(i);
+        if (m < N) data[(line0 + l) * N + m] = swapped<true>(res[l * pitch + pad8(i)]);
+    }
+}
+
 // Column stages (see tn_fft.hip), C = 2^lc columns per workgroup, C / 4 per wave.
 template <bool INV>
 __global__ __launch_bounds__(kBlock) void smooth_cols_kernel(const float2 *__restrict__ src, float2 *__restrict__ dst,
@@ -316,6 +352,8 @@ bool smooth_radices(int L, SmoothRadices &f) {
 int smooth_prepare(const FftAxis &a) {
     for (auto fn : {smooth_rows_kernel<false>, smooth_rows_kernel<true>})
         TN_HIP(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)row_lds(1024, 1)));
+    TN_HIP(hipFuncSetAttribute((const void *)smooth_product_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)row_lds(1024, 1)));
     for (auto fn : {smooth_cols_kernel<false>, smooth_cols_kernel<true>})
         TN_HIP(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)col_lds(1024, 2)));
     return TN_OK;
@@ -327,6 +365,15 @@ int smooth_rows(const FftAxis &a, bool inverse, float2 *data, int64_t nlines, hi
     hipLaunchKernelGGL(inverse ? smooth_rows_kernel<true> : smooth_rows_kernel<false>,
                        dim3((unsigned)((nlines + rpb - 1) / rpb)), dim3(kBlock), row_lds(a.L, nl), stream, data, nlines,
                        a.L, a.N, a.radices, a.tw, nl);
+    TN_HIP(hipGetLastError());
+    return TN_OK;
+}
+
+int smooth_product(const FftAxis &a, float2 *data, int64_t nlines, const float2 *kern, int64_t nk, hipStream_t stream) {
+    const int nl = row_lines(a.L, nlines);
+    const int64_t rpb = (int64_t)nl * (kBlock / kWave);
+    hipLaunchKernelGGL(smooth_product_kernel, dim3((unsigned)((nlines + rpb - 1) / rpb)), dim3(kBlock),
+                       row_lds(a.L, nl), stream, data, nlines, a.L, a.N, a.radices, a.tw, nl, kern, nk);
     TN_HIP(hipGetLastError());
     return TN_OK;
 }

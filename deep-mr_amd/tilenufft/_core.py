@@ -366,6 +366,45 @@ class NativePlan:
         return image
 
 
+class FftStages:
+    """The FFT stages between images of ``shape`` and grids of ``grid`` (2D or
+    3D) on ``device``: a ``tn_plan`` without samples or apodization."""
+
+    def __init__(self, shape, grid, device):
+        self.ndim, self.device = len(grid), device
+        self.shape, self.grid = tuple(int(n) for n in shape), tuple(int(g) for g in grid)
+        handle = ctypes.c_void_p()
+        sizes = ctypes.c_int32 * self.ndim
+        with torch.cuda.device(device):
+            _lib.check(_lib.load().tn_stages_create(self.ndim, sizes(*self.shape), sizes(*self.grid), stream_ptr(device),
+                                                    ctypes.byref(handle)), "tn_stages_create")
+        self.handle = handle
+        self._finalizer = weakref.finalize(self, _destroy, handle.value, device)
+        self.has_transform = bool(_lib.load().tn_plan_has_transform(handle))
+
+    def convolve(self, image, kern, nkern):
+        """image (nimg, *N) convolved with the k-space kernels kern (nkern, *G):
+        a new (nimg, *N) tensor."""
+        nimg, gz = int(image.shape[0]), self.grid[0] if self.ndim == 3 else 1
+        with torch.cuda.device(self.device):
+            new = {"dtype": torch.complex64, "device": self.device}
+            work0 = torch.empty((nimg, gz, *self.shape[1:]), **new) if self.ndim == 3 else None
+            work1 = torch.empty((nimg, gz, self.grid[-2], self.shape[-1]), **new)
+            out = torch.empty((nimg, *self.shape), **new)
+            _lib.check(_lib.load().tn_convolve(self.handle, ptr(image), ptr(kern), int(nkern), ptr(out), ptr(work0),
+                                               ptr(work1), nimg, stream_ptr(self.device)), "tn_convolve")
+        return out
+
+
+
+def fft_stages(shape, grid, device):
+    """FftStages of the sizes, or None where an axis has none."""
+    if len(grid) not in (2, 3) or any(not 1 <= n <= g for n, g in zip(shape, grid)) or math.prod(grid) >= 2**31 - 1:
+        return None
+    stages = FftStages(shape, grid, device)
+    return stages if stages.has_transform else None
+
+
 def _destroy(handle, device):
     try:
         with torch.cuda.device(device):

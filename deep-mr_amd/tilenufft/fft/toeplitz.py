@@ -5,7 +5,10 @@ Drop-in for deepmr's ``plan_toeplitz_nufft`` / ``apply_nufft_selfadj``
 :609-669, src/deepmr/fft/_interp/toeplitz.py). The point-spread kernel is
 computed once with the hand-written adjoint NUFFT on a 2x grid (the low-rank
 gridding kernel when a subspace basis is given); each application is
-zero-pad -> FFT -> per-voxel product -> IFFT -> crop (rocFFT via torch).
+zero-pad -> FFT -> per-voxel product -> IFFT -> crop, in fused native stages
+(tn_convolve: only the lines that carry data, the product between the two
+transforms of a row); low-rank kernels, 1D and very long axes take the same
+steps through torch.fft.
 
 Low-rank product. deepmr's per-voxel routine (_interp/toeplitz.py:109-130,
 ``out[j] += K[i][j] * in[j]``) scales each coefficient by the column sum of
@@ -45,6 +48,24 @@ class GramMatrix:
             self._colsum = None
             self.device = str(dev)
         return self
+
+    def __getstate__(self):  # copies and files hold the kernel, not the device's stages
+        return {k: v for k, v in self.__dict__.items() if k != "_stages"}
+
+    def stages(self, shape, device):
+        """FFT stages between images of ``shape`` and the kernel's grid on
+        ``device`` (None: there are none), built on first use, the last two
+        shapes kept. They hold sizes and twiddles only, nothing of the kernel
+        or of an image."""
+        held = self.__dict__.get("_stages", ())
+        for key, st in held:
+            if key == (shape, device, self.shape):
+                return st
+        if torch.cuda.is_current_stream_capturing():
+            return None
+        st = _core.fft_stages(shape, self.shape, device)
+        self._stages = (((shape, device, self.shape), st), *held[:1])
+        return st
 
     def colsum(self):
         """(voxels, ncoeff) column sums of the low-rank kernel (deepmr's product)."""
@@ -106,8 +127,11 @@ def plan_toeplitz_nufft(coord, shape, basis=None, dcf=None, width=4, device="cpu
         kern = kern.reshape(*kern.shape[:2], -1).permute(2, 1, 0).contiguous()
     kern = kern / torch.mean(torch.abs(kern[kern != 0]))
     kern = torch.nan_to_num(kern)
-    return GramMatrix(kern, tuple(int(s) for s in kshape), ndim, str(dev), basis is not None,
+    gram = GramMatrix(kern, tuple(int(s) for s in kshape), ndim, str(dev), basis is not None,
                       lowrank_product)
+    if basis is None:
+        gram.stages(tuple(int(s) for s in shape), dev)
+    return gram
 
 
 def _kspace_product(k, kern, ndim):
@@ -124,6 +148,26 @@ def _kspace_product(k, kern, ndim):
     return (val.unsqueeze(0) * kb.unsqueeze(1)).sum(dim=2).reshape(shp)
 
 
+def _convolve(x, kern, dev):
+    """The native stages' result, or None where they do not serve: low-rank,
+    real or elsewhere-held kernels, kernels whose leading axes are not the last
+    of the image's, empty batches, tracers (which record torch's own calls)."""
+    if torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
+        return None
+    ndim, value = kern.ndim, kern.value
+    lead, klead = tuple(x.shape[:-ndim]), tuple(value.shape[:-ndim])
+    if (kern.islowrank or value.dtype != torch.complex64 or value.device != dev or x.numel() == 0
+            or tuple(value.shape[-ndim:]) != tuple(kern.shape) or lead[len(lead) - len(klead):] != klead):
+        return None
+    st = kern.stages(tuple(x.shape[-ndim:]), dev)
+    if st is None:
+        return None
+    x = x.to(torch.complex64).resolve_conj().resolve_neg()
+    y = st.convolve(x.reshape(-1, *x.shape[-ndim:]).contiguous(),
+                    value.detach().resolve_conj().resolve_neg().contiguous(), int(np.prod(klead)))
+    return y.reshape(x.shape)
+
+
 def _selfadj(image, kern):
     isnumpy = isinstance(image, np.ndarray)
     x = torch.as_tensor(image)
@@ -133,6 +177,10 @@ def _selfadj(image, kern):
     odevice = x.device
     dev = torch.device(kern.device)
     x = x.to(dev)
+    y = _convolve(x, kern, dev)
+    if y is not None:
+        y = y.to(odevice)
+        return y.numpy(force=True) if isnumpy else y
     x = resize(x, list(x.shape[:-ndim]) + list(kern.shape))
     ax = tuple(range(-ndim, 0))
     k = torch.fft.fftn(x, dim=ax, norm="ortho")

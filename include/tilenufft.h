@@ -259,6 +259,22 @@ int tn_transform_forward(tn_plan *plan, const void *image, void *grid, void *wor
 int tn_transform_adjoint(tn_plan *plan, void *grid, void *image, void *work,
                          int64_t nimg, tn_stream stream);
 
+/* A plan of FFT stages alone, between images of shape[ndim] and grids of
+ * grid[ndim] ((z, y, x) order, ndim 2 or 3), without samples or apodization:
+ * for tn_transform_* and tn_convolve; entry points that need samples refuse it. */
+int tn_stages_create(int32_t ndim, const int32_t *shape, const int32_t *grid, tn_stream stream,
+                     tn_plan **out);
+
+/* Convolution of images with kernels given in k-space (the Toeplitz normal
+ * operator, src/deepmr/fft/nufft.py:609-669): image (nimg, *N) -> out
+ * (nimg, *N) = crop(IDFT(kern * DFT(pad(image)))), unnormalised DFT and 1 /
+ * prod(G) in the inverse; kern (nkern, *G) in FFT order, image i with kernel
+ * i mod nkern. No apodization. Workspaces: work1 of nimg * [Gz *] Gy * Nx
+ * complex values, work0 (3D, else NULL) of nimg * Gz * Ny * Nx. TN_E_ARG when
+ * tn_plan_has_transform is 0. */
+int tn_convolve(tn_plan *plan, const void *image, const void *kern, int64_t nkern, void *out,
+                void *work0, void *work1, int64_t nimg, tn_stream stream);
+
 /* ---- batched launches over several plans (ragged work queue) ----------
  * A batch binds `njobs` (plan, nbatch, grid offset, sample offset) tuples to
  * single launches: one interpolation launch and one gridding launch cover
