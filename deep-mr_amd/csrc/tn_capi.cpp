@@ -1006,6 +1006,20 @@ int tn_convolve(tn_plan *plan, const void *image, const void *kern, int64_t nker
                            (float2 *)work1, nimg, (hipStream_t)stream);
 }
 
+int tn_nufft_forward(tn_plan *plan, const void *image, void *grid, void *work, void *samp, int64_t nbatch,
+                     const float *weight, tn_stream stream) {
+    if (!plan) return fail(TN_E_ARG, "plan is NULL");
+    int rc = tn_transform_forward(plan, image, grid, work, nbatch * plan->p.nframes, stream);
+    return rc ? rc : tn_interp(plan, grid, samp, nbatch, weight, stream);
+}
+
+int tn_nufft_adjoint(tn_plan *plan, const void *samp, void *grid, void *work, void *image, int64_t nbatch,
+                     const float *weight, tn_stream stream) {
+    if (!plan) return fail(TN_E_ARG, "plan is NULL");
+    int rc = tn_grid(plan, samp, grid, nbatch, weight, stream);
+    return rc ? rc : tn_transform_adjoint(plan, grid, image, work, nbatch * plan->p.nframes, stream);
+}
+
 int tn_batch_create(tn_plan *const *plans, const int64_t *nbatch, const int64_t *grid_offset,
                     const int64_t *samp_offset, const int64_t *weight_offset, int32_t njobs,
                     tn_batch **out) {

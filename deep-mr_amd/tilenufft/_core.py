@@ -6,6 +6,7 @@ host exactly as deepmr does it (float32 where deepmr is float32), and the
 device plan is then built by the native library.
 """
 
+import contextlib
 import ctypes
 import math
 import weakref
@@ -45,6 +46,14 @@ def compute_device(device=None):
 
 def stream_ptr(device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+
+
+_NO_SWITCH = contextlib.nullcontext()
+
+
+def on_device(device):
+    """Context with ``device`` current; free where it is already."""
+    return _NO_SWITCH if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 def ptr(t):
@@ -220,6 +229,10 @@ class NativePlan:
         del keep
         self.handle = handle
         self._finalizer = weakref.finalize(self, _destroy, handle.value, device)
+        # True when the plan has FFT stages of its own: kernels of the grid
+        # lengths (has_fft), or of any length with factors up to 17 (G <=
+        # 1024), or chirp transforms (N + G - 1 <= 1536); not for 1D plans
+        self.has_transform = bool(lib.tn_plan_has_transform(handle))
 
     # -- introspection -----------------------------------------------------
     def device_bytes(self):
@@ -335,13 +348,6 @@ class NativePlan:
         return image
 
 
-    @property
-    def has_transform(self):
-        """True when the plan has FFT stages of its own: kernels of the grid
-        lengths (has_fft), or of any length with factors up to 17 (G <= 1024),
-        or chirp transforms (N + G - 1 <= 1536); not for 1D plans."""
-        return bool(_lib.load().tn_plan_has_transform(self.handle))
-
     def _transform_work(self, nimg):
         if self.ndim < 3:
             return None
@@ -350,7 +356,7 @@ class NativePlan:
     def transform_forward(self, image, grid, nimg):
         """image (nimg, *N) -> grid (nimg, *G): apodize, pad and forward DFT
         (3D: z first, through a (nimg, Gz, Ny, Nx) workspace)."""
-        with torch.cuda.device(self.device):
+        with on_device(self.device):
             work = self._transform_work(nimg)
             _lib.check(_lib.load().tn_transform_forward(self.handle, ptr(image), ptr(grid), ptr(work), int(nimg),
                                                         stream_ptr(self.device)), "tn_transform_forward")
@@ -359,10 +365,30 @@ class NativePlan:
     def transform_adjoint(self, grid, image, nimg):
         """grid (nimg, *G) -> image (nimg, *N): inverse DFT (1 / prod(G)), crop
         and apodize; ``grid`` is overwritten."""
-        with torch.cuda.device(self.device):
+        with on_device(self.device):
             work = self._transform_work(nimg)
             _lib.check(_lib.load().tn_transform_adjoint(self.handle, ptr(grid), ptr(image), ptr(work), int(nimg),
                                                         stream_ptr(self.device)), "tn_transform_adjoint")
+        return image
+
+    def nufft_forward(self, image, nbatch, weight=None):
+        """image (nbatch, nframes, *N) -> samples (nbatch, nframes, npts)."""
+        nimg, new = nbatch * self.nframes, {"dtype": torch.complex64, "device": self.device}
+        with on_device(self.device):
+            grid, work = torch.empty((nimg, *self.grid), **new), self._transform_work(nimg)
+            out = torch.empty((nbatch, self.nframes, self.npts), **new)
+            _lib.check(_lib.load().tn_nufft_forward(self.handle, ptr(image), ptr(grid), ptr(work), ptr(out), nbatch,
+                                                    ptr(weight), stream_ptr(self.device)), "tn_nufft_forward")
+        return out
+
+    def nufft_adjoint(self, samp, nbatch, weight=None):
+        """samples (nbatch, nframes, npts) -> image (nbatch * nframes, *N)."""
+        nimg, new = nbatch * self.nframes, {"dtype": torch.complex64, "device": self.device}
+        with on_device(self.device):
+            grid, work = torch.empty((nimg, *self.grid), **new), self._transform_work(nimg)
+            image = torch.empty((nimg, *self.shape), **new)
+            _lib.check(_lib.load().tn_nufft_adjoint(self.handle, ptr(samp), ptr(grid), ptr(work), ptr(image), nbatch,
+                                                    ptr(weight), stream_ptr(self.device)), "tn_nufft_adjoint")
         return image
 
 
@@ -386,7 +412,7 @@ class FftStages:
         """image (nimg, *N) convolved with the k-space kernels kern (nkern, *G):
         a new (nimg, *N) tensor."""
         nimg, gz = int(image.shape[0]), self.grid[0] if self.ndim == 3 else 1
-        with torch.cuda.device(self.device):
+        with on_device(self.device):
             new = {"dtype": torch.complex64, "device": self.device}
             work0 = torch.empty((nimg, gz, *self.shape[1:]), **new) if self.ndim == 3 else None
             work1 = torch.empty((nimg, gz, self.grid[-2], self.shape[-1]), **new)
@@ -412,6 +438,32 @@ def _destroy(handle, device):
             _lib.load().tn_plan_destroy(ctypes.c_void_p(handle))
     except Exception:  # interpreter shutdown
         pass
+
+
+def apply_function(cls, *args):
+    """``cls.apply(*args)`` of a Function with setup_context. Outside of
+    functorch transforms, which need that style, a twin of the same name whose
+    forward takes the context runs the same forward, setup_context and
+    backward: torch binds the arguments of the former by their signature on
+    every call (10 us of a 50 us launch of a small transform)."""
+    if torch._C._are_functorch_transforms_active():
+        return cls.apply(*args)
+    twin = _TWINS.get(cls)
+    if twin is None:
+
+        def forward(ctx, *inputs):
+            out = cls.forward(*inputs)
+            cls.setup_context(ctx, inputs, out)
+            return out
+
+        twin = type(cls.__name__, (torch.autograd.Function,),
+                    {"forward": staticmethod(forward), "backward": staticmethod(cls.backward),
+                     "__doc__": cls.__doc__, "__module__": cls.__module__})
+        _TWINS[cls] = twin
+    return twin.apply(*args)
+
+
+_TWINS = {}
 
 
 def check_tensor(t, device, name):

@@ -72,6 +72,8 @@ _SIGNATURES = {
     "tn_plan_has_transform": (c_int32, [c_void_p]),
     "tn_transform_forward": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
     "tn_transform_adjoint": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
+    "tn_nufft_forward": (c_int32, [c_void_p] * 5 + [c_int64, c_void_p, c_void_p]),
+    "tn_nufft_adjoint": (c_int32, [c_void_p] * 5 + [c_int64, c_void_p, c_void_p]),
     "tn_stages_create": (c_int32, [c_int32, ctypes.POINTER(c_int32), ctypes.POINTER(c_int32), c_void_p,
                                    ctypes.POINTER(c_void_p)]),
     "tn_convolve": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),

@@ -81,7 +81,7 @@ class NUFFTPlan:
 
     @property
     def npts(self):
-        return int(np.prod(self.ishape))
+        return math.prod(self.ishape)
 
 
 def _build_native(plan, device, shift, coord=None):
@@ -322,7 +322,7 @@ def apply_nufft(image, nufft_plan, basis_adjoint=None, weight=None, device=None,
     returns k-space (..., ncontrasts, nviews, nsamples). ``threadsperblock``
     is accepted for compatibility; launch shapes come from the plan.
     """
-    return ApplyNUFFT.apply(image, nufft_plan, basis_adjoint, weight, device, threadsperblock)
+    return _core.apply_function(ApplyNUFFT, image, nufft_plan, basis_adjoint, weight, device, threadsperblock)
 
 
 def apply_nufft_adj(kspace, nufft_plan, basis=None, weight=None, device=None, threadsperblock=128):
@@ -331,7 +331,7 @@ def apply_nufft_adj(kspace, nufft_plan, basis=None, weight=None, device=None, th
     Like deepmr, this is the adjoint divided by prod(os_shape) (both FFTs use
     norm=None).
     """
-    return ApplyNUFFTAdjoint.apply(kspace, nufft_plan, basis, weight, device, threadsperblock)
+    return _core.apply_function(ApplyNUFFTAdjoint, kspace, nufft_plan, basis, weight, device, threadsperblock)
 
 
 # --------------------------------------------------------------------------
@@ -398,25 +398,28 @@ def _apply_nufft(image, nufft_plan, basis_adjoint, weight, device, threadsperblo
             what = "subspace coefficients" if ba is not None else "contrasts"
             raise ValueError(f"expected {nimgax} {what} before the spatial axes, got {lead}")
         batch_shape = lead[:-1]
-    nbatch = int(np.prod(batch_shape))
+    nbatch = math.prod(batch_shape)
     nimg = nbatch * nimgax
     x = x.contiguous()
     native = plan.interpolator
-    with torch.cuda.device(dev):
-        grid = torch.empty((nimg, *plan.os_shape), dtype=torch.complex64, device=dev)
-        if native.has_transform:
-            k = native.transform_forward(x, grid, nimg)
-        else:
-            native.apod_pad(x, grid, nimg)
-            k = torch.fft.fftn(grid, dim=tuple(range(-ndim, 0)))
-        del grid
-        ksp_shape = (*batch_shape, nframes, *plan.ishape) if nframes > 1 else (*batch_shape, *plan.ishape)
+    ksp_shape = (*batch_shape, nframes, *plan.ishape) if nframes > 1 else (*batch_shape, *plan.ishape)
+    with _core.on_device(dev):
         w_fused, w_bcast = _fused_weight(weight, plan, dev, (nframes, *plan.ishape) if nframes > 1 else plan.ishape)
-        out = torch.empty((nbatch, nframes, plan.npts), dtype=torch.complex64, device=dev)
-        if nbatch > 0 and ba is not None:
-            _lowrank_native(plan).interp_lowrank(k, out, nbatch, nimgax, plan.npts, ba, w_fused)
-        elif nbatch > 0:
-            native.interp(k, out, nbatch, w_fused)
+        if native.has_transform and ba is None and nbatch > 0:
+            out = native.nufft_forward(x, nbatch, w_fused)
+        else:
+            grid = torch.empty((nimg, *plan.os_shape), dtype=torch.complex64, device=dev)
+            if native.has_transform:
+                k = native.transform_forward(x, grid, nimg)
+            else:
+                native.apod_pad(x, grid, nimg)
+                k = torch.fft.fftn(grid, dim=tuple(range(-ndim, 0)))
+            del grid
+            out = torch.empty((nbatch, nframes, plan.npts), dtype=torch.complex64, device=dev)
+            if nbatch > 0 and ba is not None:
+                _lowrank_native(plan).interp_lowrank(k, out, nbatch, nimgax, plan.npts, ba, w_fused)
+            elif nbatch > 0:
+                native.interp(k, out, nbatch, w_fused)
         out = out.reshape(ksp_shape)
         if w_bcast is not None:
             out = w_bcast * out
@@ -426,21 +429,29 @@ def _apply_nufft(image, nufft_plan, basis_adjoint, weight, device, threadsperblo
     return out
 
 
+def _grid_samples(y, plan, weight, dev):
+    """k-space ``y`` as (nbatch, nframes, npts): (samples, weight to fuse or
+    None, batch_shape); other weights are applied here."""
+    nframes = plan.nframes
+    w_fused, w_bcast = _fused_weight(weight, plan, dev, (nframes, *plan.ishape) if nframes > 1 else plan.ishape)
+    if w_bcast is not None:
+        y = w_bcast * y
+    batch_shape = tuple(y.shape[:-2]) if nframes == 1 else tuple(y.shape[:-3])
+    nbatch = math.prod(batch_shape)
+    if y.numel() != nbatch * nframes * plan.npts:
+        raise ValueError(f"k-space shape {tuple(y.shape)} does not match the plan "
+                         f"({nframes} frames x {plan.npts} samples)")
+    return y.reshape(nbatch, nframes, plan.npts).contiguous(), w_fused, batch_shape
+
+
 def _grid_step(y, plan, basis, weight, dev):
     """Weighting and gridding of k-space ``y`` onto the plan's (FFT-ordered)
     grid: returns (grid (nbatch, nimgax, *os_shape), batch_shape, nimgax).
     ``nimgax`` is nframes, or ncoeff for a subspace ``basis``; a single-frame
     plan keeps coefficient 0 (grid.py:117)."""
-    ndim, nframes = plan.ndim, plan.nframes
-    w_fused, w_bcast = _fused_weight(weight, plan, dev, (nframes, *plan.ishape) if nframes > 1 else plan.ishape)
-    if w_bcast is not None:
-        y = w_bcast * y
-    batch_shape = tuple(y.shape[:-2]) if nframes == 1 else tuple(y.shape[:-3])
-    nbatch = int(np.prod(batch_shape))
-    if y.numel() != nbatch * nframes * plan.npts:
-        raise ValueError(f"k-space shape {tuple(y.shape)} does not match the plan "
-                         f"({nframes} frames x {plan.npts} samples)")
-    y = y.reshape(nbatch, nframes, plan.npts).contiguous()
+    nframes = plan.nframes
+    y, w_fused, batch_shape = _grid_samples(y, plan, weight, dev)
+    nbatch = math.prod(batch_shape)
     # low rank: the image gets ncoeff subspace coefficients per batch entry
     # (grid.py:89-104)
     nimgax = nframes
@@ -471,18 +482,23 @@ def _apply_nufft_adj(kspace, nufft_plan, basis, weight, device, threadsperblock)
     y = kspace.to(dev)
     if y.dtype != torch.complex64:
         y = y.to(torch.complex64)
-    grid, batch_shape, nimgax = _grid_step(y, plan, basis, weight, dev)
-    nbatch = int(np.prod(batch_shape))
-    with torch.cuda.device(dev):
-        nimg = nbatch * nimgax
-        img = torch.empty((nimg, *plan.shape), dtype=torch.complex64, device=dev)
-        if plan.interpolator.has_transform:
-            plan.interpolator.transform_adjoint(grid, img, nimg)
+    native = plan.interpolator
+    with _core.on_device(dev):
+        if native.has_transform and basis is None:
+            y, w_fused, batch_shape = _grid_samples(y, plan, weight, dev)
+            nbatch, nimgax = math.prod(batch_shape), nframes
+            img = native.nufft_adjoint(y, nbatch, w_fused) if nbatch > 0 else y.new_empty((0, *plan.shape))
         else:
-            img_g = torch.fft.ifftn(grid, dim=tuple(range(-ndim, 0)))
-            plan.interpolator.crop_apod(img_g, img, nimg)
-            del img_g
-        del grid
+            grid, batch_shape, nimgax = _grid_step(y, plan, basis, weight, dev)
+            nimg = math.prod(batch_shape) * nimgax
+            img = torch.empty((nimg, *plan.shape), dtype=torch.complex64, device=dev)
+            if native.has_transform:
+                native.transform_adjoint(grid, img, nimg)
+            else:
+                img_g = torch.fft.ifftn(grid, dim=tuple(range(-ndim, 0)))
+                native.crop_apod(img_g, img, nimg)
+                del img_g
+            del grid
         shape = (*batch_shape, nimgax, *plan.shape) if nframes > 1 else (*batch_shape, *plan.shape)
         img = img.reshape(shape)
     img = img.to(odevice)

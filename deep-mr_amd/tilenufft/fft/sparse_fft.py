@@ -173,7 +173,7 @@ def apply_sparse_fft(image, sampling_mask, basis_adjoint=None, weight=None, devi
     (..., [ncontrasts], *shape) -> k-space (..., [ncontrasts], nviews, nsamples).
     With ``basis_adjoint`` (ncontrasts, ncoeff) the image holds ncoeff
     subspace coefficients in place of the contrasts."""
-    return ApplySparseFFT.apply(image, sampling_mask, basis_adjoint, weight, device, threadsperblock)
+    return _core.apply_function(ApplySparseFFT, image, sampling_mask, basis_adjoint, weight, device, threadsperblock)
 
 
 class ApplySparseIFFT(torch.autograd.Function):
@@ -209,7 +209,7 @@ def apply_sparse_ifft(kspace, sampling_mask, basis=None, weight=None, device=Non
     """Sparse IFFT (src/deepmr/fft/sparse_fft.py:223-258): k-space
     (..., [ncontrasts], nviews, nsamples) -> image; ``basis`` (ncoeff,
     ncontrasts) returns ncoeff subspace coefficients."""
-    return ApplySparseIFFT.apply(kspace, sampling_mask, basis, weight, device, threadsperblock)
+    return _core.apply_function(ApplySparseIFFT, kspace, sampling_mask, basis, weight, device, threadsperblock)
 
 
 @dataclass
@@ -316,4 +316,4 @@ def apply_sparse_fft_selfadj(image, toeplitz_kern, device=None, threadsperblock=
     """Self-adjoint sparse FFT via the Toeplitz kernel (sparse_fft.py:261-292, :459-503)."""
     if device is not None:
         toeplitz_kern.to(device)
-    return ApplySparseFFTSelfadjoint.apply(image, toeplitz_kern, device, threadsperblock)
+    return _core.apply_function(ApplySparseFFTSelfadjoint, image, toeplitz_kern, device, threadsperblock)

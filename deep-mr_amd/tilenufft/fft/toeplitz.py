@@ -212,4 +212,4 @@ def apply_nufft_selfadj(image, toeplitz_kern, device=None, threadsperblock=128):
     """Apply A^H A through the Toeplitz kernel (src/deepmr/fft/nufft.py:351-375, :609-669)."""
     if device is not None:
         toeplitz_kern.to(device)
-    return ApplyNUFFTSelfAdjoint.apply(image, toeplitz_kern, device, threadsperblock)
+    return _core.apply_function(ApplyNUFFTSelfAdjoint, image, toeplitz_kern, device, threadsperblock)

@@ -259,6 +259,15 @@ int tn_transform_forward(tn_plan *plan, const void *image, void *grid, void *wor
 int tn_transform_adjoint(tn_plan *plan, void *grid, void *image, void *work,
                          int64_t nimg, tn_stream stream);
 
+/* Whole transforms of plans with FFT stages: tn_transform_forward then tn_interp,
+ * and tn_grid then tn_transform_adjoint, of nbatch coils and every frame
+ * (images (nbatch, nframes, *N), samples (nbatch, nframes, npts)); grid is the
+ * (nbatch, nframes, *G) workspace between them, work as tn_transform_*. */
+int tn_nufft_forward(tn_plan *plan, const void *image, void *grid, void *work, void *samp,
+                     int64_t nbatch, const float *weight, tn_stream stream);
+int tn_nufft_adjoint(tn_plan *plan, const void *samp, void *grid, void *work, void *image,
+                     int64_t nbatch, const float *weight, tn_stream stream);
+
 /* A plan of FFT stages alone, between images of shape[ndim] and grids of
  * grid[ndim] ((z, y, x) order, ndim 2 or 3), without samples or apodization:
  * for tn_transform_* and tn_convolve; entry points that need samples refuse it. */
