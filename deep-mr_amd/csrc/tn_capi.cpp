@@ -439,6 +439,22 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
                                       : 0;
     t.grid_lds = lds_grid ? grid_lds_bytes(max_gc, max_plane, wc, gmode, gndim) : 0;
     t.interp_lds = mode == kInterpStaged ? region_coil * (size_t)max_ic + rows_bytes : 0;
+    if (mode == kInterpStaged) {
+        bool fits = wc <= staged_width(gndim), even = true;
+        int64_t cells = 0, lds = 0;  // of a region: loaded in pairs, held at an odd row pitch
+        for (const Job &j : jobs) {
+            const int64_t rows = (int64_t)(j.IT[1] + j.W[1] - 1) * (j.IT[2] + j.W[2] - 1);
+            cells = std::max<int64_t>(cells, rows * ((j.IT[0] + j.W[0]) / 2 * 2));
+            lds = std::max<int64_t>(lds, rows * ((j.IT[0] + j.W[0] - 1) | 1));
+            fits = fits && (int64_t)j.G[0] * j.G[1] * j.G[2] < (1ll << 29);  // 32-bit byte offsets
+            even = even && j.G[0] % 2 == 0 && (j.IT[0] % 2 == 0 || j.INT_[0] == 1) && j.grid_off % 2 == 0 &&
+                   j.grid_bstride % 2 == 0;
+        }
+        fits = fits && max_ic <= staged_coils(gndim) && cells <= staged_cells(gndim, wc) &&
+               sizeof(float2) * (size_t)lds * max_ic <= kInterpLdsBudget;
+        t.interp_vec = !fits ? 0 : even ? 2 : gndim == 2 ? 1 : 0;
+        if (t.interp_vec) t.interp_lds = std::max(t.interp_lds, sizeof(float2) * (size_t)lds * max_ic);
+    }
     t.interp_coils = max_ic;
     const int rc = upload_tables(jobs_st, interp, grid, fold, slot_base, t);
     t.device_bytes += copy_bytes;
@@ -486,12 +502,6 @@ void choose_tiles(tn_plan *pl) {
     } else {
         def[0] = 16; def[1] = 16; def[2] = 16;
     }
-    int idef[3];  // default staged-interpolation tiles (z, y, x): measured fastest with the default coil chunks
-    if (p.ndim == 2) {
-        idef[0] = 1; idef[1] = 16; idef[2] = 16;
-    } else {
-        idef[0] = 8; idef[1] = 8; idef[2] = 16;
-    }
     pl->ntiles_total = 1;
     pl->nitiles_total = 1;
     for (int d = 0; d < 3; ++d) {
@@ -500,7 +510,7 @@ void choose_tiles(tn_plan *pl) {
         pl->tile[d] = t;
         pl->ntiles[d] = (p.grid[d] + t - 1) / t;
         pl->ntiles_total *= pl->ntiles[d];
-        int it = p.itile[d] > 0 ? p.itile[d] : idef[d];
+        int it = p.itile[d] > 0 ? p.itile[d] : staged_tile(p.ndim, 2 - d);
         it = std::min(it, p.grid[d]);
         pl->itile[d] = it;
         pl->nitiles[d] = (p.grid[d] + it - 1) / it;

@@ -35,6 +35,20 @@ constexpr int kLoadBatch = 4;  // global loads per lane issued before their LDS 
 // 2 coils 1.33 ms vs 3 coils 1.61 ms)
 constexpr int kInterpChunk2d = 8;
 constexpr int kInterpChunk3d = 2;
+// Default staged-interpolation tiles (measured fastest with the chunks above).
+constexpr int staged_tile(int ndim, int axis) {  // axis: 0 x, 1 y, 2 z
+    return axis == 0 ? 16 : axis == 1 ? (ndim == 3 ? 8 : 16) : ndim == 3 ? 8 : 1;
+}
+// Most coils per chunk, taps and cells per region (rows rounded up to pairs)
+// of the staged interpolation's register-addressed loads: the default chunks
+// and the regions of the default tiles, in steps of a pair per lane.
+constexpr int staged_coils(int ndim) { return ndim == 3 ? kInterpChunk3d : kInterpChunk2d; }
+constexpr int staged_width(int ndim) { return ndim == 3 ? 5 : 6; }
+constexpr int staged_cells(int ndim, int wc) {
+    const int pairs = (staged_tile(ndim, 0) + wc) / 2 * (staged_tile(ndim, 1) + wc - 1) *
+                      (ndim == 3 ? staged_tile(ndim, 2) + wc - 1 : 1);
+    return (pairs + kBlock - 1) / kBlock * kBlock * 2;
+}
 constexpr int interp_segment(int ndim) { return 256 * staged_ept(ndim); }  // samples per staged work item
 constexpr int kGridSplitDefault = 2048;  // max tile entries per gridding workgroup
 constexpr int kGridBatch = 256;  // tile entries staged in LDS per gridding batch
@@ -179,6 +193,7 @@ struct LaunchTables {
     int64_t st_elems = 0;
     int st_cw = 0;  // 0: the lane-per-cell matrix kernel reads the samples in place
     int wpad = 0;   // tile gridding: words per axis of the tap records
+    int interp_vec = 0;  // staged interpolation: cells per load (2, 1), 0: row by row
     int st_cpl = 1; // coils per lane of the matrix kernel over the copy (1 or 2)
     int64_t device_bytes = 0;  // bytes of the device allocations above
 };

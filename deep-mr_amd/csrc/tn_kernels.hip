@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "tn_internal.h"
 #include "tn_kb.h"
@@ -75,6 +76,7 @@ __device__ __forceinline__ int64_t xcd_item(int64_t nitems) {
 // Clang vector types for the nontemporal load/store builtins.
 typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 template <int NDIM, int WC>
 struct Taps {
@@ -312,7 +314,19 @@ __device__ __forceinline__ void staged_taps2(const float2 *r0, const float2 *r1,
 // (400 spirals x 1000 samples, 8 coils, 5 coefficients, 240^2 grid: gathering
 // every plane's taps through L1/L2 took 0.80 ms, bound by one address per
 // lane and tap; staged 0.11 ms.)
-template <int NDIM, int WC, bool LR>
+// Region loads (VEC): every lane keeps the grid offsets of its cells of the
+// region, formed once per item, so that a coil's load is one wide load per
+// kBlock * VEC cells (VEC = 2: 16 bytes, where rows and tiles start on even
+// cells) and its LDS writes; the index arithmetic of the row-by-row load,
+// repeated for each coil, took a third of the instructions. Regions have odd
+// row pitches (rows on distinct banks), and in 3D the next chunk's loads are in
+// flight during the tap sums. Row by row -> this: 8 x 16 spirals on 512^2 120
+// -> 111 us, 20 frames of 240^2, 6 taps 53 -> 44 us, 5.1 M samples of 8 coils
+// of 256^3 898 -> 810 us (836 without the loads ahead; 906 held to 128
+// registers). VEC = 0, row by row: larger regions than the default tiles' or
+// larger chunks (where asked for), wider kernels, and in 3D grids of odd rows
+// (8-byte loads take twice the registers: 61x101x84 65 -> 70 us).
+template <int NDIM, int WC, bool LR, int VEC>
 __global__ __launch_bounds__(kBlock) void interp_staged_kernel(const Job *__restrict__ jobs,
                                                                const Item *__restrict__ items, int64_t nitems,
                                                                const float2 *__restrict__ grid,
@@ -330,7 +344,8 @@ __global__ __launch_bounds__(kBlock) void interp_staged_kernel(const Job *__rest
     const int ty = (tile / J.INT_[0]) % J.INT_[1];
     const int tz = tile / (J.INT_[0] * J.INT_[1]);
     const int ox = tx * Tx, oy = ty * Ty, oz = tz * Tz;
-    const int Rx = Tx + J.W[0] - 1, Ry = Ty + J.W[1] - 1, Rz = Tz + J.W[2] - 1;
+    // Rx: region row pitch, odd for VEC > 0 (rows on distinct banks)
+    const int rx = Tx + J.W[0] - 1, Rx = VEC > 0 ? rx | 1 : rx, Ry = Ty + J.W[1] - 1, Rz = Tz + J.W[2] - 1;
     const int Gx = J.G[0], Gy = J.G[1], Gz = J.G[2];
     const int cells = Rx * Ry * Rz;
     const int nx = J.W[0], ny = NDIM > 1 ? J.W[1] : 1, nz = NDIM > 2 ? J.W[2] : 1;
@@ -379,6 +394,100 @@ __global__ __launch_bounds__(kBlock) void interp_staged_kernel(const Job *__rest
         }
     }
 
+    // every axis at the full compiled width: branch-free tap sums
+    const bool full = nx == WC && (NDIM < 2 || ny == WC) && (NDIM < 3 || nz == WC);
+    // the tap sums of planes cc .. cc + ncoil - 1, which the region holds
+    auto sums = [&](int cc, int ncoil) {
+#pragma unroll
+        for (int q = 0; q < kStagedEpt; ++q) {
+            if (loc[q] < 0) continue;
+            // plane cc + b's tap sum: the coil's sample, or (LR) its term
+            auto put = [&](int b, float2 t) {
+                int coil = cc + b;
+                if (LR) {
+                    const int k = coil % lr.ncoeff;
+                    coil /= lr.ncoeff;
+                    const float2 w = basis[q][k];
+                    sum[q].x += w.x * t.x - w.y * t.y;
+                    sum[q].y += w.x * t.y + w.y * t.x;
+                    if (k + 1 < lr.ncoeff) return;
+                    t = sum[q];
+                    sum[q] = make_float2(0.0f, 0.0f);
+                }
+                samp[J.samp_off + (int64_t)coil * J.samp_bstride + pnt[q]] = make_float2(t.x * scl[q], t.y * scl[q]);
+            };
+            int b = 0;
+            for (; b + 2 <= ncoil; b += 2) {  // plane pairs share each tap's weight
+                const float2 *r = region + (size_t)b * cells + loc[q];
+                float2 t0, t1;
+                if (full)
+                    staged_taps2<NDIM, WC, true>(r, r + cells, w[q], nx, ny, nz, Rx, Ry, t0, t1);
+                else
+                    staged_taps2<NDIM, WC, false>(r, r + cells, w[q], nx, ny, nz, Rx, Ry, t0, t1);
+                put(b, t0);
+                put(b + 1, t1);
+            }
+            if (b < ncoil) {
+                const float2 *r = region + (size_t)b * cells + loc[q];
+                put(b, full ? staged_taps<NDIM, WC, true>(r, w[q], nx, ny, nz, Rx, Ry)
+                            : staged_taps<NDIM, WC, false>(r, w[q], nx, ny, nz, Rx, Ry));
+            }
+        }
+    };
+    if constexpr (VEC > 0) {
+        using V = std::conditional_t<VEC == 2, f32x4, f32x2>;
+        constexpr bool AHEAD = NDIM > 2;  // load the next chunk during the sums
+        constexpr int CH = staged_coils(NDIM), K = staged_cells(NDIM, WC) / (kBlock * VEC);
+        const int per_row = (rx + VEC - 1) / VEC, pieces = per_row * Ry * Rz;
+        uint32_t off[K];  // bytes; a grid is smaller than 4 GiB here
+        int at[K];        // 2 * (cell of the region) + 1 where a pair's second cell is not of the row; -1: none
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int i = (int)threadIdx.x + k * kBlock;
+            const int r = i / per_row, c = (i - r * per_row) * VEC;
+            const int z = NDIM > 2 ? r / Ry : 0, y = r - z * Ry;
+            const bool ok = i < pieces;
+            off[k] = ok ? (uint32_t)((((oz + z) % Gz) * Gy + (oy + y) % Gy) * Gx + (ox + c) % Gx) * (uint32_t)sizeof(float2) : 0;
+            at[k] = ok ? 2 * (r * Rx + c) + (c + 1 >= rx ? 1 : 0) : -1;
+        }
+        V v[CH][K];
+        auto fetch = [&](int cc) {
+            const char *g = (const char *)(grid + J.grid_off + (int64_t)cc * J.grid_bstride);
+            const int ncoil = min(chunk, it.c1 - cc);
+#pragma unroll
+            for (int b = 0; b < CH; ++b) {
+                if (b < ncoil) {
+#pragma unroll
+                    for (int k = 0; k < K; ++k)
+                        if (k * kBlock < pieces) v[b][k] = *(const V *)(g + off[k]);
+                }
+                g += J.grid_bstride * sizeof(float2);
+            }
+        };
+        if (AHEAD) fetch(it.c0);
+        for (int cc = it.c0; cc < it.c1; cc += chunk) {
+            const int ncoil = min(chunk, it.c1 - cc);
+            if (!AHEAD) fetch(cc);
+            __syncthreads();  // previous chunk consumed
+#pragma unroll
+            for (int b = 0; b < CH; ++b)
+                if (b < ncoil) {
+#pragma unroll
+                    for (int k = 0; k < K; ++k) {
+                        if (at[k] < 0) continue;
+                        float2 *r = region + b * cells + (at[k] >> 1);
+                        r[0] = make_float2(v[b][k][0], v[b][k][1]);
+                        if constexpr (VEC == 2)
+                            if (!(at[k] & 1)) r[1] = make_float2(v[b][k][2], v[b][k][3]);
+                    }
+                }
+            __syncthreads();
+            if (AHEAD && cc + chunk < it.c1) fetch(cc + chunk);
+            sums(cc, ncoil);
+        }
+        return;
+    }
+
     // wrapped grid offset of the first cell of each (z, y) row of the region,
     // once per item, in the LDS words after the chunk's region
     int *rowtab = reinterpret_cast<int *>(region + (size_t)chunk * cells);
@@ -394,8 +503,6 @@ __global__ __launch_bounds__(kBlock) void interp_staged_kernel(const Job *__rest
     const int rr = rowwise ? (int)threadIdx.x / Rx : 0;
     const int xl = (int)threadIdx.x - rr * Rx;
     const int xoff = (ox + xl) % Gx;
-    // every axis at the full compiled width: branch-free tap sums
-    const bool full = nx == WC && (NDIM < 2 || ny == WC) && (NDIM < 3 || nz == WC);
     for (int cc = it.c0; cc < it.c1; cc += chunk) {
         const int ncoil = min(chunk, it.c1 - cc);
         __syncthreads();  // previous chunk consumed; the row table written
@@ -445,41 +552,7 @@ __global__ __launch_bounds__(kBlock) void interp_staged_kernel(const Job *__rest
             }
         }
         __syncthreads();
-#pragma unroll
-        for (int q = 0; q < kStagedEpt; ++q) {
-            if (loc[q] < 0) continue;
-            // plane cc + b's tap sum: the coil's sample, or (LR) its term
-            auto put = [&](int b, float2 t) {
-                int coil = cc + b;
-                if (LR) {
-                    const int k = coil % lr.ncoeff;
-                    coil /= lr.ncoeff;
-                    const float2 w = basis[q][k];
-                    sum[q].x += w.x * t.x - w.y * t.y;
-                    sum[q].y += w.x * t.y + w.y * t.x;
-                    if (k + 1 < lr.ncoeff) return;
-                    t = sum[q];
-                    sum[q] = make_float2(0.0f, 0.0f);
-                }
-                samp[J.samp_off + (int64_t)coil * J.samp_bstride + pnt[q]] = make_float2(t.x * scl[q], t.y * scl[q]);
-            };
-            int b = 0;
-            for (; b + 2 <= ncoil; b += 2) {  // plane pairs share each tap's weight
-                const float2 *r = region + (size_t)b * cells + loc[q];
-                float2 t0, t1;
-                if (full)
-                    staged_taps2<NDIM, WC, true>(r, r + cells, w[q], nx, ny, nz, Rx, Ry, t0, t1);
-                else
-                    staged_taps2<NDIM, WC, false>(r, r + cells, w[q], nx, ny, nz, Rx, Ry, t0, t1);
-                put(b, t0);
-                put(b + 1, t1);
-            }
-            if (b < ncoil) {
-                const float2 *r = region + (size_t)b * cells + loc[q];
-                put(b, full ? staged_taps<NDIM, WC, true>(r, w[q], nx, ny, nz, Rx, Ry)
-                            : staged_taps<NDIM, WC, false>(r, w[q], nx, ny, nz, Rx, Ry));
-            }
-        }
+        sums(cc, ncoil);
     }
 }
 
@@ -1496,17 +1569,33 @@ InterpFn pick_interp(int wc) {
     }
 }
 
+template <int NDIM, int WC, bool LR>
+StagedFn staged_fn(int vec) {
+    if constexpr (WC <= staged_width(NDIM)) {
+        if (vec == 2) return interp_staged_kernel<NDIM, WC, LR, 2>;
+        if constexpr (NDIM == 2)
+            if (vec == 1) return interp_staged_kernel<NDIM, WC, LR, 1>;
+    }
+    return vec == 0 ? interp_staged_kernel<NDIM, WC, LR, 0> : nullptr;
+}
+
+// Cells per load for a grid at this address.
+int staged_vec(const LaunchTables &t, const float2 *grid) {
+    if (t.interp_vec < 2 || (uintptr_t)grid % sizeof(f32x4) == 0) return t.interp_vec;
+    return kind_ndim(t.kind_interp) == 2 ? 1 : 0;
+}
+
 template <int NDIM, bool LR>
-StagedFn pick_staged(int wc) {
+StagedFn pick_staged(int wc, int vec) {
     switch (wc) {
-        case 1: return interp_staged_kernel<NDIM, 1, LR>;
-        case 2: return interp_staged_kernel<NDIM, 2, LR>;
-        case 3: return interp_staged_kernel<NDIM, 3, LR>;
-        case 4: return interp_staged_kernel<NDIM, 4, LR>;
-        case 5: return interp_staged_kernel<NDIM, 5, LR>;
-        case 6: return interp_staged_kernel<NDIM, 6, LR>;
-        case 7: return interp_staged_kernel<NDIM, 7, LR>;
-        case 8: return interp_staged_kernel<NDIM, 8, LR>;
+        case 1: return staged_fn<NDIM, 1, LR>(vec);
+        case 2: return staged_fn<NDIM, 2, LR>(vec);
+        case 3: return staged_fn<NDIM, 3, LR>(vec);
+        case 4: return staged_fn<NDIM, 4, LR>(vec);
+        case 5: return staged_fn<NDIM, 5, LR>(vec);
+        case 6: return staged_fn<NDIM, 6, LR>(vec);
+        case 7: return staged_fn<NDIM, 7, LR>(vec);
+        case 8: return staged_fn<NDIM, 8, LR>(vec);
         default: return nullptr;
     }
 }
@@ -1556,7 +1645,8 @@ int launch_interp(const LaunchTables &t, const float2 *grid, float2 *samp, const
     if (t.n_interp == 0) return TN_OK;
     const int ndim = kind_ndim(t.kind_interp), wc = kind_width(t.kind_interp);
     if (t.interp_mode == kInterpStaged) {
-        StagedFn fn = ndim == 2 ? pick_staged<2, false>(wc) : ndim == 3 ? pick_staged<3, false>(wc) : nullptr;
+        const int vec = staged_vec(t, grid);
+        StagedFn fn = ndim == 2 ? pick_staged<2, false>(wc, vec) : ndim == 3 ? pick_staged<3, false>(wc, vec) : nullptr;
         if (!fn) return fail(TN_E_ARG, "unsupported kernel (ndim=%d, width=%d)", ndim, wc);
         hipLaunchKernelGGL(fn, dim3(xcd_blocks(t.n_interp)), dim3(kBlock), t.interp_lds, stream, t.d_jobs,
                            t.d_interp, t.n_interp, grid, samp, weight, t.interp_coils, LowRank{});
@@ -1695,7 +1785,8 @@ int launch_interp_lowrank(const LaunchTables &t, const float2 *grid, float2 *sam
     if (t.n_interp == 0) return TN_OK;
     const int ndim = kind_ndim(t.kind_interp), wc = kind_width(t.kind_interp);
     if (t.interp_mode == kInterpStaged) {
-        StagedFn fn = ndim == 2 ? pick_staged<2, true>(wc) : ndim == 3 ? pick_staged<3, true>(wc) : nullptr;
+        const int vec = staged_vec(t, grid);
+        StagedFn fn = ndim == 2 ? pick_staged<2, true>(wc, vec) : ndim == 3 ? pick_staged<3, true>(wc, vec) : nullptr;
         if (!fn) return fail(TN_E_ARG, "unsupported kernel (ndim=%d, width=%d)", ndim, wc);
         hipLaunchKernelGGL(fn, dim3(xcd_blocks(t.n_interp)), dim3(kBlock), t.interp_lds, stream, t.d_jobs,
                            t.d_interp, t.n_interp, grid, samp, weight, t.interp_coils, lr);
