@@ -61,6 +61,7 @@ void make_jobs(const tn_plan *plan, int64_t nbatch, int64_t grid_off, int64_t sa
         j.mrow = plan->d_mrow ? plan->d_mrow + (int64_t)f * gvol : nullptr;
         j.mnz = plan->d_mnz;
         j.tent = plan->d_tent;
+        j.rows = plan->d_rows ? plan->d_rows + (int64_t)f * (plan->ntiles_total / plan->ntiles[2]) : nullptr;
         j.taps = plan->d_taps ? plan->d_taps + (int64_t)f * p.npts * tiles_tap_stride(p.ndim, plan->wpad) : nullptr;
         j.mlong = p.grid_split == 0  ? (p.ndim == 3 ? kMatrixLongRow3d : kMatrixLongRow)
                   : p.grid_split < 0 ? matrix_stage(p.ndim)
@@ -535,6 +536,7 @@ void destroy(tn_plan *pl) {
     if (pl->d_mnz) (void)hipFree(pl->d_mnz);
     if (pl->d_taps) (void)hipFree(pl->d_taps);
     if (pl->d_tent) (void)hipFree(pl->d_tent);
+    if (pl->d_rows) (void)hipFree(pl->d_rows);
     if (pl->d_fft) (void)hipFree(pl->d_fft);
     for (int d = 0; d < 3; ++d)
         if (pl->d_apod[d]) (void)hipFree(pl->d_apod[d]);
@@ -608,6 +610,50 @@ int check_device(int device) {
     if (cur != device)
         return fail(TN_E_ARG, "plan lives on device %d but device %d is current", device, cur);
     return TN_OK;
+}
+
+int grid_samples(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, const float *weight, hipStream_t stream,
+                 bool ranged) {
+    clear_error();
+    if (!plan) return fail(TN_E_ARG, "plan is NULL");
+    if (nbatch < 1 || nbatch >= INT32_MAX) return fail(TN_E_ARG, "nbatch must be >= 1");
+    if (!grid || (!samp && plan->p.npts > 0)) return fail(TN_E_ARG, "NULL data pointer");
+    int rc = check_device(plan->device);
+    if (rc) return rc;
+    LaunchTables *t = plan_tables(plan, nbatch, &rc);
+    if (!t) return rc;
+    return launch_grid(*t, (const float2 *)samp, (float2 *)grid, weight, stream, LowRank{}, nullptr, ranged);
+}
+
+// The whole FFT stages; ranged: only the grid cells of the plan's row ranges
+// hold values (the other cells are neither written nor read).
+int transform_forward(tn_plan *plan, const void *image, void *grid, void *work, int64_t nimg, hipStream_t s,
+                      bool ranged) {
+    clear_error();
+    if (!plan) return fail(TN_E_ARG, "plan is NULL");
+    if (!plan->d_fft) return fail(TN_E_ARG, "the plan has no FFT stages");
+    if (nimg < 0) return fail(TN_E_ARG, "nimg must be >= 0");
+    const bool d3 = plan->p.ndim == 3;
+    if (nimg > 0 && (!image || !grid || (d3 && !work))) return fail(TN_E_ARG, "NULL data pointer");
+    int rc = check_device(plan->device);
+    if (rc) return rc;
+    if (!d3) return launch_fft_forward(plan, (const float2 *)image, (float2 *)grid, nimg, s, ranged);
+    rc = launch_fft_z_forward(plan, (const float2 *)image, (float2 *)work, nimg, s);
+    return rc ? rc : launch_fft_forward(plan, (const float2 *)work, (float2 *)grid, nimg * plan->p.grid[0], s, ranged);
+}
+
+int transform_adjoint(tn_plan *plan, void *grid, void *image, void *work, int64_t nimg, hipStream_t s, bool ranged) {
+    clear_error();
+    if (!plan) return fail(TN_E_ARG, "plan is NULL");
+    if (!plan->d_fft) return fail(TN_E_ARG, "the plan has no FFT stages");
+    if (nimg < 0) return fail(TN_E_ARG, "nimg must be >= 0");
+    const bool d3 = plan->p.ndim == 3;
+    if (nimg > 0 && (!image || !grid || (d3 && !work))) return fail(TN_E_ARG, "NULL data pointer");
+    int rc = check_device(plan->device);
+    if (rc) return rc;
+    if (!d3) return launch_fft_adjoint(plan, (float2 *)grid, (float2 *)image, nimg, s, ranged);
+    rc = launch_fft_adjoint(plan, (float2 *)grid, (float2 *)work, nimg * plan->p.grid[0], s, ranged);
+    return rc ? rc : launch_fft_z_adjoint(plan, (const float2 *)work, (float2 *)image, nimg, s);
 }
 
 }  // namespace
@@ -768,6 +814,7 @@ int64_t tn_plan_device_bytes(const tn_plan *plan) {
              sizeof(int2) * std::max<int64_t>(plan->mnnz, 1);
     if (plan->d_taps)                                                                      // tile gridding
         b += sizeof(float) * tiles_tap_stride(p.ndim, plan->wpad) * total + sizeof(int2) * plan->nentries;
+    if (plan->d_rows) b += sizeof(int2) * p.nframes * (plan->ntiles_total / plan->ntiles[2]);
     for (int d = 0; d < 3; ++d)
         if (plan->d_apod[d]) b += sizeof(float) * p.shape[d];
     b += plan->fft_bytes;
@@ -831,15 +878,7 @@ int tn_interp(tn_plan *plan, const void *grid, void *samp, int64_t nbatch, const
 
 int tn_grid(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, const float *weight,
             tn_stream stream) {
-    clear_error();
-    if (!plan) return fail(TN_E_ARG, "plan is NULL");
-    if (nbatch < 1 || nbatch >= INT32_MAX) return fail(TN_E_ARG, "nbatch must be >= 1");
-    if (!grid || (!samp && plan->p.npts > 0)) return fail(TN_E_ARG, "NULL data pointer");
-    int rc = check_device(plan->device);
-    if (rc) return rc;
-    LaunchTables *t = plan_tables(plan, nbatch, &rc);
-    if (!t) return rc;
-    return launch_grid(*t, (const float2 *)samp, (float2 *)grid, weight, (hipStream_t)stream);
+    return grid_samples(plan, samp, grid, nbatch, weight, (hipStream_t)stream, false);
 }
 
 int tn_grid_static(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, const float *weight,
@@ -973,33 +1012,11 @@ int tn_fft_z_adjoint(tn_plan *plan, const void *zin, void *image, int64_t nimg, 
 }
 
 int tn_transform_forward(tn_plan *plan, const void *image, void *grid, void *work, int64_t nimg, tn_stream stream) {
-    clear_error();
-    if (!plan) return fail(TN_E_ARG, "plan is NULL");
-    if (!plan->d_fft) return fail(TN_E_ARG, "the plan has no FFT stages");
-    if (nimg < 0) return fail(TN_E_ARG, "nimg must be >= 0");
-    const bool d3 = plan->p.ndim == 3;
-    if (nimg > 0 && (!image || !grid || (d3 && !work))) return fail(TN_E_ARG, "NULL data pointer");
-    int rc = check_device(plan->device);
-    if (rc) return rc;
-    hipStream_t s = (hipStream_t)stream;
-    if (!d3) return launch_fft_forward(plan, (const float2 *)image, (float2 *)grid, nimg, s);
-    rc = launch_fft_z_forward(plan, (const float2 *)image, (float2 *)work, nimg, s);
-    return rc ? rc : launch_fft_forward(plan, (const float2 *)work, (float2 *)grid, nimg * plan->p.grid[0], s);
+    return transform_forward(plan, image, grid, work, nimg, (hipStream_t)stream, false);
 }
 
 int tn_transform_adjoint(tn_plan *plan, void *grid, void *image, void *work, int64_t nimg, tn_stream stream) {
-    clear_error();
-    if (!plan) return fail(TN_E_ARG, "plan is NULL");
-    if (!plan->d_fft) return fail(TN_E_ARG, "the plan has no FFT stages");
-    if (nimg < 0) return fail(TN_E_ARG, "nimg must be >= 0");
-    const bool d3 = plan->p.ndim == 3;
-    if (nimg > 0 && (!image || !grid || (d3 && !work))) return fail(TN_E_ARG, "NULL data pointer");
-    int rc = check_device(plan->device);
-    if (rc) return rc;
-    hipStream_t s = (hipStream_t)stream;
-    if (!d3) return launch_fft_adjoint(plan, (float2 *)grid, (float2 *)image, nimg, s);
-    rc = launch_fft_adjoint(plan, (float2 *)grid, (float2 *)work, nimg * plan->p.grid[0], s);
-    return rc ? rc : launch_fft_z_adjoint(plan, (const float2 *)work, (float2 *)image, nimg, s);
+    return transform_adjoint(plan, grid, image, work, nimg, (hipStream_t)stream, false);
 }
 
 int tn_convolve(tn_plan *plan, const void *image, const void *kern, int64_t nkern, void *out, void *work0, void *work1,
@@ -1019,15 +1036,17 @@ int tn_convolve(tn_plan *plan, const void *image, const void *kern, int64_t nker
 int tn_nufft_forward(tn_plan *plan, const void *image, void *grid, void *work, void *samp, int64_t nbatch,
                      const float *weight, tn_stream stream) {
     if (!plan) return fail(TN_E_ARG, "plan is NULL");
-    int rc = tn_transform_forward(plan, image, grid, work, nbatch * plan->p.nframes, stream);
+    int rc = transform_forward(plan, image, grid, work, nbatch * plan->p.nframes, (hipStream_t)stream, rows_ranged(plan, nbatch));
     return rc ? rc : tn_interp(plan, grid, samp, nbatch, weight, stream);
 }
 
 int tn_nufft_adjoint(tn_plan *plan, const void *samp, void *grid, void *work, void *image, int64_t nbatch,
                      const float *weight, tn_stream stream) {
     if (!plan) return fail(TN_E_ARG, "plan is NULL");
-    int rc = tn_grid(plan, samp, grid, nbatch, weight, stream);
-    return rc ? rc : tn_transform_adjoint(plan, grid, image, work, nbatch * plan->p.nframes, stream);
+    const bool ranged = rows_ranged(plan, nbatch);
+    int rc = grid_samples(plan, samp, grid, nbatch, weight, (hipStream_t)stream, ranged);
+    return rc ? rc
+              : transform_adjoint(plan, grid, image, work, nbatch * plan->p.nframes, (hipStream_t)stream, ranged);
 }
 
 int tn_batch_create(tn_plan *const *plans, const int64_t *nbatch, const int64_t *grid_offset,

@@ -152,6 +152,7 @@ struct alignas(16) Job {
     int64_t st_off;           // matrix / tile gridding: this job's coil-minor sample copy in the table's buffer
     const int2 *tent;         // tile gridding: (sample, tile-local footprint origin x, y, z + 16 in bytes 0-2),
                               // sorted by tile, samples ascending; bin_off holds the offsets
+    const int2 *rows;         // tile gridding: this frame's row ranges (tn_plan::d_rows)
     const float *taps;        // tile gridding: tap records of this frame's samples
 };
 
@@ -256,6 +257,10 @@ struct tn_plan {
     int64_t fft_bytes = 0;
     int64_t mnnz = 0;
     int2 *d_tent = nullptr;     // tile gridding entries
+    // tile gridding: per frame and (z, y) row of tiles, the signed x range
+    // [lo, hi) of its tiles that footprints reach (x - G for the upper half of
+    // the grid, so that a range around the centre of k-space is one piece)
+    int2 *d_rows = nullptr;
     float *d_taps = nullptr;    // tile gridding: tap records, tiles_tap_stride words per sample
     int wpad = 0;
     std::map<int64_t, tn::LaunchTables> cache;
@@ -285,7 +290,8 @@ int launch_interp(const LaunchTables &t, const float2 *grid, float2 *samp,
                   const float *weight, hipStream_t stream);
 int launch_grid(const LaunchTables &t, const float2 *samp, float2 *grid,
                 const float *weight, hipStream_t stream, LowRank lr = LowRank{},
-                float *scratch = nullptr);
+                float *scratch = nullptr, bool ranged = false);
+// (ranged: cells beyond the row ranges may be left unwritten)
 // Device address of the fixed gridding workspace on `device` (looked up once
 // per device with hipGetSymbolAddress; no allocation).
 int static_scratch(int device, float **out);
@@ -310,16 +316,21 @@ inline bool tiles_fit(const tn_plan_params &p) {
 }
 bool tiles_serve(const tn_plan_params &p);
 int launch_tiles(const LaunchTables &t, const float2 *samp, float2 *grid, const float *weight, hipStream_t stream,
-                 const LowRank &lr, float *scratch);
+                 const LowRank &lr, float *scratch, bool ranged = false);
 int build_matrix(tn_plan *plan, hipStream_t stream);
 // Pruned, fused oversampled-grid FFT stages (2D and 3D plans).
 int build_fft(tn_plan *plan, hipStream_t stream);
-int launch_fft_forward(const tn_plan *plan, const float2 *image, float2 *grid, int64_t nimg, hipStream_t stream);
-int launch_fft_adjoint(const tn_plan *plan, float2 *grid, float2 *image, int64_t nimg, hipStream_t stream);
+int launch_fft_forward(const tn_plan *plan, const float2 *image, float2 *grid, int64_t nimg, hipStream_t stream,
+                       bool ranged = false);
+int launch_fft_adjoint(const tn_plan *plan, float2 *grid, float2 *image, int64_t nimg, hipStream_t stream,
+                       bool ranged = false);
 int launch_fft_z_forward(const tn_plan *plan, const float2 *image, float2 *zout, int64_t nimg, hipStream_t stream);
 int launch_fft_z_adjoint(const tn_plan *plan, const float2 *zin, float2 *image, int64_t nimg, hipStream_t stream);
 int launch_convolve(const tn_plan *plan, const float2 *image, const float2 *kern, int64_t nkern, float2 *out,
                     float2 *work0, float2 *work1, int64_t nimg, hipStream_t stream);
+// Whether the plan's whole transforms leave out the grid cells that no
+// footprint reaches (3D, row ranges, and a kernel of its own length along x).
+bool rows_ranged(const tn_plan *plan, int64_t nbatch);
 // Lengths with factors up to 17 (tn_smooth.hip).
 bool smooth_radices(int L, SmoothRadices &f);
 int smooth_prepare(const FftAxis &a);

@@ -71,4 +71,7 @@ __device__ __forceinline__ int wrap_add(int base, int k, int G) {
     return i >= G ? i - G : i;
 }
 
+// Grid index as a signed frequency, the centre of k-space at zero.
+__host__ __device__ __forceinline__ int signed_x(int x, int G) { return x < (G + 1) / 2 ? x : x - G; }
+
 }  // namespace tn

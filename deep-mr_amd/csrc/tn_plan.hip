@@ -214,6 +214,26 @@ __global__ void tiles_emit_kernel(BinGeom geo, const float *__restrict__ coord, 
     }
 }
 
+// Row ranges (tn_plan::d_rows) from the tile offsets: one lane per row of tiles.
+__global__ void tiles_rows_kernel(BinGeom geo, const int32_t *__restrict__ bin_off, int64_t nrows,
+                                  int2 *__restrict__ rows) {
+    const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (r >= nrows) return;
+    const AxisGeom a = geo.ax[0];
+    const int64_t t0 = r * geo.NT[0];
+    int lo = 0, hi = 0;
+    for (int t = 0; t < geo.NT[0]; ++t) {
+        if (bin_off[t0 + t] == bin_off[t0 + t + 1]) continue;
+        for (int x = t * a.T; x < min((t + 1) * a.T, a.G); ++x) {
+            const int u = signed_x(x, a.G);
+            const bool first = lo == hi;
+            lo = first ? u : min(lo, u);
+            hi = first ? u + 1 : max(hi, u + 1);
+        }
+    }
+    rows[r] = make_int2(lo, hi);
+}
+
 // Tap records of the tile gridding (tiles_tap_stride): the taps
 // the other gridding variants evaluate, padded with zeros.
 template <int WP>
@@ -573,6 +593,13 @@ int build_bins(tn_plan *plan, hipStream_t stream) {
     if (plan->grid_mode == kGridTiles) {
         int rc = build_tiles(plan, geo, nbins, stream);
         if (rc) return rc;
+        if (plan->p.ndim == 3) {
+            const int64_t nrows = nbins / geo.NT[0];
+            TN_HIP(hipMalloc(&plan->d_rows, sizeof(int2) * nrows));
+            hipLaunchKernelGGL(tiles_rows_kernel, dim3((unsigned)((nrows + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream,
+                               geo, plan->d_bin_off, nrows, plan->d_rows);
+            TN_HIP(hipGetLastError());
+        }
     } else if (plan->grid_mode == kGridMatrix) {  // gridding reads the matrix instead
         TN_HIP(hipMemsetAsync(plan->d_bin_off, 0, sizeof(int32_t) * (nbins + 1), stream));
         plan->nentries = 0;

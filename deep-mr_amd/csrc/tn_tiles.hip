@@ -80,6 +80,7 @@ struct TileSrc {
     LowRank lr;
     uint32_t div_mul;  // s / lr.frame_npts = (umulhi(div_mul, s) + s) >> div_shift
     int32_t div_shift;
+    bool ranged;  // empty tiles outside the row ranges need not be written
 };
 
 // Taps d .. d + 3 of an axis, zeros outside [0, WP): a barrel shift of the taps
@@ -141,6 +142,18 @@ __global__ __launch_bounds__(kBlock, NC <= 2 ? 4 : 2) void grid_tiles_kernel(
     const Item it = items[idx];
     if (it.job < 0) return;  // filler
     const Job &J = jobs[it.job];
+    if (src.ranged && it.e0 == it.e1 && it.slot < 0 && (it.unit & kTilesJoin) == 0) {
+        // an empty tile: written (zeros) only where the transform reads it
+        const int2 range = J.rows[it.unit / J.NT[0]];
+        const int x0 = it.unit % J.NT[0] * TX;
+        bool read = false;
+#pragma unroll
+        for (int c = 0; c < TX; ++c) {
+            const int u = signed_x(x0 + c, J.G[0]);
+            read |= x0 + c < J.G[0] && u >= range.x && u < range.y;
+        }
+        if (!read) return;
+    }
     const int lane = threadIdx.x % kWave, k = lane >> 4, i = lane & 15, cx = i & 3, cy = i >> 2;
     const int nc = it.c1 - it.c0;
     float4 *const swt = lds[wave], *const sval = swt + B * 4;
@@ -402,14 +415,14 @@ TilesFn pick_tiles(int ndim, int wpad, int blocks) {
 }  // namespace
 
 int launch_tiles(const LaunchTables &t, const float2 *samp, float2 *grid, const float *weight, hipStream_t stream,
-                 const LowRank &lr, float *scratch) {
+                 const LowRank &lr, float *scratch, bool ranged) {
     const int ndim = kind_ndim(t.kind_grid);
     const int blocks = (t.grid_coils + 7) / 8;
     if ((ndim != 2 && ndim != 3) || kind_width(t.kind_grid) > kTilesMaxWidth || blocks < 1 || blocks > kTilesBlocks)
         return fail(TN_E_ARG, "tile gridding: %dD, width %d, %d coils per item", ndim, kind_width(t.kind_grid),
                     t.grid_coils);
     const bool copy = lr.ncoeff == 0 && t.st_cw > 0;
-    TileSrc src{samp, weight, t.d_st, t.st_cw, lr, 0u, 0};
+    TileSrc src{samp, weight, t.d_st, t.st_cw, lr, 0u, 0, ranged};
     if (lr.ncoeff > 0) {
         // division of a sample index (< 2^31) by frame_npts: l = ceil(log2 d),
         // m = floor(2^32 (2^l - d) / d) + 1
