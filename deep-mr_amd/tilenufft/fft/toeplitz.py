@@ -54,18 +54,17 @@ class GramMatrix:
 
     def stages(self, shape, device):
         """FFT stages between images of ``shape`` and the kernel's grid on
-        ``device`` (None: there are none), built on first use, the last two
-        shapes kept. They hold sizes and twiddles only, nothing of the kernel
-        or of an image."""
-        held = self.__dict__.get("_stages", ())
-        for key, st in held:
-            if key == (shape, device, self.shape):
-                return st
-        if torch.cuda.is_current_stream_capturing():
-            return None
-        st = _core.fft_stages(shape, self.shape, device)
-        self._stages = (((shape, device, self.shape), st), *held[:1])
-        return st
+        ``device`` (None: there are none), built on first use and kept as long
+        as this object: a captured graph holds the addresses of their tables,
+        so none are dropped for another shape's (a few KB each). They hold
+        sizes and twiddles only, nothing of the kernel or of an image."""
+        held = self.__dict__.setdefault("_stages", {})
+        key = (shape, device, self.shape)
+        if key not in held:
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            held.setdefault(key, _core.fft_stages(shape, self.shape, device))
+        return held[key]
 
     def colsum(self):
         """(voxels, ncoeff) column sums of the low-rank kernel (deepmr's product)."""
