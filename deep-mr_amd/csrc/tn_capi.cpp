@@ -755,6 +755,19 @@ int tn_plan_create(const tn_plan_params *params, const float *coord_dev, tn_stre
             hipStreamSynchronize(s) != hipSuccess)
             return cleanup(fail(TN_E_HIP, "apodization upload failed"));
     }
+    if (pl->grid_mode == kGridTiles) {
+        // more entries than 32-bit offsets hold: register runs, whose larger
+        // tiles make fewer (kernels of at most kTilesMaxWidth taps all fit them)
+        int64_t n = 0;
+        rc = tile_entries(pl, s, n);
+        if (rc) return cleanup(rc);
+        if (n >= INT32_MAX) {
+            pl->grid_mode = kGridRuns;
+            pl->wpad = 0;
+            for (int d = 0; d < 3; ++d) pl->p.tile[d] = 0;  // as for the tiles, whatever was asked
+            choose_tiles(pl);
+        }
+    }
     rc = build_bins(pl, s);
     if (rc) return cleanup(rc);
     rc = build_fft(pl, s);

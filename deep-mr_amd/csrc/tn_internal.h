@@ -315,6 +315,8 @@ inline bool tiles_fit(const tn_plan_params &p) {
     return true;
 }
 bool tiles_serve(const tn_plan_params &p);
+// Entries of a tile plan (coordinates uploaded): below 2^31 - 1 an upper bound, else exact.
+int tile_entries(const tn_plan *plan, hipStream_t stream, int64_t &n);
 int launch_tiles(const LaunchTables &t, const float2 *samp, float2 *grid, const float *weight, hipStream_t stream,
                  const LowRank &lr, float *scratch, bool ranged = false);
 int build_matrix(tn_plan *plan, hipStream_t stream);

@@ -180,6 +180,29 @@ __device__ __forceinline__ int tile_pieces(const BinGeom &geo, const float *c, i
     return n;
 }
 
+// Tile entries of all samples, in 64 bits (the offsets are 32-bit): pieces of
+// the tile gridding's footprints, or distinct tiles.
+template <bool PIECES>
+__global__ void entry_total_kernel(BinGeom geo, const float *__restrict__ coord, unsigned long long *__restrict__ sum) {
+    const int64_t total = geo.npts * geo.nframes;
+    unsigned long long n = 0;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        int c = 1;
+        if (PIECES) {
+            int nt[3], tile[3][kMaxPieces], local[3][kMaxPieces];
+            c = tile_pieces(geo, coord + i * geo.ndim, nt, tile, local);
+        } else {
+            for (int d = 0; d < geo.ndim; ++d) {
+                int tl[kMaxWidth];
+                c *= axis_tiles(geo.ax[d], axis_base(geo.ax[d], coord[i * geo.ndim + d]), tl);
+            }
+        }
+        n += (unsigned long long)c;
+    }
+    if (n > 0) atomicAdd(sum, n);
+}
+
 __global__ void tiles_count_kernel(BinGeom geo, const float *__restrict__ coord, int32_t *__restrict__ counts) {
     const int64_t total = geo.npts * geo.nframes;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
@@ -491,8 +514,31 @@ int order_by_origin(const BinGeom &geo, const uint32_t *bin_keys, int64_t n, flo
     return TN_OK;
 }
 
+// Tile entries of all samples. Exact (a pass over the samples) only where their
+// largest possible number passes the 32 bits of the offsets, else that number.
+int entry_total(const BinGeom &geo, const float *coord, bool pieces, hipStream_t stream, int64_t &n) {
+    const uint64_t total = (uint64_t)geo.npts * (uint64_t)geo.nframes;
+    uint64_t most = total;
+    for (int d = 0; d < geo.ndim; ++d) most *= most_pieces(geo.ax[d].W, geo.ax[d].T);
+    n = (int64_t)most;
+    if (most < (uint64_t)INT32_MAX) return TN_OK;
+    DevBuf sum;
+    unsigned long long exact = 0;
+    TN_HIP(hipMalloc(&sum.p, sizeof(exact)));
+    TN_HIP(hipMemsetAsync(sum.p, 0, sizeof(exact), stream));
+    hipLaunchKernelGGL(pieces ? entry_total_kernel<true> : entry_total_kernel<false>,
+                       dim3(std::min(grid_blocks((int64_t)total), 2048u)), dim3(kBlock), 0, stream, geo, coord,
+                       (unsigned long long *)sum.p);
+    TN_HIP(hipGetLastError());
+    TN_HIP(hipMemcpyAsync(&exact, sum.p, sizeof(exact), hipMemcpyDeviceToHost, stream));
+    TN_HIP(hipStreamSynchronize(stream));
+    n = (int64_t)exact;
+    return TN_OK;
+}
+
 // Entries (sorted by (frame, tile), each tile's samples ascending: the sums'
-// fixed order) and tap records of the tile gridding.
+// fixed order) and tap records of the tile gridding, for plans of fewer than
+// 2^31 - 1 entries (tile_entries).
 int build_tiles(tn_plan *plan, const BinGeom &geo, int64_t nbins, hipStream_t stream) {
     const int64_t total = geo.npts * geo.nframes;
     DevBuf counts, offsets, tmp;
@@ -553,7 +599,7 @@ bool tiles_serve(const tn_plan_params &p) {
     for (int d = 3 - p.ndim; d < 3; ++d) {
         const int T = tiles_dim(p.ndim, 2 - d);
         wmax = std::max(wmax, p.width[d]);
-        pieces *= (p.width[d] + T - 2) / T + 2;  // tiles met, one more for a wrap
+        pieces *= most_pieces(p.width[d], T);
     }
     const uint64_t total = (uint64_t)p.nframes * (uint64_t)p.npts;
     uint64_t tiles = p.nframes;
@@ -563,6 +609,10 @@ bool tiles_serve(const tn_plan_params &p) {
     }
     return wmax <= kTilesMaxWidth && total * pieces < (uint64_t)INT32_MAX && tiles < (uint64_t)INT32_MAX / 2 &&
            total * 4 * tiles_tap_stride(p.ndim, tiles_pad(wmax)) + total * pieces * 8 <= 4 * kMatrixAutoBytes;
+}
+
+int tile_entries(const tn_plan *plan, hipStream_t stream, int64_t &n) {
+    return entry_total(make_geom(plan), plan->d_coord, true, stream, n);
 }
 
 int build_bins(tn_plan *plan, hipStream_t stream) {
@@ -606,6 +656,10 @@ int build_bins(tn_plan *plan, hipStream_t stream) {
         int rc = build_matrix(plan, stream);
         if (rc) return rc;
     } else {
+        int64_t n = 0;
+        int rc = entry_total(geo, plan->d_coord, false, stream, n);
+        if (rc) return rc;
+        if (n >= INT32_MAX) return fail(TN_E_RANGE, "too many tile entries (%lld)", (long long)n);
         DevBuf counts, offsets, scan_tmp;
         TN_HIP(hipMalloc(&counts.p, sizeof(int32_t) * total));
         TN_HIP(hipMalloc(&offsets.p, sizeof(int32_t) * (total + 1)));
@@ -624,8 +678,7 @@ int build_bins(tn_plan *plan, hipStream_t stream) {
         TN_HIP(hipMemcpyAsync(&last_cnt, (int32_t *)counts.p + (total - 1), sizeof(int32_t),
                               hipMemcpyDeviceToHost, stream));
         TN_HIP(hipStreamSynchronize(stream));
-        const int64_t n = (int64_t)last_off + last_cnt;
-        if (n >= INT32_MAX) return fail(TN_E_RANGE, "too many tile entries (%lld)", (long long)n);
+        n = (int64_t)last_off + last_cnt;
         plan->nentries = n;
         DevBuf keys, vals;
         TN_HIP(hipMalloc(&keys.p, sizeof(uint32_t) * n));
@@ -634,8 +687,8 @@ int build_bins(tn_plan *plan, hipStream_t stream) {
                            plan->d_coord, (const int32_t *)offsets.p, (uint32_t *)keys.p,
                            (int32_t *)vals.p);
         TN_HIP(hipGetLastError());
-        int rc = sort_entries(geo, plan->d_coord, keys.p, vals.p, n, plan->d_bin_off,
-                              &plan->d_entries, stream, plan->grid_mode == kGridRuns ? kOrderOrigin : kOrderSpread);
+        rc = sort_entries(geo, plan->d_coord, keys.p, vals.p, n, plan->d_bin_off, &plan->d_entries, stream,
+                          plan->grid_mode == kGridRuns ? kOrderOrigin : kOrderSpread);
         if (rc) return rc;
         plan->h_bin_off.assign(nbins + 1, 0);
         TN_HIP(hipMemcpyAsync(plan->h_bin_off.data(), plan->d_bin_off, sizeof(int32_t) * (nbins + 1),

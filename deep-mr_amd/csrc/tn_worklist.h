@@ -40,6 +40,10 @@ TN_HOST_DEVICE inline int axis_pieces(int base, int W, int G, int T, int (&tile)
     return n;
 }
 
+// Most pieces of a footprint of W taps along an axis of tiles of T cells: the
+// tiles it can meet, one more for a wrap.
+constexpr int most_pieces(int W, int T) { return (W + T - 2) / T + 2; }
+
 constexpr int kMatrixCoils = 16;   // widest record of the matrix gridding (coils per item)
 constexpr int kMatrixStage = 1024; // entries of a run of cells staged in LDS (also the longest short row), 3D
 constexpr int kMatrixStage2d = 512; // the same in 2D: a smaller stage leaves LDS for more workgroups per CU

@@ -91,7 +91,8 @@ typedef struct tn_plan_params {
                              plan table (4 bytes per padded tap and axis);
                              a tile of many samples takes a workgroup's
                              four waves; grid_chunk <= 32 (0: equal
-                             chunks of at most 32); tile ignored        */
+                             chunks of at most 32); tile ignored; plans of
+                             2^31 - 1 tile entries or more take 2       */
     float inv_scale;    /* 1 / kernel scaling (src/deepmr/fft/_interp/plan.py:190) */
     const float *apod[3]; /* host apodization vectors of length shape[d], or
                              NULL for ones (src/deepmr/fft/nufft.py:423-447)   */
