@@ -56,6 +56,24 @@ def on_device(device):
     return _NO_SWITCH if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
+_TRACER_MODES = tuple(torch._C._TorchDispatchModeKey.__members__.values())  # fake tensors, proxies, functional
+
+
+def traced(*tensors):
+    """Whether tensors without memory of their own stand for the values of
+    this call: under compilation and in the modes of fake, proxy and functional
+    tensors, for the wrappers of functorch transforms, and for subclasses with
+    a dispatch of their own. Native code, which takes addresses, cannot serve
+    such a call (modes that only watch, as counters do, are none)."""
+    if torch.compiler.is_compiling():
+        return True
+    if torch._C._len_torch_dispatch_stack() > 0 and any(
+            torch._C._get_dispatch_mode(mode) is not None for mode in _TRACER_MODES):
+        return True
+    return any(torch._C._functorch.is_functorch_wrapped_tensor(t) or torch._is_functional_tensor(t)
+               or type(t).__torch_dispatch__ is not torch.Tensor.__torch_dispatch__ for t in tensors)
+
+
 def ptr(t):
     """Raw device pointer of ``t`` for the C ABI. Lazy conjugate / negative
     views are refused: their memory does not hold the values they denote."""

@@ -150,10 +150,11 @@ def _kspace_product(k, kern, ndim):
 def _convolve(x, kern, dev):
     """The native stages' result, or None where they do not serve: low-rank,
     real or elsewhere-held kernels, kernels whose leading axes are not the last
-    of the image's, empty batches, tracers (which record torch's own calls)."""
-    if torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
-        return None
+    of the image's, empty batches, tensors without memory of their own (tracers
+    and functorch transforms, which take torch's calls)."""
     ndim, value = kern.ndim, kern.value
+    if _core.traced(x, value):
+        return None
     lead, klead = tuple(x.shape[:-ndim]), tuple(value.shape[:-ndim])
     if (kern.islowrank or value.dtype != torch.complex64 or value.device != dev or x.numel() == 0
             or tuple(value.shape[-ndim:]) != tuple(kern.shape) or lead[len(lead) - len(klead):] != klead):
