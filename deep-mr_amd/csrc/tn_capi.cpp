@@ -368,14 +368,21 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
                               : pl->p.grid_split < 0 ? INT32_MAX
                                                      : pl->p.grid_split;
         const int64_t cells = (int64_t)j.T[0] * j.T[1] * j.T[2];  // partial size per coil
-        std::vector<int32_t> order;
-        if (tiles) order = brick_order(j.NT, j.ndim);
+        std::vector<int32_t> order, empty;
+        if (tiles) {
+            order = brick_order(j.NT, j.ndim);
+            empty = empty_runs(goff, j.NT, kTilesFillCells / j.T[0]);
+        }
         for (int64_t ti = 0; ti < ntiles; ++ti) {
             const int64_t tl = tiles ? order[ti] : ti;
             const int32_t b0 = goff[tl], b1 = goff[tl + 1];
             const int nparts = (int)std::max<int64_t>(1, ((int64_t)(b1 - b0) + split - 1) / split);
             for (int c0 = 0; c0 < j.nbatch; c0 += gc) {
                 const int c1 = std::min(j.nbatch, c0 + gc);
+                if (tiles && b0 == b1) {  // zeroed by the item of its run
+                    if (empty[tl] > 0) grid.push_back(Item{(int)ji, (int)tl, c0, c1, 0, empty[tl], 0, kTilesFill});
+                    continue;
+                }
                 if (nparts == 1 && (!tiles || b1 - b0 <= wave_max)) {
                     grid.push_back(Item{(int)ji, (int)tl, c0, c1, b0, b1, 0, -1});
                     continue;

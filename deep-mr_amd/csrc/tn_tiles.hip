@@ -80,7 +80,7 @@ struct TileSrc {
     LowRank lr;
     uint32_t div_mul;  // s / lr.frame_npts = (umulhi(div_mul, s) + s) >> div_shift
     int32_t div_shift;
-    bool ranged;  // empty tiles outside the row ranges need not be written
+    bool ranged;  // cells outside the row ranges need not be written
 };
 
 // Taps d .. d + 3 of an axis, zeros outside [0, WP): a barrel shift of the taps
@@ -99,6 +99,43 @@ __device__ __forceinline__ float4 tap_window(const float (&t)[WP], int d) {
             if (j < 3 + sh) a[j] = on ? (j + sh < WP + 8 ? a[j + sh] : 0.0f) : a[j];
     }
     return make_float4(a[0], a[1], a[2], a[3]);
+}
+
+// Zeros for a run of it.e1 tiles without entries, in rows of up to
+// kTilesFillCells cells, two per lane and two rows per store (ranged: where
+// the transform reads). A tile by itself is stored in 32-byte pieces, which
+// the memory takes at 1.7 TB/s once the grids pass the caches: 500 spokes x
+// 256 samples, 8 coils of 256^3, 73% of the tiles empty: 650 us, 447 in runs
+// (the gridding matrix 488); their first adjoint, which builds the work list,
+// 8.0 -> 4.7 ms.
+template <int NDIM>
+__device__ __forceinline__ void fill_tiles(const Job &J, const Item &it, bool ranged, float2 *__restrict__ grid,
+                                           int lane) {
+    constexpr int TX = tiles_dim(NDIM, 0), TY = tiles_dim(NDIM, 1), TZ = tiles_dim(NDIM, 2);
+    constexpr int PAIRS = kTilesFillCells / 2;
+    const int Gx = J.G[0], Gy = J.G[1], Gz = J.G[2], row = it.unit / J.NT[0];
+    const int x0 = it.unit % J.NT[0] * TX, y0 = row % J.NT[1] * TY, z0 = row / J.NT[1] * TZ;
+    const int x = x0 + 2 * (lane % PAIRS), end = min(x0 + it.e1 * TX, Gx);
+    bool read = x < end;
+    if (ranged) {
+        const int2 range = J.rows[row];
+        const int a = signed_x(x, Gx), b = signed_x(x + 1, Gx);
+        read = read && ((a >= range.x && a < range.y) || (x + 1 < end && b >= range.x && b < range.y));
+        if (!__any(read)) return;
+    }
+    const Pair2 zeros = {{0.0f, 0.0f, 0.0f, 0.0f}};
+    const int rows = (it.c1 - it.c0) * TY * TZ;
+    float2 *const g = grid + J.grid_off + it.c0 * J.grid_bstride + x;
+#pragma unroll 4
+    for (int r = lane / PAIRS; r < rows; r += kWave / PAIRS) {
+        const int y = y0 + r % TY, z = z0 + r / TY % TZ;
+        if (!read || y >= Gy || z >= Gz) continue;
+        float2 *p = g + r / (TY * TZ) * J.grid_bstride + ((int64_t)z * Gy + y) * Gx;
+        if (x + 1 < end)
+            *(Pair2 *)p = zeros;
+        else
+            *p = make_float2(0.0f, 0.0f);
+    }
 }
 
 // Tile gridding. The entries are taken sixteen at a time. Loading: four lanes
@@ -142,17 +179,9 @@ __global__ __launch_bounds__(kBlock, NC <= 2 ? 4 : 2) void grid_tiles_kernel(
     const Item it = items[idx];
     if (it.job < 0) return;  // filler
     const Job &J = jobs[it.job];
-    if (src.ranged && it.e0 == it.e1 && it.slot < 0 && (it.unit & kTilesJoin) == 0) {
-        // an empty tile: written (zeros) only where the transform reads it
-        const int2 range = J.rows[it.unit / J.NT[0]];
-        const int x0 = it.unit % J.NT[0] * TX;
-        bool read = false;
-#pragma unroll
-        for (int c = 0; c < TX; ++c) {
-            const int u = signed_x(x0 + c, J.G[0]);
-            read |= x0 + c < J.G[0] && u >= range.x && u < range.y;
-        }
-        if (!read) return;
+    if (it.slot == kTilesFill) {
+        fill_tiles<NDIM>(J, it, src.ranged, grid, threadIdx.x % kWave);
+        return;
     }
     const int lane = threadIdx.x % kWave, k = lane >> 4, i = lane & 15, cx = i & 3, cy = i >> 2;
     const int nc = it.c1 - it.c0;

@@ -90,6 +90,32 @@ constexpr int kDealXcds = 8;    // XCDs the hardware deals workgroups to in turn
 constexpr int kTilesBase = 24;  // a tile's own cost in entries, for the balance over the XCDs
 constexpr int32_t kTilesJoin = 1 << 30;  // flag of an item's unit: the workgroup's four items share the tile
 
+constexpr int32_t kTilesFill = -2;       // slot of an item that zeroes a run of e1 tiles without entries
+constexpr int kTilesFillCells = 64;      // most cells of such a run: 512-byte rows
+
+// Runs of tiles without entries along the rows of a frame: at a run's first
+// tile its length (at most `longest`), 0 at every other tile.
+inline std::vector<int32_t> empty_runs(const int32_t *off, const int32_t (&nt)[3], int longest) {
+    std::vector<int32_t> run((size_t)nt[0] * nt[1] * nt[2], 0);
+    for (size_t row = 0; row < run.size(); row += nt[0])
+        for (int x = 0, first = -1; x < nt[0]; ++x) {
+            const size_t t = row + x;
+            if (off[t] != off[t + 1]) {
+                first = -1;
+                continue;
+            }
+            if (first < 0 || run[row + first] == longest) first = x;
+            ++run[row + first];
+        }
+    return run;
+}
+
+// Cost of an item in entries, for the balance: a tile's own cost is mostly its
+// stores, which a run of empty tiles makes in longer rows.
+inline int64_t tiles_cost(const Item &it) {
+    return it.slot == kTilesFill ? (int64_t)kTilesBase / 2 * it.e1 : kTilesBase + (it.e1 - it.e0);
+}
+
 // Tiles of a frame in bricks (x fastest inside and over the bricks), so that
 // neighbours along every axis are near each other in the work list.
 inline std::vector<int32_t> brick_order(const int32_t (&nt)[3], int ndim) {
@@ -125,14 +151,14 @@ inline void tiles_deal(std::vector<Item> &joined, std::vector<Item> &grid) {
     while (grid.size() % (per * kXcds)) grid.push_back(none);
     const int64_t wg = ((int64_t)rest.size() + per - 1) / per;
     double total = 0;
-    for (const Item &it : rest) total += kTilesBase + (it.e1 - it.e0);
+    for (const Item &it : rest) total += tiles_cost(it);
     int64_t first[kXcds + 1] = {0}, longest = 0;  // workgroup ranges
     double sum = 0;
     int x = 0;
     for (int64_t w = 0; w < wg; ++w) {
         while (x + 1 < kXcds && sum >= total * (x + 1) / kXcds) first[++x] = w;
         for (int64_t q = w * per; q < std::min<int64_t>((w + 1) * per, (int64_t)rest.size()); ++q)
-            sum += kTilesBase + (rest[q].e1 - rest[q].e0);
+            sum += tiles_cost(rest[q]);
     }
     while (x < kXcds) first[++x] = wg;
     for (x = 0; x < kXcds; ++x) longest = std::max(longest, first[x + 1] - first[x]);
