@@ -49,6 +49,24 @@ constexpr int staged_cells(int ndim, int wc) {
                       (ndim == 3 ? staged_tile(ndim, 2) + wc - 1 : 1);
     return (pairs + kBlock - 1) / kBlock * kBlock * 2;
 }
+// Where those loads are used. They hold more registers than the row-by-row
+// load (2D, 4 taps: 84 for 66, five waves per SIMD for seven; single cells 100;
+// 3D, 4 taps: 167 for 110), which costs nothing while a launch's workgroups are
+// all resident, up to kStagedFew of them (four per CU), and has to be made up
+// by fewer instructions per plane beyond. Fewest planes of an item for which
+// it is, measured against row by row: pairs of cells in 2D with one to three
+// taps from the first plane on (0.95 to 1.02 of the time), four and six taps
+// from three (one plane 1.06, three 0.97; eight 0.81), five, where the waves
+// drop from six to four, from six (three 1.05, six 0.98, eight 0.88); single
+// cells only with six taps from three (three 0.98; four taps 1.19 with one
+// plane and 1.07 with eight); 3D from three (one 1.18, two 1.04 to 1.10, three
+// 0.93 to 1.02, eight 0.84). 0: at no number.
+constexpr int64_t kStagedFew = 1024;
+constexpr int staged_planes(int ndim, int wc, int vec) {
+    if (ndim == 3) return 3;
+    if (vec == 1) return wc == 6 ? 3 : 0;
+    return wc <= 3 ? 1 : wc == 5 ? 6 : 3;
+}
 constexpr int interp_segment(int ndim) { return 256 * staged_ept(ndim); }  // samples per staged work item
 constexpr int kGridSplitDefault = 2048;  // max tile entries per gridding workgroup
 constexpr int kGridBatch = 256;  // tile entries staged in LDS per gridding batch
@@ -194,7 +212,8 @@ struct LaunchTables {
     int64_t st_elems = 0;
     int st_cw = 0;  // 0: the lane-per-cell matrix kernel reads the samples in place
     int wpad = 0;   // tile gridding: words per axis of the tap records
-    int interp_vec = 0;  // staged interpolation: cells per load (2, 1), 0: row by row
+    int interp_vec = 0;  // staged interpolation: cells per load the regions allow (2, 1), 0: row by row only
+    int interp_planes = 0;  // fewest planes of a job
     int st_cpl = 1; // coils per lane of the matrix kernel over the copy (1 or 2)
     int64_t device_bytes = 0;  // bytes of the device allocations above
 };

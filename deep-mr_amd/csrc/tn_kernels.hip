@@ -323,7 +323,8 @@ __device__ __forceinline__ void staged_taps2(const float2 *r0, const float2 *r1,
 // flight during the tap sums. Row by row -> this: 8 x 16 spirals on 512^2 120
 // -> 111 us, 20 frames of 240^2, 6 taps 53 -> 44 us, 5.1 M samples of 8 coils
 // of 256^3 898 -> 810 us (836 without the loads ahead; 906 held to 128
-// registers). VEC = 0, row by row: larger regions than the default tiles' or
+// registers). VEC = 0, row by row: large launches of few planes, whose waves per
+// SIMD count for more (staged_planes), larger regions than the default tiles' or
 // larger chunks (where asked for), wider kernels, and in 3D grids of odd rows
 // (8-byte loads take twice the registers: 61x101x84 65 -> 70 us).
 template <int NDIM, int WC, bool LR, int VEC>
@@ -1579,10 +1580,13 @@ StagedFn staged_fn(int vec) {
     return vec == 0 ? interp_staged_kernel<NDIM, WC, LR, 0> : nullptr;
 }
 
-// Cells per load for a grid at this address.
+// Cells per load for a grid at this address, 0: row by row.
 int staged_vec(const LaunchTables &t, const float2 *grid) {
-    if (t.interp_vec < 2 || (uintptr_t)grid % sizeof(f32x4) == 0) return t.interp_vec;
-    return kind_ndim(t.kind_interp) == 2 ? 1 : 0;
+    const int ndim = kind_ndim(t.kind_interp);
+    int vec = t.interp_vec;
+    if (vec == 2 && (uintptr_t)grid % sizeof(f32x4) != 0) vec = ndim == 2 ? 1 : 0;
+    const int planes = staged_planes(ndim, kind_width(t.kind_interp), vec);
+    return t.n_interp <= kStagedFew || (planes > 0 && t.interp_planes >= planes) ? vec : 0;
 }
 
 template <int NDIM, bool LR>
