@@ -600,16 +600,12 @@ int check_lowrank(const tn_plan *plan, int64_t nbatch, int32_t ncoeff, int32_t f
     return TN_OK;
 }
 
-// Whether two plans of different gridding variants may share a batch: both
-// chosen automatically among the tile and the matrix gridding, or one of
-// those chosen and the matrix asked for (automatic plans and explicit matrix
-// plans batch together).
+// Whether two plans may share a batch: plans of one gridding variant, plans
+// whose variants were both chosen automatically, and automatic plans with plans
+// for which the variant was asked for that they would have without the tiles.
 bool batch_modes_mix(const tn_plan *a, const tn_plan *b) {
-    auto ok = [](const tn_plan *p) {
-        return (p->p.grid_mode == kGridAuto && (p->grid_mode == kGridTiles || p->grid_mode == kGridMatrix)) ||
-               p->p.grid_mode == kGridMatrix;
-    };
-    return ok(a) && ok(b);
+    return a->grid_mode == b->grid_mode || a->mix_mode == b->mix_mode ||
+           (a->p.grid_mode == kGridAuto && b->p.grid_mode == kGridAuto);
 }
 
 // Checks that the current device is the plan's device.
@@ -713,15 +709,12 @@ int tn_plan_create(const tn_plan_params *params, const float *coord_dev, tn_stre
                         "grid_mode 4 (register tiles) needs a 3D plan with at most 4 taps per axis and grid "
                         "lengths that are multiples of 8 x 8 x 4 with at least two such blocks per axis");
         }
-        pl->grid_mode = params->grid_mode == kGridSpread   ? kGridSpread
-                        : params->grid_mode == kGridMatrix ? kGridMatrix
-                        : params->grid_mode == kGridRuns   ? kGridRuns
-                        : params->grid_mode == kGridTiles  ? kGridTiles
-                        : tiles_serve(*params)             ? kGridTiles
-                        : matrix_ok                        ? kGridMatrix
-                        : tiles_ok                         ? kGridTiles
-                        : runs_ok                          ? kGridRuns
-                                                           : kGridSpread;
+        pl->mix_mode = params->grid_mode != kGridAuto ? params->grid_mode
+                       : matrix_ok                    ? kGridMatrix
+                       : tiles_ok                     ? kGridTiles
+                       : runs_ok                      ? kGridRuns
+                                                      : kGridSpread;
+        pl->grid_mode = params->grid_mode == kGridAuto && tiles_serve(*params) ? kGridTiles : pl->mix_mode;
         if (pl->grid_mode == kGridTiles) {  // the tile the kernel is built for, whatever was asked
             pl->ntiles_total = 1;
             int wmax = 1;
@@ -1097,7 +1090,7 @@ int tn_batch_create(tn_plan *const *plans, const int64_t *nbatch, const int64_t 
         if (pl->p.ndim != ndim) return fail(TN_E_ARG, "plans mix 2D and 3D");
         if (nbatch[k] < 1 || nbatch[k] >= INT32_MAX) return fail(TN_E_ARG, "nbatch[%d] < 1", k);
         if (grid_offset[k] < 0 || samp_offset[k] < 0) return fail(TN_E_ARG, "negative offset");
-        if (pl->grid_mode != plans[0]->grid_mode && !batch_modes_mix(pl, plans[0]))
+        if (!batch_modes_mix(pl, plans[0]))
             return fail(TN_E_ARG, "batched plans must share the gridding variant");
         auto part = std::find_if(parts.begin(), parts.end(), [&](const Part &q) { return q.mode == pl->grid_mode && q.wpad == pl->wpad; });
         if (part == parts.end()) part = parts.insert(parts.end(), Part{pl->grid_mode, pl->wpad, {}, {}});

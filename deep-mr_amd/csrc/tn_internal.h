@@ -267,6 +267,7 @@ struct tn_plan {
     int64_t nentries = 0;
     int64_t footprint = -1;
     int grid_mode = tn::kGridSpread;  // effective gridding variant (entry order)
+    int mix_mode = tn::kGridSpread;   // the variant asked for, or the automatic one without the tiles (batch_modes_mix)
     int32_t *d_mrow = nullptr;  // matrix gridding: row offsets, (nframes * cells + 1)
     int2 *d_mnz = nullptr;      // matrix gridding: (sample, weight bits) sorted by (frame, cell)
     tn::FftAxis axis[3];        // line transforms of the FFT stages, (x, y, z)
