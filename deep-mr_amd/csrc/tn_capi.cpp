@@ -170,17 +170,33 @@ static int tiles_chunk(int64_t nbatch) {
     return (int)(8 * ((blocks + std::max<int64_t>(chunks, 1) - 1) / std::max<int64_t>(chunks, 1)));
 }
 
-// Entries per workgroup of a split tile, for plans without a split of their
-// own: four waves' worth, doubled until the table's partial tiles fit the
-// fixed gridding workspace, so that allocation-free launches take every table.
-static int tiles_doubling(const std::vector<Job> &jobs, const std::vector<const tn_plan *> &plan_of) {
-    for (int times = 1;; times *= 2) {
+// Entries per workgroup of a split tile before the doubling below (0: tiles
+// are not split): the plan's split, or four waves' worth.
+static int64_t tiles_part(const tn_plan *pl) {
+    return pl->p.grid_split < 0   ? 0
+           : pl->p.grid_split > 0 ? pl->p.grid_split
+                                  : (int64_t)kTilesWave * (kBlock / kWave);
+}
+
+// Whether the table's doubling applies to a plan: unless it asked for the tile
+// gridding with a split of its own. (For automatic plans grid_split says how
+// fine to split, whichever variant they get: a partial sum of the matrix is one
+// cell's, of a tile 64 cells', many times the memory for a fine split.)
+static bool tiles_doubled(const tn_plan *pl) {
+    return pl->p.grid_split == 0 || pl->p.grid_mode != kGridTiles;
+}
+
+// Factor on the entries per workgroup of a split tile: doubled until the
+// table's partial tiles fit the fixed gridding workspace, so that
+// allocation-free launches take every table.
+static int64_t tiles_doubling(const std::vector<Job> &jobs, const std::vector<const tn_plan *> &plan_of) {
+    for (int64_t times = 1;; times *= 2) {
         int64_t floats = 0;
         for (size_t ji = 0; ji < jobs.size(); ++ji) {
             const Job &j = jobs[ji];
             const tn_plan *pl = plan_of[ji];
-            if (pl->p.grid_split != 0) continue;
-            const int64_t part = (int64_t)kTilesWave * (kBlock / kWave) * times;
+            const int64_t part = tiles_part(pl) * times;
+            if (part == 0 || !tiles_doubled(pl)) continue;
             const int32_t *off = pl->h_bin_off.data() + (j.bin_off - pl->d_bin_off);
             int64_t parts = 0;
             for (int64_t tl = 0; tl < pl->ntiles_total; ++tl) {
@@ -189,7 +205,7 @@ static int tiles_doubling(const std::vector<Job> &jobs, const std::vector<const 
             }
             floats += parts * 2 * j.nbatch * j.T[0] * j.T[1] * j.T[2];
         }
-        if (floats <= kStaticScratchFloats || times >= 1 << 20) return times;
+        if (floats <= kStaticScratchFloats || times > INT32_MAX) return times;
     }
 }
 
@@ -272,7 +288,7 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
     std::vector<Item> interp, grid, fold, tr, joined;
     std::vector<int64_t> slot_base;
     int64_t scratch = 0;
-    const int tiles_times = gmode == kGridTiles ? tiles_doubling(jobs, plan_of) : 0;
+    const int64_t tiles_times = gmode == kGridTiles ? tiles_doubling(jobs, plan_of) : 0;
     const bool tcopy = gmode == kGridTiles && lr_coeffs == 0 && !force_gather && tiles_copy(jobs);
     for (size_t ji = 0; ji < jobs.size(); ++ji) {
         const Job &j = jobs[ji];
@@ -364,9 +380,10 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
                                           : pl->p.grid_split < 0 ? INT32_MAX
                                                                  : (pl->p.grid_split + waves - 1) / waves)
                                        : 0;
-        const int64_t split = pl->p.grid_split == 0  ? (tiles ? wave_max * waves * tiles_times : kGridSplitDefault)
-                              : pl->p.grid_split < 0 ? INT32_MAX
-                                                     : pl->p.grid_split;
+        const int64_t split = pl->p.grid_split < 0 ? INT32_MAX
+                              : tiles              ? tiles_part(pl) * (tiles_doubled(pl) ? tiles_times : 1)
+                              : pl->p.grid_split   ? pl->p.grid_split
+                                                   : kGridSplitDefault;
         const int64_t cells = (int64_t)j.T[0] * j.T[1] * j.T[2];  // partial size per coil
         std::vector<int32_t> order, empty;
         if (tiles) {
