@@ -173,9 +173,6 @@ Fns fns_for() {
     return f;
 }
 
-// Convolution lengths: at most a third apart, so that padding costs little.
-constexpr int kLengths[] = {32, 48, 64, 96, 128, 160, 192, 240, 256, 320, 384, 480, 512, 640, 768, 1024, 1280, 1536};
-
 Fns fns(int M) {
     switch (M) {
         case 32: return fns_for<32>();
@@ -230,13 +227,6 @@ void host_dft(const Cd *in, int stride, Cd *out, int n, const std::vector<Cd> &r
 }
 
 }  // namespace
-
-int chirp_length(int N, int L) {
-    if (L < 2) return 0;  // unit axes (1D data as one row) keep the separate kernels
-    for (int M : kLengths)
-        if (M >= N + L - 1) return M;
-    return 0;
-}
 
 // tw[M], then per direction (forward, inverse) in, out and b. Signed pixel
 // n = m - N / 2; c(n) = exp(-i pi n^2 / L).

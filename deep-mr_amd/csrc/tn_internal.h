@@ -360,10 +360,9 @@ int smooth_rows(const FftAxis &a, bool inverse, float2 *data, int64_t nlines, hi
 int smooth_product(const FftAxis &a, float2 *data, int64_t nlines, const float2 *kern, int64_t nk, hipStream_t stream);
 int smooth_cols(const FftAxis &a, bool inverse, const float2 *src, float2 *dst, int64_t nimg, int cols, int pitch,
                 int hx, const float *apx, const float *apy, float scale, hipStream_t stream);
-// Chirp transforms (tn_chirp.hip): the convolution length of an axis (0:
-// none), its tables in float2 (appended to `host`; chirp_bind sets the
-// pointers for a table that starts at `base`), and the stages.
-int chirp_length(int N, int L);
+// Chirp transforms (tn_chirp.hip) of axes with a chirp_length: their tables in
+// float2 (appended to `host`; chirp_bind sets the pointers for a table that
+// starts at `base`), and the stages.
 void chirp_tables(const FftAxis &a, std::vector<float2> &host);
 void chirp_bind(FftAxis &a, const float2 *base);
 int chirp_prepare(const FftAxis &a);

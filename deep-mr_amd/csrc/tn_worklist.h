@@ -40,6 +40,18 @@ TN_HOST_DEVICE inline int axis_pieces(int base, int W, int G, int T, int (&tile)
     return n;
 }
 
+// Convolution length of an axis of N pixels and L grid points done as a chirp
+// transform, 0: none. Lengths at most a half apart, from 96 on a third, so that
+// padding costs little; unit axes (1D data as one row) keep the separate kernels.
+constexpr int kChirpLengths[] = {32,  48,  64,  96,  128, 160, 192, 240,  256,
+                                 320, 384, 480, 512, 640, 768, 1024, 1280, 1536};
+inline int chirp_length(int N, int L) {
+    if (L < 2) return 0;
+    for (int M : kChirpLengths)
+        if (M >= (int64_t)N + L - 1) return M;
+    return 0;
+}
+
 // Most pieces of a footprint of W taps along an axis of tiles of T cells: the
 // tiles it can meet, one more for a wrap.
 constexpr int most_pieces(int W, int T) { return (W + T - 2) / T + 2; }
