@@ -101,6 +101,15 @@ __device__ __forceinline__ float4 tap_window(const float (&t)[WP], int d) {
     return make_float4(a[0], a[1], a[2], a[3]);
 }
 
+// Orders this wave's LDS traffic for the compiler: lanes read words that other
+// lanes of the wave stored, and store words that others have read, which the
+// hardware keeps in program order but a lane's own addresses do not show. No
+// instruction.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Zeros for a run of it.e1 tiles without entries, in rows of up to
 // kTilesFillCells cells, two per lane and two rows per store (ranged: where
 // the transform reads). A tile by itself is stored in 32-byte pieces, which
@@ -284,6 +293,7 @@ __global__ __launch_bounds__(kBlock, NC <= 2 ? 4 : 2) void grid_tiles_kernel(
                          __builtin_isfinite(v[n].w));
                 sval[n * B * 4 + 4 * j + r] = v[n];
             }
+            wave_lds_order();  // the step's words stored
             en = next;
             if (e + B < it.e1) {  // the next sixteen
                 axis_taps_of(en.x, t);
@@ -311,6 +321,7 @@ __global__ __launch_bounds__(kBlock, NC <= 2 ? 4 : 2) void grid_tiles_kernel(
                     wy[u][1] = ws[12 + cy];
                 }
             }
+            wave_lds_order();  // and read
 #pragma unroll
             for (int p = 0; p < 4; ++p)
 #pragma unroll
@@ -376,7 +387,10 @@ __global__ __launch_bounds__(kBlock, NC <= 2 ? 4 : 2) void grid_tiles_kernel(
     const int64_t poff = ((int64_t)pz * Gy + py) * Gx + px;
 #pragma unroll
     for (int n = 0; n < NC; ++n) {
-        if (joined && n > 0) __syncthreads();  // the previous block's sums read
+        if (joined && n > 0)
+            __syncthreads();  // the previous block's sums read
+        else
+            wave_lds_order();
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
             const int x = NDIM == 3 ? cx : cx + 4 * (p & 1), y = NDIM == 3 ? cy : cy + 4 * (p >> 1);
@@ -384,7 +398,10 @@ __global__ __launch_bounds__(kBlock, NC <= 2 ? 4 : 2) void grid_tiles_kernel(
             out[2 * k * CP + cell] = make_float2(acc[p][n][0], acc[p][n][1]);
             out[(2 * k + 1) * CP + cell] = make_float2(acc[p][n][2], acc[p][n][3]);
         }
-        if (joined) __syncthreads();
+        if (joined)
+            __syncthreads();
+        else
+            wave_lds_order();
 #pragma unroll
         for (int q = 0; q < 8 / CPI; ++q) {
             const int c = q * CPI + lane / PAIRS;
