@@ -70,8 +70,13 @@ def traced(*tensors):
     if torch._C._len_torch_dispatch_stack() > 0 and any(
             torch._C._get_dispatch_mode(mode) is not None for mode in _TRACER_MODES):
         return True
-    return any(torch._C._functorch.is_functorch_wrapped_tensor(t) or torch._is_functional_tensor(t)
-               or type(t).__torch_dispatch__ is not torch.Tensor.__torch_dispatch__ for t in tensors)
+    transforms = torch._C._are_functorch_transforms_active()
+    for t in tensors:
+        if type(t) is not torch.Tensor and type(t).__torch_dispatch__ is not torch.Tensor.__torch_dispatch__:
+            return True
+        if torch._is_functional_tensor(t) or transforms and torch._C._functorch.is_functorch_wrapped_tensor(t):
+            return True
+    return False
 
 
 def ptr(t):
