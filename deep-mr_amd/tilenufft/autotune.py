@@ -3,9 +3,12 @@
 Tunable per plan: the gridding variant and tile (bin size), the coils per
 gridding workgroup, the hot-tile split threshold, and the interpolation
 variant, tile and coils per work item. Candidates are timed on
-the actual batch with HIP events; the choice is cached on disk keyed by the
-geometry (ndim, N, G, W, coils, samples per trajectory rounded, number of
-trajectories).
+the actual batch with HIP events, the gridding's with the transform that reads
+its grid: what a variant leaves in the caches counts too (8 x 16 spirals on
+512^2: the matrix 170 us by itself and the tiles 172, forward and adjoint with
+them 560 and 524 us). The choice is cached on disk keyed by the kernels'
+generation and the geometry (ndim, N, G, W, coils, samples per trajectory
+rounded, number of trajectories).
 """
 
 __all__ = ["tune_batch", "default_candidates"]
@@ -18,6 +21,11 @@ import torch
 
 from .batch import BatchedNUFFT
 from .fft.nufft import retune
+
+
+# Counts up when a gridding or interpolation variant changes its kernel, so that
+# choices cached for the former one are not used.
+_GENERATION = 2
 
 
 def default_candidates(ndim):
@@ -44,9 +52,9 @@ def _key(plans, ncoils):
     p = plans[0]
     m = int(np.median([q.npts * q.nframes for q in plans]))
     bucket = int(2 ** round(np.log2(max(m, 1))))
-    # the library is built for gfx950 only, so the geometry alone identifies a
-    # tuning problem (device-name queries are not stable under profilers)
-    return f"gfx950|d{p.ndim}|N{p.shape}|G{p.os_shape}|W{p.width}|C{max(ncoils)}|M{bucket}|P{len(plans)}"
+    # the library is built for gfx950 only, so generation and geometry identify
+    # a tuning problem (device-name queries are not stable under profilers)
+    return f"gfx950|k{_GENERATION}|d{p.ndim}|N{p.shape}|G{p.os_shape}|W{p.width}|C{max(ncoils)}|M{bucket}|P{len(plans)}"
 
 
 def _time(fn, reps, device):
@@ -106,13 +114,13 @@ def tune_batch(plans, ncoils, candidates=None, reps=5, use_cache=True, verbose=F
                     if gm == 0 and plans[0].interpolator.grid_mode_effective() != 4:
                         continue  # a variant tried under its own number
                     b = BatchedNUFFT(plans, ncoils)
-                    t = _time(lambda: b.gridding(b.grid), reps, dev)
+                    t = _time(b.adjoint, reps, dev)
                 except RuntimeError as exc:  # variant unsupported for this width
                     results.append(("tile", (gm, tile), str(exc)))
                     continue
                 results.append(("tile", (gm, tile), t))
                 if verbose:
-                    print(f"autotune grid_mode {gm} tile {tile}: grid {t:.3f} ms", flush=True)
+                    print(f"autotune grid_mode {gm} tile {tile}: adjoint {t:.3f} ms", flush=True)
                 if t < best_t:
                     best_tile, best_t, best_gm = tile, t, gm
         # 2) coils per gridding workgroup
@@ -122,7 +130,7 @@ def tune_batch(plans, ncoils, candidates=None, reps=5, use_cache=True, verbose=F
                 continue
             _apply(plans, best_tile, 0, gc, gmode=best_gm)
             b = BatchedNUFFT(plans, ncoils)
-            t = _time(lambda: b.gridding(b.grid), reps, dev)
+            t = _time(b.adjoint, reps, dev)
             results.append(("grid_chunk", gc, t))
             if t < best_gt:
                 best_gc, best_gt = gc, t
@@ -134,10 +142,10 @@ def tune_batch(plans, ncoils, candidates=None, reps=5, use_cache=True, verbose=F
         for sp in cand.get(splits, []):
             _apply(plans, best_tile, 0, best_gc, split=sp, gmode=best_gm)
             b = BatchedNUFFT(plans, ncoils)
-            t = _time(lambda: b.gridding(b.grid), reps, dev)
+            t = _time(b.adjoint, reps, dev)
             results.append(("grid_split", sp, t))
             if verbose:
-                print(f"autotune grid_split {sp}: grid {t:.3f} ms", flush=True)
+                print(f"autotune grid_split {sp}: adjoint {t:.3f} ms", flush=True)
             if t < best_gt:
                 best_split, best_gt = sp, t
         # 3) interpolation: gather variant (coils per item) and LDS-staged
@@ -160,9 +168,11 @@ def tune_batch(plans, ncoils, candidates=None, reps=5, use_cache=True, verbose=F
                 best_i, best_it = (mode, itile, ic), t
         mode, itile, best_ic = best_i
         _apply(plans, best_tile, best_ic, best_gc, mode, itile, best_split, best_gm)
+        b = BatchedNUFFT(plans, ncoils)
+        grid_ms = _time(lambda: b.gridding(b.grid), reps, dev)
     best = dict(tile=list(best_tile), grid_mode=best_gm, grid_chunk=best_gc, grid_split=best_split,
                 interp_mode=mode,
-                itile=list(itile) if itile else None, interp_chunk=best_ic, grid_ms=best_gt,
+                itile=list(itile) if itile else None, interp_chunk=best_ic, grid_ms=grid_ms,
                 interp_ms=best_it)
     if use_cache:
         cache[key] = best
