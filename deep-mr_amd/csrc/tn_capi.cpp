@@ -210,15 +210,17 @@ static int64_t tiles_doubling(const std::vector<Job> &jobs, const std::vector<co
 }
 
 // Whether a table's tile gridding reads its samples from a coil-minor copy:
-// from kTilesCopyBytes of them on, or where a job's offsets pass 32 bits.
+// from kTilesCopyBytes of them on (of one coil each a copy would gain nothing),
+// or where a job's offsets pass 32 bits.
 static bool tiles_copy(const std::vector<Job> &jobs) {
     int64_t bytes = 0;
-    bool wide = false;
+    bool wide = false, coils = false;
     for (const Job &j : jobs) {
         bytes += (int64_t)sizeof(float2) * j.npts * j.nbatch;
         wide |= (j.nbatch - 1) * j.samp_bstride + j.npts >= (1ll << 29);
+        coils |= j.nbatch > 1;
     }
-    return wide || bytes >= kTilesCopyBytes;
+    return wide || (coils && bytes >= kTilesCopyBytes);
 }
 
 // Work lists. Interpolation items are (job, sample block, coil range);
@@ -634,8 +636,9 @@ int check_device(int device) {
     return TN_OK;
 }
 
-int grid_samples(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, const float *weight, hipStream_t stream,
-                 bool ranged) {
+// (workspace: for the partial sums, null: the tables' own)
+int grid_samples(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, const float *weight, float *workspace,
+                 hipStream_t stream, bool ranged) {
     clear_error();
     if (!plan) return fail(TN_E_ARG, "plan is NULL");
     if (nbatch < 1 || nbatch >= INT32_MAX) return fail(TN_E_ARG, "nbatch must be >= 1");
@@ -644,7 +647,7 @@ int grid_samples(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, co
     if (rc) return rc;
     LaunchTables *t = plan_tables(plan, nbatch, &rc);
     if (!t) return rc;
-    return launch_grid(*t, (const float2 *)samp, (float2 *)grid, weight, stream, LowRank{}, nullptr, ranged);
+    return launch_grid(*t, (const float2 *)samp, (float2 *)grid, weight, stream, LowRank{}, workspace, ranged);
 }
 
 // The whole FFT stages; ranged: only the grid cells of the plan's row ranges
@@ -910,7 +913,23 @@ int tn_interp(tn_plan *plan, const void *grid, void *samp, int64_t nbatch, const
 
 int tn_grid(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, const float *weight,
             tn_stream stream) {
-    return grid_samples(plan, samp, grid, nbatch, weight, (hipStream_t)stream, false);
+    return tn_grid_ws(plan, samp, grid, nbatch, weight, nullptr, stream);
+}
+
+int64_t tn_plan_workspace(tn_plan *plan, int64_t nbatch, int32_t ncoeff) {
+    clear_error();
+    if (!plan) return fail(TN_E_ARG, "plan is NULL");
+    if (nbatch < 1 || nbatch >= INT32_MAX) return fail(TN_E_ARG, "nbatch must be >= 1");
+    if (ncoeff < 0 || nbatch * (int64_t)std::max(ncoeff, 1) >= INT32_MAX) return fail(TN_E_RANGE, "nbatch * ncoeff too large");
+    int rc = check_device(plan->device);
+    if (rc) return rc;
+    const LaunchTables *t = plan_tables(plan, nbatch, &rc, ncoeff > 0 ? kTablesLowRank : kTablesPlain, std::max(ncoeff, 1));
+    return t ? t->scratch_floats : rc;
+}
+
+int tn_grid_ws(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, const float *weight, float *workspace,
+               tn_stream stream) {
+    return grid_samples(plan, samp, grid, nbatch, weight, workspace, (hipStream_t)stream, false);
 }
 
 int tn_grid_static(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, const float *weight,
@@ -956,6 +975,11 @@ int tn_interp_lowrank(tn_plan *plan, const void *grid, void *samp, int64_t nbatc
 
 int tn_grid_lowrank(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, int32_t ncoeff,
                     int32_t frame_npts, const void *basis, const float *weight, tn_stream stream) {
+    return tn_grid_lowrank_ws(plan, samp, grid, nbatch, ncoeff, frame_npts, basis, weight, nullptr, stream);
+}
+
+int tn_grid_lowrank_ws(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, int32_t ncoeff, int32_t frame_npts,
+                       const void *basis, const float *weight, float *workspace, tn_stream stream) {
     clear_error();
     if (!plan) return fail(TN_E_ARG, "plan is NULL");
     if (nbatch < 1 || nbatch >= INT32_MAX) return fail(TN_E_ARG, "nbatch must be >= 1");
@@ -968,7 +992,7 @@ int tn_grid_lowrank(tn_plan *plan, const void *samp, void *grid, int64_t nbatch,
     // accumulator coils are (coil, coeff) pairs
     LaunchTables *t = plan_tables(plan, nbatch, &rc, kTablesLowRank, ncoeff);
     if (!t) return rc;
-    return launch_grid(*t, (const float2 *)samp, (float2 *)grid, weight, (hipStream_t)stream, lr);
+    return launch_grid(*t, (const float2 *)samp, (float2 *)grid, weight, (hipStream_t)stream, lr, workspace);
 }
 
 int tn_apod_pad(tn_plan *plan, const void *image, void *grid, int64_t nimg, tn_stream stream) {
@@ -1074,9 +1098,14 @@ int tn_nufft_forward(tn_plan *plan, const void *image, void *grid, void *work, v
 
 int tn_nufft_adjoint(tn_plan *plan, const void *samp, void *grid, void *work, void *image, int64_t nbatch,
                      const float *weight, tn_stream stream) {
+    return tn_nufft_adjoint_ws(plan, samp, grid, work, image, nbatch, weight, nullptr, stream);
+}
+
+int tn_nufft_adjoint_ws(tn_plan *plan, const void *samp, void *grid, void *work, void *image, int64_t nbatch,
+                        const float *weight, float *workspace, tn_stream stream) {
     if (!plan) return fail(TN_E_ARG, "plan is NULL");
     const bool ranged = rows_ranged(plan, nbatch);
-    int rc = grid_samples(plan, samp, grid, nbatch, weight, (hipStream_t)stream, ranged);
+    int rc = grid_samples(plan, samp, grid, nbatch, weight, workspace, (hipStream_t)stream, ranged);
     return rc ? rc
               : transform_adjoint(plan, grid, image, work, nbatch * plan->p.nframes, (hipStream_t)stream, ranged);
 }

@@ -251,6 +251,7 @@ class NativePlan:
             torch.cuda.current_stream(device).synchronize()
         del keep
         self.handle = handle
+        self._workspaces = {}
         self._finalizer = weakref.finalize(self, _destroy, handle.value, device)
         # True when the plan has FFT stages of its own: kernels of the grid
         # lengths (has_fft), or of any length with factors up to 17 (G <=
@@ -293,9 +294,26 @@ class NativePlan:
                                          stream_ptr(self.device)), "tn_interp")
         return out
 
+    def _workspace(self, nbatch, ncoeff=0):
+        """Floats of the gridding's partial sums for ``nbatch`` coils. Each
+        call brings its own (from torch, on its stream), so that calls of one
+        plan may overlap on several streams."""
+        n = self._workspaces.get((nbatch, ncoeff))
+        if n is None:
+            n = int(_lib.load().tn_plan_workspace(self.handle, nbatch, ncoeff))
+            if n < 0:
+                _lib.check(n, "tn_plan_workspace")
+            self._workspaces[nbatch, ncoeff] = n
+        return n
+
+    def _partials(self, nbatch, ncoeff=0):
+        n = self._workspace(int(nbatch), int(ncoeff))
+        return torch.empty(n, dtype=torch.float32, device=self.device) if n else None
+
     def gridding(self, samp, out, nbatch, weight=None):
-        _lib.check(_lib.load().tn_grid(self.handle, ptr(samp), ptr(out), int(nbatch), ptr(weight),
-                                       stream_ptr(self.device)), "tn_grid")
+        ws = self._partials(nbatch)
+        _lib.check(_lib.load().tn_grid_ws(self.handle, ptr(samp), ptr(out), int(nbatch), ptr(weight), ptr(ws),
+                                          stream_ptr(self.device)), "tn_grid_ws")
         return out
 
     def interp_lowrank(self, grid, out, nbatch, ncoeff, frame_npts, basis_adjoint, weight=None):
@@ -307,9 +325,10 @@ class NativePlan:
 
     def gridding_lowrank(self, samp, out, nbatch, ncoeff, frame_npts, basis, weight=None):
         """samp (nbatch, npts) -> out (nbatch, ncoeff, *G); one-frame plan."""
-        _lib.check(_lib.load().tn_grid_lowrank(self.handle, ptr(samp), ptr(out), int(nbatch), int(ncoeff),
-                                               int(frame_npts), ptr(basis), ptr(weight),
-                                               stream_ptr(self.device)), "tn_grid_lowrank")
+        ws = self._partials(nbatch, ncoeff)
+        _lib.check(_lib.load().tn_grid_lowrank_ws(self.handle, ptr(samp), ptr(out), int(nbatch), int(ncoeff),
+                                                  int(frame_npts), ptr(basis), ptr(weight), ptr(ws),
+                                                  stream_ptr(self.device)), "tn_grid_lowrank_ws")
         return out
 
     def apod_pad(self, image, out, nimg):
@@ -408,10 +427,15 @@ class NativePlan:
         """samples (nbatch, nframes, npts) -> image (nbatch * nframes, *N)."""
         nimg, new = nbatch * self.nframes, {"dtype": torch.complex64, "device": self.device}
         with on_device(self.device):
-            grid, work = torch.empty((nimg, *self.grid), **new), self._transform_work(nimg)
+            # one buffer: the grid, then (512-byte aligned) the partial sums of its gridding
+            cells, partials = nimg * math.prod(self.grid), self._workspace(nbatch)
+            at = (cells + 63) // 64 * 64 if partials else cells
+            buf, work = torch.empty(at + (partials + 1) // 2, **new), self._transform_work(nimg)
             image = torch.empty((nimg, *self.shape), **new)
-            _lib.check(_lib.load().tn_nufft_adjoint(self.handle, ptr(samp), ptr(grid), ptr(work), ptr(image), nbatch,
-                                                    ptr(weight), stream_ptr(self.device)), "tn_nufft_adjoint")
+            workspace = ctypes.c_void_p(buf.data_ptr() + 8 * at) if partials else None
+            _lib.check(_lib.load().tn_nufft_adjoint_ws(self.handle, ptr(samp), ptr(buf), ptr(work), ptr(image), nbatch,
+                                                       ptr(weight), workspace, stream_ptr(self.device)),
+                       "tn_nufft_adjoint_ws")
         return image
 
 

@@ -74,6 +74,11 @@ _SIGNATURES = {
     "tn_transform_adjoint": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
     "tn_nufft_forward": (c_int32, [c_void_p] * 5 + [c_int64, c_void_p, c_void_p]),
     "tn_nufft_adjoint": (c_int32, [c_void_p] * 5 + [c_int64, c_void_p, c_void_p]),
+    "tn_plan_workspace": (c_int64, [c_void_p, c_int64, c_int32]),
+    "tn_grid_ws": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p]),
+    "tn_grid_lowrank_ws": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p,
+                                     c_void_p, c_void_p]),
+    "tn_nufft_adjoint_ws": (c_int32, [c_void_p] * 5 + [c_int64, c_void_p, c_void_p, c_void_p]),
     "tn_stages_create": (c_int32, [c_int32, ctypes.POINTER(c_int32), ctypes.POINTER(c_int32), c_void_p,
                                    ctypes.POINTER(c_void_p)]),
     "tn_convolve": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),

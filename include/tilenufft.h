@@ -165,6 +165,19 @@ int tn_grid(tn_plan *plan, const void *samp, void *grid, int64_t nbatch,
 int tn_grid_static(tn_plan *plan, const void *samp, void *grid, int64_t nbatch,
                    const float *weight, tn_stream stream);
 
+/* Gridding as tn_grid with its partial sums (split tiles, long matrix rows) in
+ * a workspace of the caller's, tn_plan_workspace floats of them, 16-byte
+ * aligned; NULL: the launch tables' own, which every call of this plan with
+ * this nbatch shares. With a workspace per call, calls of one plan may overlap
+ * on several streams while their samples take less than 48 MiB or are of one
+ * coil (the tables hold one coil-minor copy of larger ones).
+ * tn_plan_workspace makes the launch tables (as tn_plan_prepare) and returns
+ * their need in floats, which may be 0, or a negative TN_E_* code; ncoeff > 0:
+ * of tn_grid_lowrank. */
+int64_t tn_plan_workspace(tn_plan *plan, int64_t nbatch, int32_t ncoeff);
+int tn_grid_ws(tn_plan *plan, const void *samp, void *grid, int64_t nbatch,
+               const float *weight, float *workspace, tn_stream stream);
+
 /* Low-rank (subspace) interpolation. The plan must hold every frame's
  * samples as one trajectory (nframes = 1, npts = nframes_lr * frame_npts,
  * frame f = samples [f*frame_npts, (f+1)*frame_npts)).
@@ -186,6 +199,10 @@ int tn_interp_lowrank(tn_plan *plan, const void *grid, void *samp, int64_t nbatc
 int tn_grid_lowrank(tn_plan *plan, const void *samp, void *grid, int64_t nbatch,
                     int32_t ncoeff, int32_t frame_npts, const void *basis,
                     const float *weight, tn_stream stream);
+/* The same with the partial sums in the caller's workspace (tn_grid_ws). */
+int tn_grid_lowrank_ws(tn_plan *plan, const void *samp, void *grid, int64_t nbatch,
+                       int32_t ncoeff, int32_t frame_npts, const void *basis,
+                       const float *weight, float *workspace, tn_stream stream);
 
 /* Fused apodize + centred zero-pad + ifftshift: image (nimg, *N) ->
  * grid (nimg, *G) ready for an unnormalised forward FFT. Replaces
@@ -268,6 +285,9 @@ int tn_nufft_forward(tn_plan *plan, const void *image, void *grid, void *work, v
                      int64_t nbatch, const float *weight, tn_stream stream);
 int tn_nufft_adjoint(tn_plan *plan, const void *samp, void *grid, void *work, void *image,
                      int64_t nbatch, const float *weight, tn_stream stream);
+/* The same with the partial sums in the caller's workspace (tn_grid_ws). */
+int tn_nufft_adjoint_ws(tn_plan *plan, const void *samp, void *grid, void *work, void *image,
+                        int64_t nbatch, const float *weight, float *workspace, tn_stream stream);
 
 /* A plan of FFT stages alone, between images of shape[ndim] and grids of
  * grid[ndim] ((z, y, x) order, ndim 2 or 3), without samples or apodization:
