@@ -65,6 +65,11 @@ def variant_key(plan, kind, ncoils):
         auto_long = 256 if plan.ndim == 3 else 128  # the library's defaults
         long_row = auto_long if split == 0 else 1024 if split < 0 else min(split, 1024)
         return f"grid|matrix|record={record}|long={long_row}"
+    if kind == "grid" and plan.interpolator.grid_mode_effective() == 4:
+        blocks = (ncoils + 7) // 8  # the library's default: equal chunks of at most four blocks of 8 coils
+        coils = min(plan.grid_chunk, 32) if plan.grid_chunk > 0 else 8 * -(-blocks // -(-blocks // 4))
+        split = plan.grid_split if plan.grid_split != 0 else 384
+        return f"grid|tiles|coils={min(coils, ncoils)}|split={split if split > 0 else 'never'}"
     if kind == "grid":
         return (f"grid|mode={plan.grid_mode}|tile={list(plan.interpolator.tile())}|chunk={plan.grid_chunk}"
                 f"|split={plan.grid_split}")
@@ -78,7 +83,7 @@ STAGE_KERNELS = {
     "grid": ("samp_transpose_kernel", "grid_matrix_t_kernel", "grid_matrix_kernel", "matrix_fold_kernel",
              "tiles_copy_kernel", "grid_tiles_kernel", "grid_runs_kernel", "grid_kernel", "fold_kernel"),
     "interp": ("interp_staged_kernel", "interp_kernel"),
-    "fft_fwd": ("fft_cols_fwd_kernel", "fft_rows_kernel|false"),
+    "fft_fwd": ("fft_cols_fwd_kernel", "fft_rows_kernel|false"),  # second template argument: the direction
     "fft_adj": ("fft_rows_kernel|true", "fft_cols_inv_kernel"),
 }
 
@@ -100,11 +105,12 @@ def short_kernel_name(name):
 
 
 def _stage_of(kname):
-    base = kname.split("<")[0]
+    base, _, args = kname.rstrip(">").partition("<")
+    args = args.split(", ")
     for stage, names in STAGE_KERNELS.items():
         for entry in names:
             nm, _, flag = entry.partition("|")
-            if base == nm and (not flag or kname.rstrip(">").endswith(flag)):
+            if base == nm and (not flag or args[1:2] == [flag]):
                 return stage
     return None
 
