@@ -10,7 +10,12 @@
 //
 // The alternative is the library's transform of the whole padded grid between
 // the separate pad and crop kernels, which reads and writes the zeros, and
-// takes passes and transposes of its own for lengths with large factors.
+// takes passes and transposes of its own for lengths with large factors. It is
+// slower up to the longest convolution (1018^2 grids, N + G - 1 = 1526: one
+// image 46 us for 94, 32 images 815 for 1240; 127^3, 4 images 190 for 418).
+// Two transforms round twice: outputs move both ways against the library's
+// (whole calls with such lengths: error against 64 bits 0.8 to 1.07 of the
+// former).
 #include <cmath>
 #include <complex>
 #include <vector>

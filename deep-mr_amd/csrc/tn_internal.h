@@ -76,10 +76,9 @@ constexpr int kGridPad = 4;      // accumulator row padding (floats)
 // across footprint origins, or per-lane register runs over origin-sorted
 // entries (for at most kRunsMaxTaps taps per sample).
 // Matrix: per-cell sums over the plan's sparse gridding matrix (CSR by grid
-// cell), one lane per cell. Tiles (3D): one wave per gridding tile of
-// kTilesT cells, its cells' sums in registers (lane = (x, y), one register
-// set per z plane), over the tile's entries in sample order with per-sample
-// taps from a plan table.
+// cell), one lane per cell. Tiles (2D and 3D): one wave per small tile, whose
+// cells' sums the matrix cores form over the tile's entries in sample order with
+// per-sample taps from a plan table (tn_tiles.hip).
 enum GridMode { kGridAuto = 0, kGridSpread = 1, kGridRuns = 2, kGridMatrix = 3, kGridTiles = 4 };
 // Tile gridding (matrix cores): a tile is four patches of 4x4 cells, the z
 // planes of a 4x4x4 tile in 3D and the quadrants of an 8x8 tile in 2D.
@@ -96,11 +95,14 @@ constexpr int kTilesCopyCoils = 8; // coils per workgroup of the coil-minor copy
 // (CG-SENSE, 195 k entries: 1.95 ms a solve at 64-96, 2.02 at 160, 2.16 at
 // 256); the large kooshball (27 M entries) takes 4% longer than at 384.
 constexpr int kTilesWave = 96;
-// samples of a table (bytes) from which the gridding reads a coil-minor copy:
-// in place, the records of an entry's coils lie in different rows and a wave's
-// loads touch four times the cache lines, which costs nothing while the samples
-// stay in the L2s (12 coils, 31 MB: 46 us against 37 + 15 for the copy) and
-// most of the time beyond (kooshball, 328 MB: 1.63 ms against 0.98 + 0.11)
+// Samples of a table (bytes) from which the gridding reads a coil-minor copy: in
+// place, the records of an entry's coils lie in different rows and a wave's
+// loads touch four times the cache lines, which the L2s serve while they hold
+// the samples. In 2D the copy costs 5 us (16 coils, 31 MiB: 50 us in place, 56
+// with it); in 3D it gains 5% already at 8 MiB and 10% from 40 MiB on (8 coils
+// of 256^3, 39 MiB: 624 and 573 us; 312 MiB: 1494 and 1350). The line is a
+// compromise of the two: radials of 75 and 150 MiB would be faster in place (92
+// and 179 us for 118 and 203).
 constexpr int64_t kTilesCopyBytes = 48ll << 20;
 // Tap record of a sample: the taps of each axis, padded with zeros to wpad
 // words (16-byte aligned).

@@ -158,15 +158,17 @@ __device__ __forceinline__ void fill_tiles(const Job &J, const Item &it, bool ra
 // a wave uses only its own part of the LDS, whose operations complete in
 // order, so there are no barriers.
 //
-// What bounds it: the matrix instructions and the vector instructions around
-// them, about half the issue time each (kooshball 128^3, 8 coils, osf 2: 27 M
-// entries, 0.98 ms against 3.13 ms for the gridding matrix, whose gathers of one
-// record per tap were bound by their rate; 16 spirals, 256^2: 0.126 ms for the
-// kernel and 0.031 for the copy against 0.147 + 0.046). The dense product
-// spends most of its terms on zeros, hence small tiles, and the patches that
-// none of a group's four entries reaches are left out (1.02 -> 0.94 ms in 3D,
-// 52 -> 38 us in 2D). The patches are the outer loop: with the groups outside,
-// the compiler copied every sum at every branch (1.8 ms). Each lane loading its
+// What bounds it. 3D (kooshball 128^3, 8 coils, osf 2: 27 M entries): issue; the
+// vector units work 53% of their cycles and the matrix cores 33%. Copy, kernel
+// and fold take 0.12 + 1.19 + 0.02 ms with every cell written and 0.11 + 1.00 +
+// 0.02 in the whole adjoint, against 3.37 ms for the gridding matrix, whose
+// gathers of one record per tap were bound by their rate. 2D (8 x 16 spirals on
+// 512^2): latency, 22% and 14% at 12 waves per CU; 0.032 + 0.121 + 0.009 ms
+// against 0.028 + 0.147. The dense product spends most of its terms on zeros,
+// hence small tiles, and the patches that none of a group's four entries reaches
+// are left out (when that was added: 1.02 -> 0.94 ms in 3D, 52 -> 38 us in 2D).
+// The patches are the outer loop: with the groups outside, the compiler copied
+// every sum at every branch (1.8 ms). Each lane loading its
 // own operands from memory took 2.4 ms: the texture addresser was busy 80% of
 // the time, 18 cycles for each of 21 load instructions per sixteen entries.
 template <int NDIM, int WP, int NC, int FROM>
