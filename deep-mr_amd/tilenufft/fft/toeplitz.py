@@ -151,9 +151,10 @@ def _convolve(x, kern, dev):
     """The native stages' result, or None where they do not serve: low-rank,
     real or elsewhere-held kernels, kernels whose leading axes are not the last
     of the image's, empty batches, tensors without memory of their own (tracers
-    and functorch transforms, which take torch's calls)."""
+    and functorch transforms, which take torch's calls), backward passes that
+    are differentiated again (torch's calls record themselves)."""
     ndim, value = kern.ndim, kern.value
-    if _core.traced(x, value):
+    if _core.traced(x, value) or (torch.is_grad_enabled() and (x.requires_grad or value.requires_grad)):
         return None
     lead, klead = tuple(x.shape[:-ndim]), tuple(value.shape[:-ndim])
     if (kern.islowrank or value.dtype != torch.complex64 or value.device != dev or x.numel() == 0
