@@ -127,7 +127,6 @@ static int upload_tables(const std::vector<Job> &jobs, const std::vector<Item> &
     TN_HIP(hipMalloc(&t.d_grid, sizeof(Item) * std::max<size_t>(grid.size(), 1)));
     TN_HIP(hipMalloc(&t.d_fold, sizeof(Item) * std::max<size_t>(fold.size(), 1)));
     TN_HIP(hipMalloc(&t.d_slot_base, sizeof(int64_t) * std::max<size_t>(slot_base.size(), 1)));
-    TN_HIP(hipMalloc(&t.d_scratch, sizeof(float) * std::max<int64_t>(t.scratch_floats, 1)));
     hipStream_t us = nullptr;
     int rc = upload_stream(&us);
     if (rc) return rc;
@@ -147,8 +146,15 @@ static int upload_tables(const std::vector<Job> &jobs, const std::vector<Item> &
     t.device_bytes = (int64_t)(sizeof(Job) * std::max<size_t>(jobs.size(), 1) +
                                sizeof(Item) * (std::max<size_t>(interp.size(), 1) + std::max<size_t>(grid.size(), 1) +
                                                std::max<size_t>(fold.size(), 1)) +
-                               sizeof(int64_t) * std::max<size_t>(slot_base.size(), 1) +
-                               sizeof(float) * std::max<int64_t>(t.scratch_floats, 1));
+                               sizeof(int64_t) * std::max<size_t>(slot_base.size(), 1));
+    return TN_OK;
+}
+
+// Partial sums of the table's own, for launches that bring none (once).
+static int own_scratch(LaunchTables &t) {
+    if (t.d_scratch || t.scratch_floats == 0) return TN_OK;
+    TN_HIP(hipMalloc(&t.d_scratch, sizeof(float) * t.scratch_floats));
+    t.device_bytes += (int64_t)sizeof(float) * t.scratch_floats;
     return TN_OK;
 }
 
@@ -389,6 +395,17 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
         const int64_t cells = (int64_t)j.T[0] * j.T[1] * j.T[2];  // partial size per coil
         std::vector<int32_t> order, empty;
         if (tiles) {
+            size_t shared = 0, single = 0;  // (growing the list by doubling took half of its time)
+            for (int64_t tl = 0; tl < ntiles; ++tl) {
+                const int64_t n = goff[tl + 1] - goff[tl];
+                if (n > wave_max) shared += (size_t)std::max<int64_t>(1, (n + split - 1) / split);
+                single += n <= wave_max;
+            }
+            const size_t chunks = (j.nbatch + gc - 1) / gc;
+            if (jobs.size() == 1) {
+                joined.reserve(waves * (shared * chunks + kDealXcds) + 2 * single * chunks);
+                grid.reserve(single * chunks);
+            }
             order = brick_order(j.NT, j.ndim);
             empty = empty_runs(goff, j.NT, kTilesFillCells / j.T[0]);
         }
@@ -575,8 +592,9 @@ void destroy(tn_plan *pl) {
 enum TableUse { kTablesPlain = 0, kTablesGather = 1, kTablesLowRank = 2 };
 
 // Tables of a plan for `nbatch` coils; low-rank tables hold nbatch * ncoeff
-// accumulator coils.
-tn::LaunchTables *plan_tables(tn_plan *plan, int64_t nbatch, int *rc, int use = kTablesPlain, int ncoeff = 1) {
+// accumulator coils. own: with partial sums of their own.
+tn::LaunchTables *plan_tables(tn_plan *plan, int64_t nbatch, int *rc, int use = kTablesPlain, int ncoeff = 1,
+                              bool own = true) {
     if (plan->stages_only) {
         *rc = fail(TN_E_ARG, "the plan holds FFT stages only, no samples");
         return nullptr;
@@ -585,14 +603,15 @@ tn::LaunchTables *plan_tables(tn_plan *plan, int64_t nbatch, int *rc, int use = 
     const int64_t key = use == kTablesLowRank ? nbatch << 32 | ncoeff : nbatch;
     auto it = cache.find(key);
     if (it != cache.end()) {
-        *rc = TN_OK;
-        return &it->second;
+        *rc = own ? own_scratch(it->second) : TN_OK;
+        return *rc == TN_OK ? &it->second : nullptr;
     }
     std::vector<Job> jobs;
     make_jobs(plan, nbatch * ncoeff, 0, 0, 0, jobs);
     std::vector<const tn_plan *> owners(jobs.size(), plan);
     LaunchTables t;
     *rc = build_tables_for(jobs, owners, t, use == kTablesGather, use == kTablesLowRank ? ncoeff : 0);
+    if (*rc == TN_OK && own) *rc = own_scratch(t);
     if (*rc != TN_OK) {
         free_tables(t);
         return nullptr;
@@ -645,9 +664,22 @@ int grid_samples(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, co
     if (!grid || (!samp && plan->p.npts > 0)) return fail(TN_E_ARG, "NULL data pointer");
     int rc = check_device(plan->device);
     if (rc) return rc;
-    LaunchTables *t = plan_tables(plan, nbatch, &rc);
+    LaunchTables *t = plan_tables(plan, nbatch, &rc, kTablesPlain, 1, workspace == nullptr);
     if (!t) return rc;
     return launch_grid(*t, (const float2 *)samp, (float2 *)grid, weight, stream, LowRank{}, workspace, ranged);
+}
+
+int interp_samples(tn_plan *plan, const void *grid, void *samp, int64_t nbatch, const float *weight, bool own,
+                   hipStream_t stream) {
+    clear_error();
+    if (!plan) return fail(TN_E_ARG, "plan is NULL");
+    if (nbatch < 1 || nbatch >= INT32_MAX) return fail(TN_E_ARG, "nbatch must be >= 1");
+    if ((!grid || !samp) && plan->p.npts > 0) return fail(TN_E_ARG, "NULL data pointer");
+    int rc = check_device(plan->device);
+    if (rc) return rc;
+    LaunchTables *t = plan_tables(plan, nbatch, &rc, kTablesPlain, 1, own);
+    if (!t) return rc;
+    return launch_interp(*t, (const float2 *)grid, (float2 *)samp, weight, stream);
 }
 
 // The whole FFT stages; ranged: only the grid cells of the plan's row ranges
@@ -900,15 +932,7 @@ int tn_plan_prepare(tn_plan *plan, int64_t nbatch) {
 
 int tn_interp(tn_plan *plan, const void *grid, void *samp, int64_t nbatch, const float *weight,
               tn_stream stream) {
-    clear_error();
-    if (!plan) return fail(TN_E_ARG, "plan is NULL");
-    if (nbatch < 1 || nbatch >= INT32_MAX) return fail(TN_E_ARG, "nbatch must be >= 1");
-    if ((!grid || !samp) && plan->p.npts > 0) return fail(TN_E_ARG, "NULL data pointer");
-    int rc = check_device(plan->device);
-    if (rc) return rc;
-    LaunchTables *t = plan_tables(plan, nbatch, &rc);
-    if (!t) return rc;
-    return launch_interp(*t, (const float2 *)grid, (float2 *)samp, weight, (hipStream_t)stream);
+    return interp_samples(plan, grid, samp, nbatch, weight, true, (hipStream_t)stream);
 }
 
 int tn_grid(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, const float *weight,
@@ -923,7 +947,8 @@ int64_t tn_plan_workspace(tn_plan *plan, int64_t nbatch, int32_t ncoeff) {
     if (ncoeff < 0 || nbatch * (int64_t)std::max(ncoeff, 1) >= INT32_MAX) return fail(TN_E_RANGE, "nbatch * ncoeff too large");
     int rc = check_device(plan->device);
     if (rc) return rc;
-    const LaunchTables *t = plan_tables(plan, nbatch, &rc, ncoeff > 0 ? kTablesLowRank : kTablesPlain, std::max(ncoeff, 1));
+    const LaunchTables *t = plan_tables(plan, nbatch, &rc, ncoeff > 0 ? kTablesLowRank : kTablesPlain,
+                                        std::max(ncoeff, 1), false);
     return t ? t->scratch_floats : rc;
 }
 
@@ -967,8 +992,8 @@ int tn_interp_lowrank(tn_plan *plan, const void *grid, void *samp, int64_t nbatc
     if (rc) return rc;
     // the low-rank table's interpolation items hold (coil, coefficient) planes;
     // plans that do not stage their interpolation gather, by coil
-    LaunchTables *t = plan_tables(plan, nbatch, &rc, kTablesLowRank, ncoeff);
-    if (t && t->interp_mode != kInterpStaged) t = plan_tables(plan, nbatch, &rc, kTablesGather);
+    LaunchTables *t = plan_tables(plan, nbatch, &rc, kTablesLowRank, ncoeff, false);
+    if (t && t->interp_mode != kInterpStaged) t = plan_tables(plan, nbatch, &rc, kTablesGather, 1, false);
     if (!t) return rc;
     return launch_interp_lowrank(*t, (const float2 *)grid, (float2 *)samp, weight, (hipStream_t)stream, lr);
 }
@@ -990,7 +1015,7 @@ int tn_grid_lowrank_ws(tn_plan *plan, const void *samp, void *grid, int64_t nbat
     rc = check_device(plan->device);
     if (rc) return rc;
     // accumulator coils are (coil, coeff) pairs
-    LaunchTables *t = plan_tables(plan, nbatch, &rc, kTablesLowRank, ncoeff);
+    LaunchTables *t = plan_tables(plan, nbatch, &rc, kTablesLowRank, ncoeff, workspace == nullptr);
     if (!t) return rc;
     return launch_grid(*t, (const float2 *)samp, (float2 *)grid, weight, (hipStream_t)stream, lr, workspace);
 }
@@ -1093,7 +1118,7 @@ int tn_nufft_forward(tn_plan *plan, const void *image, void *grid, void *work, v
                      const float *weight, tn_stream stream) {
     if (!plan) return fail(TN_E_ARG, "plan is NULL");
     int rc = transform_forward(plan, image, grid, work, nbatch * plan->p.nframes, (hipStream_t)stream, rows_ranged(plan, nbatch));
-    return rc ? rc : tn_interp(plan, grid, samp, nbatch, weight, stream);
+    return rc ? rc : interp_samples(plan, grid, samp, nbatch, weight, false, (hipStream_t)stream);
 }
 
 int tn_nufft_adjoint(tn_plan *plan, const void *samp, void *grid, void *work, void *image, int64_t nbatch,
@@ -1150,7 +1175,7 @@ int tn_batch_create(tn_plan *const *plans, const int64_t *nbatch, const int64_t 
     b->plans.assign(plans, plans + njobs);
     b->tables.resize(parts.size());
     for (size_t q = 0; q < parts.size() && rc == TN_OK; ++q)
-        rc = build_tables_for(parts[q].jobs, parts[q].owners, b->tables[q]);
+        if ((rc = build_tables_for(parts[q].jobs, parts[q].owners, b->tables[q])) == TN_OK) rc = own_scratch(b->tables[q]);
     if (rc) {
         for (LaunchTables &t : b->tables) free_tables(t);
         delete b;

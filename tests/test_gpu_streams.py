@@ -64,3 +64,27 @@ def test_workspace_need_and_own_workspace():
             grids.append(torch.view_as_real(g))
         torch.cuda.synchronize()
     assert torch.equal(grids[0], grids[1]) and torch.equal(grids[0], grids[2])
+
+
+def test_tables_hold_partial_sums_only_for_calls_without_a_workspace():
+    """The Python calls leave the launch tables without partial sums; the first
+    call that brings no workspace, and tn_plan_prepare, allocate them once."""
+    print("tables without partial sums", flush=True)
+    lib = _lib.load()
+    k = testing.complex_normal((3, 400000), seed=6).to(DEV)
+    for prepare in (False, True):
+        plan = tilenufft.fft.plan_nufft(hot(2), 32, 4, 2.0, device=DEV)
+        native = plan.interpolator
+        x = tilenufft.fft.apply_nufft_adj(k.reshape(3, 4, 100000), plan)
+        tilenufft.fft.apply_nufft(x, plan)
+        lean, need = native.device_bytes(), 4 * native._workspaces[3, 0]
+        assert need > 0
+        for _ in range(2):
+            if prepare:
+                native.prepare(3)
+            else:
+                g = torch.empty((3, *plan.os_shape), dtype=torch.complex64, device=DEV)
+                with torch.cuda.device(DEV):
+                    _lib.check(lib.tn_grid(native.handle, _core.ptr(k), _core.ptr(g), 3, None, _core.stream_ptr(DEV)))
+                    torch.cuda.synchronize()
+            assert native.device_bytes() == lean + need
