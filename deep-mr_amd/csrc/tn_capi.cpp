@@ -192,27 +192,30 @@ static bool tiles_doubled(const tn_plan *pl) {
     return pl->p.grid_split == 0 || pl->p.grid_mode != kGridTiles;
 }
 
-// Factor on the entries per workgroup of a split tile: doubled until the
-// table's partial tiles fit the fixed gridding workspace, so that
-// allocation-free launches take every table.
-static int64_t tiles_doubling(const std::vector<Job> &jobs, const std::vector<const tn_plan *> &plan_of) {
-    for (int64_t times = 1;; times *= 2) {
-        int64_t floats = 0;
-        for (size_t ji = 0; ji < jobs.size(); ++ji) {
-            const Job &j = jobs[ji];
-            const tn_plan *pl = plan_of[ji];
-            const int64_t part = tiles_part(pl) * times;
-            if (part == 0 || !tiles_doubled(pl)) continue;
-            const int32_t *off = pl->h_bin_off.data() + (j.bin_off - pl->d_bin_off);
+// Factor on the entries per workgroup of a split tile, per job: doubled until
+// the partial tiles of the job's plan (every frame, at the job's coils) fit the
+// fixed gridding workspace, so that allocation-free launches take every plan. A
+// plan's factor does not depend on the other plans of a batch, nor do its sums.
+static std::vector<int64_t> tiles_doubling(const std::vector<Job> &jobs, const std::vector<const tn_plan *> &plan_of) {
+    std::vector<int64_t> times(jobs.size(), 1);
+    for (size_t j0 = 0; j0 < jobs.size();) {
+        const tn_plan *pl = plan_of[j0];
+        const size_t j1 = std::min(jobs.size(), j0 + pl->p.nframes);
+        const int64_t one = tiles_part(pl);
+        for (int64_t f = 1; one > 0 && tiles_doubled(pl); f *= 2) {
+            const Job &j = jobs[j0];
+            const int64_t part = one * f;
             int64_t parts = 0;
-            for (int64_t tl = 0; tl < pl->ntiles_total; ++tl) {
-                const int64_t n = off[tl + 1] - off[tl];
+            for (int64_t tl = 0; tl < pl->ntiles_total * pl->p.nframes; ++tl) {
+                const int64_t n = pl->h_bin_off[tl + 1] - pl->h_bin_off[tl];
                 if (n > part) parts += (n + part - 1) / part;
             }
-            floats += parts * 2 * j.nbatch * j.T[0] * j.T[1] * j.T[2];
+            std::fill(times.begin() + j0, times.begin() + j1, f);
+            if (parts * 2 * j.nbatch * j.T[0] * j.T[1] * j.T[2] <= kStaticScratchFloats || f > INT32_MAX) break;
         }
-        if (floats <= kStaticScratchFloats || times > INT32_MAX) return times;
+        j0 = j1;
     }
+    return times;
 }
 
 // Whether a table's tile gridding reads its samples from a coil-minor copy:
@@ -296,7 +299,7 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
     std::vector<Item> interp, grid, fold, tr, joined;
     std::vector<int64_t> slot_base;
     int64_t scratch = 0;
-    const int64_t tiles_times = gmode == kGridTiles ? tiles_doubling(jobs, plan_of) : 0;
+    const std::vector<int64_t> tiles_times = gmode == kGridTiles ? tiles_doubling(jobs, plan_of) : std::vector<int64_t>();
     const bool tcopy = gmode == kGridTiles && lr_coeffs == 0 && !force_gather && tiles_copy(jobs);
     for (size_t ji = 0; ji < jobs.size(); ++ji) {
         const Job &j = jobs[ji];
@@ -389,7 +392,7 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
                                                                  : (pl->p.grid_split + waves - 1) / waves)
                                        : 0;
         const int64_t split = pl->p.grid_split < 0 ? INT32_MAX
-                              : tiles              ? tiles_part(pl) * (tiles_doubled(pl) ? tiles_times : 1)
+                              : tiles              ? tiles_part(pl) * tiles_times[ji]
                               : pl->p.grid_split   ? pl->p.grid_split
                                                    : kGridSplitDefault;
         const int64_t cells = (int64_t)j.T[0] * j.T[1] * j.T[2];  // partial size per coil
