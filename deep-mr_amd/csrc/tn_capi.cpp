@@ -488,19 +488,18 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
     t.interp_lds = mode == kInterpStaged ? region_coil * (size_t)max_ic + rows_bytes : 0;
     if (mode == kInterpStaged) {
         bool fits = wc <= staged_width(gndim), even = true;
-        t.interp_planes = jobs.empty() ? 0 : jobs[0].nbatch;
         int64_t cells = 0, lds = 0;  // of a region: loaded in pairs, held at an odd row pitch
         for (const Job &j : jobs) {
             const int64_t rows = (int64_t)(j.IT[1] + j.W[1] - 1) * (j.IT[2] + j.W[2] - 1);
             cells = std::max<int64_t>(cells, rows * ((j.IT[0] + j.W[0]) / 2 * 2));
             lds = std::max<int64_t>(lds, rows * ((j.IT[0] + j.W[0] - 1) | 1));
             fits = fits && (int64_t)j.G[0] * j.G[1] * j.G[2] < (1ll << 29);  // 32-bit byte offsets
-            t.interp_planes = std::min(t.interp_planes, j.nbatch);
             even = even && j.G[0] % 2 == 0 && (j.IT[0] % 2 == 0 || j.INT_[0] == 1) && j.grid_off % 2 == 0 &&
                    j.grid_bstride % 2 == 0;
         }
         fits = fits && max_ic <= staged_coils(gndim) && cells <= staged_cells(gndim, wc) &&
                sizeof(float2) * (size_t)lds * max_ic <= kInterpLdsBudget;
+        t.interp_planes = mean_planes(jobs);
         t.interp_vec = !fits ? 0 : even ? 2 : gndim == 2 ? 1 : 0;
         if (t.interp_vec) t.interp_lds = std::max(t.interp_lds, sizeof(float2) * (size_t)lds * max_ic);
     }

@@ -215,7 +215,7 @@ struct LaunchTables {
     int st_cw = 0;  // 0: the lane-per-cell matrix kernel reads the samples in place
     int wpad = 0;   // tile gridding: words per axis of the tap records
     int interp_vec = 0;  // staged interpolation: cells per load the regions allow (2, 1), 0: row by row only
-    int interp_planes = 0;  // fewest planes of a job
+    int interp_planes = 0;  // planes per sample, the average over the jobs
     int st_cpl = 1; // coils per lane of the matrix kernel over the copy (1 or 2)
     int64_t device_bytes = 0;  // bytes of the device allocations above
 };

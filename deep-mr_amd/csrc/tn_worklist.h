@@ -56,6 +56,18 @@ inline int chirp_length(int N, int L) {
 // tiles it can meet, one more for a wrap.
 constexpr int most_pieces(int W, int T) { return (W + T - 2) / T + 2; }
 
+// Planes per sample of a launch, the rounded average over its jobs: a small job
+// of few planes does not choose the others' loads (the staged interpolation).
+template <class Jobs>
+int mean_planes(const Jobs &jobs) {
+    int64_t samples = 0, planes = 0;
+    for (const auto &j : jobs) {
+        samples += j.npts;
+        planes += j.npts * j.nbatch;
+    }
+    return samples == 0 ? 0 : (int)((planes + samples / 2) / samples);
+}
+
 constexpr int kMatrixCoils = 16;   // widest record of the matrix gridding (coils per item)
 constexpr int kMatrixStage = 1024; // entries of a run of cells staged in LDS (also the longest short row), 3D
 constexpr int kMatrixStage2d = 512; // the same in 2D: a smaller stage leaves LDS for more workgroups per CU
