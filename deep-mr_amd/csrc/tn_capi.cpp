@@ -150,13 +150,25 @@ static int upload_tables(const std::vector<Job> &jobs, const std::vector<Item> &
     return TN_OK;
 }
 
-// Partial sums of the table's own, for launches that bring none (once).
+// Partial sums and (tile gridding) sample copy of the table's own, for launches
+// that bring none (once).
 static int own_scratch(LaunchTables &t) {
-    if (t.d_scratch || t.scratch_floats == 0) return TN_OK;
-    TN_HIP(hipMalloc(&t.d_scratch, sizeof(float) * t.scratch_floats));
-    t.device_bytes += (int64_t)sizeof(float) * t.scratch_floats;
+    if (!t.d_scratch && t.scratch_floats > 0) {
+        TN_HIP(hipMalloc(&t.d_scratch, sizeof(float) * t.scratch_floats));
+        t.device_bytes += (int64_t)sizeof(float) * t.scratch_floats;
+    }
+    if (!t.d_st && t.st_elems > 0) {
+        TN_HIP(hipMalloc(&t.d_st, sizeof(float2) * t.st_elems));
+        t.device_bytes += (int64_t)sizeof(float2) * t.st_elems;
+    }
     return TN_OK;
 }
+
+// Where a caller's workspace holds the sample copy of the tile gridding: behind
+// the partial sums, 16-byte aligned; of the matrix every call of a table shares
+// the table's.
+static bool copy_in_workspace(const LaunchTables &t) { return t.grid_mode == kGridTiles && t.st_elems > 0; }
+static int64_t copy_at(const LaunchTables &t) { return (t.scratch_floats + 3) / 4 * 4; }
 
 // Matrix-gridding runs of frame f, cached in the plan per cells-per-item
 // limit (matrix_runs_of).
@@ -220,10 +232,10 @@ static std::vector<int64_t> tiles_doubling(const std::vector<Job> &jobs, const s
 
 // Whether a table's tile gridding reads its samples from a coil-minor copy:
 // from kTilesCopyBytes of them on (of one coil each a copy would gain nothing),
-// or where a job's offsets pass 32 bits.
-static bool tiles_copy(const std::vector<Job> &jobs) {
+// or where a job's offsets pass 32 bits (wide).
+static bool tiles_copy(const std::vector<Job> &jobs, bool &wide) {
     int64_t bytes = 0;
-    bool wide = false, coils = false;
+    bool coils = false;
     for (const Job &j : jobs) {
         bytes += (int64_t)sizeof(float2) * j.npts * j.nbatch;
         wide |= (j.nbatch - 1) * j.samp_bstride + j.npts >= (1ll << 29);
@@ -300,7 +312,7 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
     std::vector<int64_t> slot_base;
     int64_t scratch = 0;
     const std::vector<int64_t> tiles_times = gmode == kGridTiles ? tiles_doubling(jobs, plan_of) : std::vector<int64_t>();
-    const bool tcopy = gmode == kGridTiles && lr_coeffs == 0 && !force_gather && tiles_copy(jobs);
+    const bool tcopy = gmode == kGridTiles && lr_coeffs == 0 && !force_gather && tiles_copy(jobs, t.st_wide);
     for (size_t ji = 0; ji < jobs.size(); ++ji) {
         const Job &j = jobs[ji];
         const tn_plan *pl = plan_of[ji];
@@ -479,11 +491,10 @@ static int build_tables_for(const std::vector<Job> &jobs, const std::vector<cons
             TN_HIP(hipMemcpyAsync(t.d_tr, tr.data(), sizeof(Item) * tr.size(), hipMemcpyHostToDevice, us));
             TN_HIP(hipStreamSynchronize(us));
         }
-        TN_HIP(hipMalloc(&t.d_st, sizeof(float2) * std::max<int64_t>(off, 1)));
+        if (gmode == kGridMatrix) TN_HIP(hipMalloc(&t.d_st, sizeof(float2) * std::max<int64_t>(off, 1)));
     }
-    const int64_t copy_bytes = t.d_st ? (int64_t)(sizeof(Item) * std::max<size_t>(tr.size(), 1) +
-                                                  sizeof(float2) * std::max<int64_t>(t.st_elems, 1))
-                                      : 0;
+    const int64_t copy_bytes = (t.d_tr ? (int64_t)(sizeof(Item) * std::max<size_t>(tr.size(), 1)) : 0) +
+                               (t.d_st ? (int64_t)(sizeof(float2) * std::max<int64_t>(t.st_elems, 1)) : 0);
     t.grid_lds = lds_grid ? grid_lds_bytes(max_gc, max_plane, wc, gmode, gndim) : 0;
     t.interp_lds = mode == kInterpStaged ? region_coil * (size_t)max_ic + rows_bytes : 0;
     if (mode == kInterpStaged) {
@@ -594,7 +605,7 @@ void destroy(tn_plan *pl) {
 enum TableUse { kTablesPlain = 0, kTablesGather = 1, kTablesLowRank = 2 };
 
 // Tables of a plan for `nbatch` coils; low-rank tables hold nbatch * ncoeff
-// accumulator coils. own: with partial sums of their own.
+// accumulator coils. own: with partial sums and a sample copy of their own.
 tn::LaunchTables *plan_tables(tn_plan *plan, int64_t nbatch, int *rc, int use = kTablesPlain, int ncoeff = 1,
                               bool own = true) {
     if (plan->stages_only) {
@@ -657,7 +668,7 @@ int check_device(int device) {
     return TN_OK;
 }
 
-// (workspace: for the partial sums, null: the tables' own)
+// (workspace: for the partial sums and the sample copy, null: the tables' own)
 int grid_samples(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, const float *weight, float *workspace,
                  hipStream_t stream, bool ranged) {
     clear_error();
@@ -668,7 +679,8 @@ int grid_samples(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, co
     if (rc) return rc;
     LaunchTables *t = plan_tables(plan, nbatch, &rc, kTablesPlain, 1, workspace == nullptr);
     if (!t) return rc;
-    return launch_grid(*t, (const float2 *)samp, (float2 *)grid, weight, stream, LowRank{}, workspace, ranged);
+    float2 *copy = workspace && copy_in_workspace(*t) ? (float2 *)(workspace + copy_at(*t)) : nullptr;
+    return launch_grid(*t, (const float2 *)samp, (float2 *)grid, weight, stream, LowRank{}, workspace, ranged, copy);
 }
 
 int interp_samples(tn_plan *plan, const void *grid, void *samp, int64_t nbatch, const float *weight, bool own,
@@ -951,7 +963,8 @@ int64_t tn_plan_workspace(tn_plan *plan, int64_t nbatch, int32_t ncoeff) {
     if (rc) return rc;
     const LaunchTables *t = plan_tables(plan, nbatch, &rc, ncoeff > 0 ? kTablesLowRank : kTablesPlain,
                                         std::max(ncoeff, 1), false);
-    return t ? t->scratch_floats : rc;
+    if (!t) return rc;
+    return ncoeff == 0 && copy_in_workspace(*t) ? copy_at(*t) + 2 * t->st_elems : t->scratch_floats;
 }
 
 int tn_grid_ws(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, const float *weight, float *workspace,
@@ -974,6 +987,8 @@ int tn_grid_static(tn_plan *plan, const void *samp, void *grid, int64_t nbatch, 
     if (t.scratch_floats > kStaticScratchFloats)
         return fail(TN_E_RANGE, "gridding needs %lld workspace floats, the fixed workspace holds %lld",
                     (long long)t.scratch_floats, (long long)kStaticScratchFloats);
+    if (t.st_wide && !t.d_st)
+        return fail(TN_E_ARG, "no sample copy for %lld coils: call tn_plan_prepare first", (long long)nbatch);
     float *ws = nullptr;
     rc = static_scratch(plan->device, &ws);
     if (rc) return rc;

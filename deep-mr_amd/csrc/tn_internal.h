@@ -210,9 +210,10 @@ struct LaunchTables {
     // st_cw coils, [chunk][sample][st_cw] per job, built by the copy items
     Item *d_tr = nullptr;
     int64_t n_tr = 0;
-    float2 *d_st = nullptr;
+    float2 *d_st = nullptr;  // of the tile gridding only for launches that bring none
     int64_t st_elems = 0;
-    int st_cw = 0;  // 0: the lane-per-cell matrix kernel reads the samples in place
+    int st_cw = 0;  // 0: the samples are read in place
+    bool st_wide = false;  // tile gridding: offsets of samples read in place would pass 32 bits
     int wpad = 0;   // tile gridding: words per axis of the tap records
     int interp_vec = 0;  // staged interpolation: cells per load the regions allow (2, 1), 0: row by row only
     int interp_planes = 0;  // planes per sample, the average over the jobs
@@ -312,8 +313,9 @@ int launch_interp(const LaunchTables &t, const float2 *grid, float2 *samp,
                   const float *weight, hipStream_t stream);
 int launch_grid(const LaunchTables &t, const float2 *samp, float2 *grid,
                 const float *weight, hipStream_t stream, LowRank lr = LowRank{},
-                float *scratch = nullptr, bool ranged = false);
-// (ranged: cells beyond the row ranges may be left unwritten)
+                float *scratch = nullptr, bool ranged = false, float2 *copy = nullptr);
+// (ranged: cells beyond the row ranges may be left unwritten; copy: room for the
+// sample copy of the tile gridding, null: the table's own, or none)
 // Device address of the fixed gridding workspace on `device` (looked up once
 // per device with hipGetSymbolAddress; no allocation).
 int static_scratch(int device, float **out);
@@ -340,7 +342,7 @@ bool tiles_serve(const tn_plan_params &p);
 // Entries of a tile plan (coordinates uploaded): below 2^31 - 1 an upper bound, else exact.
 int tile_entries(const tn_plan *plan, hipStream_t stream, int64_t &n);
 int launch_tiles(const LaunchTables &t, const float2 *samp, float2 *grid, const float *weight, hipStream_t stream,
-                 const LowRank &lr, float *scratch, bool ranged = false);
+                 const LowRank &lr, float *scratch, bool ranged, float2 *st);
 int build_matrix(tn_plan *plan, hipStream_t stream);
 // Pruned, fused oversampled-grid FFT stages (2D and 3D plans).
 int build_fft(tn_plan *plan, hipStream_t stream);

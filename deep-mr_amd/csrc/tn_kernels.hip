@@ -1693,7 +1693,7 @@ MatrixFn pick_matrix(int coils) {
 }
 
 int launch_grid(const LaunchTables &t, const float2 *samp, float2 *grid, const float *weight,
-                hipStream_t stream, LowRank lr, float *scratch, bool ranged) {
+                hipStream_t stream, LowRank lr, float *scratch, bool ranged, float2 *copy) {
     if (t.n_grid == 0) return TN_OK;
     if (scratch == nullptr) scratch = t.d_scratch;
     if (t.grid_mode == kGridMatrix && lr.ncoeff == 0 && t.st_cw > 0) {
@@ -1738,7 +1738,7 @@ int launch_grid(const LaunchTables &t, const float2 *samp, float2 *grid, const f
         TN_HIP(hipGetLastError());
         return launch_matrix_fold(t, grid, scratch, stream);
     }
-    if (t.grid_mode == kGridTiles) return launch_tiles(t, samp, grid, weight, stream, lr, scratch, ranged);
+    if (t.grid_mode == kGridTiles) return launch_tiles(t, samp, grid, weight, stream, lr, scratch, ranged, copy);
     if (t.grid_mode == kGridMatrix) {
         if (t.grid_coils > kMatrixCoils) return fail(TN_E_ARG, "matrix gridding: %d coils per item", t.grid_coils);
         MatrixFn fn = lr.ncoeff > 0 ? pick_matrix<true>(t.grid_coils) : pick_matrix<false>(t.grid_coils);

@@ -463,14 +463,18 @@ TilesFn pick_tiles(int ndim, int wpad, int blocks) {
 }  // namespace
 
 int launch_tiles(const LaunchTables &t, const float2 *samp, float2 *grid, const float *weight, hipStream_t stream,
-                 const LowRank &lr, float *scratch, bool ranged) {
+                 const LowRank &lr, float *scratch, bool ranged, float2 *st) {
     const int ndim = kind_ndim(t.kind_grid);
     const int blocks = (t.grid_coils + 7) / 8;
     if ((ndim != 2 && ndim != 3) || kind_width(t.kind_grid) > kTilesMaxWidth || blocks < 1 || blocks > kTilesBlocks)
         return fail(TN_E_ARG, "tile gridding: %dD, width %d, %d coils per item", ndim, kind_width(t.kind_grid),
                     t.grid_coils);
-    const bool copy = lr.ncoeff == 0 && t.st_cw > 0;
-    TileSrc src{samp, weight, t.d_st, t.st_cw, lr, 0u, 0, ranged};
+    if (st == nullptr) st = t.d_st;
+    // without room for the copy the samples are read in place: the same bits,
+    // where their offsets fit
+    const bool copy = lr.ncoeff == 0 && t.st_cw > 0 && st != nullptr;
+    if (lr.ncoeff == 0 && t.st_wide && !copy) return fail(TN_E_ARG, "tile gridding: no room for the sample copy");
+    TileSrc src{samp, weight, st, t.st_cw, lr, 0u, 0, ranged};
     if (lr.ncoeff > 0) {
         // division of a sample index (< 2^31) by frame_npts: l = ceil(log2 d),
         // m = floor(2^32 (2^l - d) / d) + 1
@@ -482,7 +486,7 @@ int launch_tiles(const LaunchTables &t, const float2 *samp, float2 *grid, const 
     }
     if (copy) {
         hipLaunchKernelGGL(tiles_copy_kernel, dim3((unsigned)t.n_tr), dim3(kBlock), 0, stream, t.d_jobs, t.d_tr, samp,
-                           weight, t.d_st, t.st_cw);
+                           weight, st, t.st_cw);
         TN_HIP(hipGetLastError());
     }
     const TilesFn fn = lr.ncoeff > 0 ? pick_tiles<kLowRank>(ndim, t.wpad, blocks)

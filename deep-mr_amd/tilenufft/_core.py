@@ -295,9 +295,9 @@ class NativePlan:
         return out
 
     def _workspace(self, nbatch, ncoeff=0):
-        """Floats of the gridding's partial sums for ``nbatch`` coils. Each
-        call brings its own (from torch, on its stream), so that calls of one
-        plan may overlap on several streams."""
+        """Floats of the gridding's partial sums and sample copy for ``nbatch``
+        coils. Each call brings its own (from torch, on its stream), so that
+        calls of one plan may overlap on several streams."""
         n = self._workspaces.get((nbatch, ncoeff))
         if n is None:
             n = int(_lib.load().tn_plan_workspace(self.handle, nbatch, ncoeff))
@@ -427,7 +427,7 @@ class NativePlan:
         """samples (nbatch, nframes, npts) -> image (nbatch * nframes, *N)."""
         nimg, new = nbatch * self.nframes, {"dtype": torch.complex64, "device": self.device}
         with on_device(self.device):
-            # one buffer: the grid, then (512-byte aligned) the partial sums of its gridding
+            # one buffer: the grid, then (512-byte aligned) the workspace of its gridding
             cells, partials = nimg * math.prod(self.grid), self._workspace(nbatch)
             at = (cells + 63) // 64 * 64 if partials else cells
             buf, work = torch.empty(at + (partials + 1) // 2, **new), self._transform_work(nimg)

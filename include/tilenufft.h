@@ -165,15 +165,15 @@ int tn_grid(tn_plan *plan, const void *samp, void *grid, int64_t nbatch,
 int tn_grid_static(tn_plan *plan, const void *samp, void *grid, int64_t nbatch,
                    const float *weight, tn_stream stream);
 
-/* Gridding as tn_grid with its partial sums (split tiles, long matrix rows) in
- * a workspace of the caller's, tn_plan_workspace floats of them, 16-byte
- * aligned; NULL: the launch tables' own, which every call of this plan with
- * this nbatch shares. With a workspace per call, calls of one plan may overlap
- * on several streams while their samples take less than 48 MiB or are of one
- * coil (the tables hold one coil-minor copy of larger ones).
- * tn_plan_workspace makes the launch tables (as tn_plan_prepare, without partial
- * sums of their own) and returns their need in floats, which may be 0, or a
- * negative TN_E_* code; ncoeff > 0: of tn_grid_lowrank. */
+/* Gridding as tn_grid with its partial sums (split tiles, long matrix rows) and
+ * the tiles' coil-minor sample copy in a workspace of the caller's,
+ * tn_plan_workspace floats, 16-byte aligned; NULL: the launch tables' own, which
+ * every call of this plan with this nbatch shares. With a workspace per call,
+ * calls of one plan may overlap on several streams (plans of grid_mode 3: those
+ * of one coil; of more coils the tables hold one copy).
+ * tn_plan_workspace makes the launch tables (as tn_plan_prepare, without buffers
+ * of their own) and returns their need in floats, which may be 0, or a negative
+ * TN_E_* code; ncoeff > 0: of tn_grid_lowrank. */
 int64_t tn_plan_workspace(tn_plan *plan, int64_t nbatch, int32_t ncoeff);
 int tn_grid_ws(tn_plan *plan, const void *samp, void *grid, int64_t nbatch,
                const float *weight, float *workspace, tn_stream stream);
