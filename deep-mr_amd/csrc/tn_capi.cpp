@@ -151,8 +151,10 @@ static int upload_tables(const std::vector<Job> &jobs, const std::vector<Item> &
 }
 
 // Partial sums and (tile gridding) sample copy of the table's own, for launches
-// that bring none (once).
+// that bring none (once, also where threads of calls on one plan meet here).
+static std::mutex g_scratch_mu;
 static int own_scratch(LaunchTables &t) {
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
     if (!t.d_scratch && t.scratch_floats > 0) {
         TN_HIP(hipMalloc(&t.d_scratch, sizeof(float) * t.scratch_floats));
         t.device_bytes += (int64_t)sizeof(float) * t.scratch_floats;
